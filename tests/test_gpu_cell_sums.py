@@ -1,0 +1,71 @@
+"""Sums over a cell's blocks (moments, pressure tensor) split over several workgroups per cell,
+against numpy in FP64 on the downloaded f.
+
+The kernels add FP64 products of the stored values; with N terms of one sign the rounding of any
+summation order stays below N 2^-53 of the sum of the terms' magnitudes (N < 2^17 here: 1.5e-11),
+plus a few 2^-53 for the velocities.  The bound below is 1e-10 of that sum.
+"""
+import numpy as np
+import pytest
+
+from vlasiator_amd import vacc as V
+
+pytestmark = pytest.mark.gpu
+
+MASS, CHARGE = 1.67262158e-27, 1.60217653e-19
+LEN, VMIN, VMAX = (33, 20, 17), (-1.3e6, -0.8e6, -0.7e6), (1.34e6, 0.8e6, 0.66e6)
+# blocks per cell around the 16-block and 64-block strides of a workgroup, and empty cells
+COUNTS = {"one": [1], "edges": [0, 15, 16, 17, 0, 63, 64, 65, 255, 257, 1025], "large": [9000],
+          "many": [(7 * i) % 41 for i in range(700)]}
+
+
+def _cells(counts, seed):
+    rng = np.random.default_rng(seed)
+    total = int(np.prod(LEN))
+    return [(np.sort(rng.choice(total, n, replace=False)).astype(np.uint32),
+             (10.0 ** rng.uniform(-15, -11, (n, 64))).astype(np.float32)) for n in counts]
+
+
+def _velocities(g):
+    x, y, z = g % LEN[0], g // LEN[0] % LEN[1], g // (LEN[0] * LEN[1])
+    e = np.arange(64)
+    out = []
+    for d, (b, i) in enumerate(((x, e & 3), (y, e >> 2 & 3), (z, e >> 4))):
+        h = (VMAX[d] - VMIN[d]) / LEN[d] / 4
+        out.append(VMIN[d] + (4.0 * b[:, None] + i[None, :] + 0.5) * h)
+    return out
+
+
+def _dv3():
+    return float(np.prod([(VMAX[d] - VMIN[d]) / LEN[d] / 4 for d in range(3)]))
+
+
+def _context(store, **opts):
+    return V.Context(V.make_mesh(LEN, VMIN, VMAX), V.make_species(MASS, CHARGE), V.make_options(V.PPM, storage=store, **opts))
+
+
+@pytest.mark.parametrize("store", [V.STORE_F32, V.STORE_BF16, V.STORE_F16])
+@pytest.mark.parametrize("sizes", sorted(COUNTS))
+def test_moments_and_pressure(sizes, store):
+    counts = COUNTS[sizes]
+    n = len(counts)
+    ctx = _context(store)
+    ctx.upload_cells(_cells(counts, 3))
+    pivot = np.random.default_rng(5).uniform(-3e5, 3e5, (n, 3))
+    mom, own, given = ctx.moments(n), ctx.pressure(n), ctx.pressure(n, pivot)
+    cells = ctx.download_cells()
+    ctx.close()
+    for c, (g, f) in enumerate(cells):
+        f = f.astype(np.float64)
+        v = _velocities(g.astype(np.int64))
+        first = np.array([f.sum()] + [(f * v[d]).sum() for d in range(3)]) * _dv3()
+        size = np.array([f.sum()] + [(f * np.abs(v[d])).sum() for d in range(3)]) * _dv3()
+        assert np.all(np.abs(mom[c] - first) <= 1e-10 * size), (c, mom[c], first)
+        bulk = first[1:] / first[0] if first[0] else np.zeros(3)
+        for got, at in ((own[c], bulk), (given[c], pivot[c])):
+            d = [v[k] - at[k] for k in range(3)]
+            for k, (a, b) in enumerate(((0, 0), (1, 1), (2, 2), (1, 2), (0, 2), (0, 1))):
+                want = MASS * _dv3() * (f * d[a] * d[b]).sum()
+                # the pivot's own rounding moves every velocity difference by about 1e-16 of |v|
+                most = MASS * _dv3() * (f * (np.abs(v[a]) + abs(at[a])) * (np.abs(v[b]) + abs(at[b]))).sum()
+                assert abs(got[k] - want) <= 1e-10 * most, (c, k, got[k], want)

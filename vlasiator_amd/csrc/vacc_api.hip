@@ -80,6 +80,8 @@ struct vacc_ctx {
    double* isect = nullptr;
    TransformIn* fields = nullptr;
    double* moments = nullptr;
+   double* parts = nullptr;          // [6*parts_max(ncells)] partial sums of the moment kernels
+   double* press = nullptr;          // [9*ncells] pressure tensor, and the caller's pivot
    double* pivot = nullptr;          // [4*ncells] plasma pivot of a multi-population step
    double* rho_loss = nullptr;
    // subcycling (vacc_subcycle_count / vacc_subcycle_step): per cell max_v_dt, subcycle count,
@@ -247,12 +249,13 @@ static void free_cells(vacc_ctx* c) {
    if (c->pivot) (void)hipFree(c->pivot);
    if (c->rho_loss) (void)hipFree(c->rho_loss);
    void* subs[] = {c->sub_maxdt, c->sub_dt, c->sub_n, c->active, c->sub_nmax, c->minval, c->csum_pre, c->csum_post,
-                   c->keep_bm, c->keep_box, c->cell_hist};
+                   c->keep_bm, c->keep_box, c->cell_hist, c->parts, c->press};
    for (void* p : subs)
       if (p) (void)hipFree(p);
    c->keep_bm = nullptr;
    c->keep_box = nullptr;
    c->cell_hist = nullptr;
+   c->parts = c->press = nullptr;
    c->sub_maxdt = c->sub_dt = nullptr;
    c->sub_n = c->sub_nmax = nullptr;
    c->minval = c->csum_pre = c->csum_post = nullptr;
@@ -264,6 +267,11 @@ static void free_cells(vacc_ctx* c) {
    c->pivot = nullptr;
    c->rho_loss = nullptr;
    c->cell_cap = 0;
+}
+
+// Most workgroups that cell_split gives any number of cells up to n.
+static size_t parts_max(uint32_t n) {
+   return std::min<size_t>((size_t)CELL_SPLIT_MAX * n, std::max<size_t>(CELL_PARTS, n)) + 1;
 }
 
 static int alloc_cells(vacc_ctx* c, uint32_t n) {
@@ -284,6 +292,8 @@ static int alloc_cells(vacc_ctx* c, uint32_t n) {
    HIPCHK(hipMalloc(&c->moments, m * 4 * sizeof(double)));
    HIPCHK(hipMalloc(&c->pivot, m * 4 * sizeof(double)));
    HIPCHK(hipMalloc(&c->rho_loss, m * sizeof(double)));
+   HIPCHK(hipMalloc(&c->parts, 6 * parts_max(n) * sizeof(double)));
+   HIPCHK(hipMalloc(&c->press, 9 * m * sizeof(double)));
    HIPCHK(hipMalloc(&c->sub_maxdt, m * sizeof(double)));
    HIPCHK(hipMalloc(&c->sub_dt, m * sizeof(double)));
    HIPCHK(hipMalloc(&c->sub_n, m * sizeof(uint32_t)));
@@ -1502,10 +1512,8 @@ static void to_tin(const vacc_cell_fields& in, TransformIn& t) {
    t.dt = in.dt;
 }
 
-// Enqueue the moments of the current list unless they are resident.
-static void enqueue_moments(vacc_ctx* c) {
-   if (c->moments_valid) return;
-   ProfScope ps(c, 3);
+// Arguments of the moment kernels over the current list.
+static MomentArgs moment_args(const vacc_ctx* c) {
    MomentArgs ma{};
    ma.cell_off = c->off[c->lcur];
    ma.gid = c->gid[c->lcur];
@@ -1519,6 +1527,14 @@ static void enqueue_moments(vacc_ctx* c) {
       ma.cell[d] = c->mi.cell[d];
    }
    ma.gs = make_gid_split(c->mi.len);
+   return ma;
+}
+
+// Enqueue the moments of the current list unless they are resident.
+static void enqueue_moments(vacc_ctx* c) {
+   if (c->moments_valid) return;
+   ProfScope ps(c, 3);
+   MomentArgs ma = moment_args(c);
    ma.blk_stats = c->stats_valid ? c->blk_stats : nullptr;
    launch_moments(ma, c->stream);
    c->moments_valid = true;
@@ -2030,34 +2046,12 @@ int vacc_pressure(vacc_ctx* c, const double* pivot, double* out) {
    if (!c || (!out && c->ncells)) return set_err(VACC_E_ARG, "null argument");
    if (!c->ncells) return 0;
    const size_t n = c->ncells;
-   std::vector<double> piv(3 * n);
-   if (pivot) {
-      std::copy(pivot, pivot + 3 * n, piv.begin());
-   } else {   // the population's own bulk velocity from its first moments
-      std::vector<double> mo(4 * n);
-      int rc = vacc_moments(c, mo.data());
-      if (rc) return rc;
-      for (size_t i = 0; i < n; ++i)
-         for (int d = 0; d < 3; ++d) piv[3 * i + d] = (mo[4 * i] != 0.0) ? mo[4 * i + 1 + d] / mo[4 * i] : 0.0;
-   }
-   DevTemps tmp;
-   double *d_piv = nullptr, *d_out = nullptr;
-   HIPCHK(tmp.alloc(&d_piv, 3 * n * sizeof(double)));
-   HIPCHK(tmp.alloc(&d_out, 6 * n * sizeof(double)));
-   HIPCHK(hipMemcpyAsync(d_piv, piv.data(), 3 * n * sizeof(double), hipMemcpyHostToDevice, c->stream));
-   MomentArgs ma{};
-   ma.cell_off = c->off[c->lcur];
-   ma.gid = c->gid[c->lcur];
-   ma.src = c->src[c->lcur];
-   ma.pool = pool(c, c->fcur);
-   ma.ncells = c->ncells;
-   for (int d = 0; d < 3; ++d) {
-      ma.len[d] = c->mi.len[d];
-      ma.vmin[d] = c->mi.vmin[d];
-      ma.cell[d] = c->mi.cell[d];
-   }
-   ma.gs = make_gid_split(c->mi.len);
-   launch_pressure(ma, d_piv, c->sp.mass, d_out, c->stream);
+   // without a pivot the kernel takes the population's own bulk velocity from its first moments
+   double *d_out = c->press, *d_piv = c->press + 6 * n;
+   if (pivot) HIPCHK(hipMemcpyAsync(d_piv, pivot, 3 * n * sizeof(double), hipMemcpyHostToDevice, c->stream));
+   else enqueue_moments(c);
+   MomentArgs ma = moment_args(c);
+   launch_pressure(ma, pivot ? d_piv : nullptr, c->sp.mass, c->parts, d_out, c->stream);
    HIPCHK(hipGetLastError());
    HIPCHK(hipMemcpyAsync(out, d_out, 6 * n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
    HIPCHK(hipStreamSynchronize(c->stream));

@@ -1497,46 +1497,93 @@ __global__ __launch_bounds__(WG) void k_content(const uint32_t* src, Pool pl, ui
    }
 }
 
-// Second moments of one population about a pivot (arch_moments.h:123-150): one workgroup per
-// cell, one lane per velocity cell of a block, FP64 sums; DV3 and the mass applied once.
-__global__ __launch_bounds__(WG) void k_pressure(MomentArgs a, const double* pivot, double mass, double* out) {
+// Second moments of one population about a pivot (arch_moments.h:123-150), split workgroups
+// per cell (blockIdx.x), 16 lanes per block and one float4 row (i = 0..3 at fixed j, k) per
+// lane, UNR blocks per lane group in flight.  With X the offset of the row's first cell from the
+// pivot along x and h the cell size, the row's sums S = sum f, A = sum i f, B = sum i^2 f give
+//   sum f dx = X S + h A,   sum f dx^2 = X (X S + 2 h A) + h^2 B,
+// and dy, dz are the row's: about 30 FP64 operations per row of four cells instead of 15 per
+// cell.  Each workgroup writes its six FP64 sums to part; k_cell_parts adds a cell's parts in
+// order, so the result does not depend on the schedule.
+// Bound by HBM reads (256 bytes per block).  The form before it, a wave per block with one
+// lane per cell, one block in flight and one workgroup per cell, was bound by the latency of
+// each block's loads and by the largest cell: 3.92 -> 1.36 ms over 26 million FP32 blocks in
+// 8192 cells (5.0 TB/s), 1.15 -> 0.022 ms over 64 cells of 300 to 20000 blocks.
+template <int ST>
+__global__ __launch_bounds__(WG) void k_pressure(MomentArgs a, const double* pivot, double* part, uint32_t split) {
    __shared__ double red[6][WG / 64];
-   const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-   const uint32_t c = blockIdx.x;
+   const int t = threadIdx.x;
+   const uint32_t c = blockIdx.x / split, sp = blockIdx.x - c * split;
    const uint32_t off = a.cell_off[c], n = a.cell_off[c + 1] - off;
-   const int i = lane & 3, j = (lane >> 2) & 3, k = lane >> 4;
-   const double px = pivot[3 * (size_t)c], py = pivot[3 * (size_t)c + 1], pz = pivot[3 * (size_t)c + 2];
-   const uint32_t nx = a.len[0], nxy = a.len[0] * a.len[1];
-   double s[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-   for (uint32_t b = w; b < n; b += WG / 64) {
-      const uint32_t sidx = a.src[off + b];
-      if (sidx == INVALID) continue;
-      const double f = pool_value(a.pool, sidx, lane);
-      const uint32_t g = a.gid[off + b];
-      uint32_t x, y, z;
-      gid_xyz(g, a.gs, x, y, z);
-      const double dx = (a.vmin[0] + (x * WID + i + 0.5) * a.cell[0]) - px;
-      const double dy = (a.vmin[1] + (y * WID + j + 0.5) * a.cell[1]) - py;
-      const double dz = (a.vmin[2] + (z * WID + k + 0.5) * a.cell[2]) - pz;
-      s[0] += f * dx * dx;
-      s[1] += f * dy * dy;
-      s[2] += f * dz * dz;
-      s[3] += f * dy * dz;
-      s[4] += f * dx * dz;
-      s[5] += f * dx * dy;
+   const int q = t & 15;
+   double p[3];
+   if (pivot) {
+      for (int d = 0; d < 3; ++d) p[d] = pivot[3 * (size_t)c + d];
+   } else {   // the population's own bulk velocity
+      const double* mo = a.out + 4 * (size_t)c;
+      for (int d = 0; d < 3; ++d) p[d] = (mo[0] != 0.0) ? mo[1 + d] / mo[0] : 0.0;
    }
+   // velocity of the row's first cell in block (0, 0, 0), from the pivot
+   const double h = a.cell[0];
+   const double ox = (a.vmin[0] + 0.5 * h) - p[0];
+   const double oy = (a.vmin[1] + ((q & 3) + 0.5) * a.cell[1]) - p[1];
+   const double oz = (a.vmin[2] + ((q >> 2) + 0.5) * a.cell[2]) - p[2];
+   const double bx = h * WID, by = a.cell[1] * WID, bz = a.cell[2] * WID, h2 = 2.0 * h;
+   double s[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0}, sb = 0.0;
+   constexpr uint32_t GROUPS = WG / 16;
+   constexpr int UNR = 4;
+   for (uint32_t b = sp * GROUPS + (t >> 4); b < n; b += UNR * GROUPS * split) {
+      uint32_t sv[UNR], gv[UNR];
+      float4 v[UNR];
 #pragma unroll
-   for (int q = 0; q < 6; ++q) {
-      for (int o = 32; o > 0; o >>= 1) s[q] += __shfl_down(s[q], o, 64);
-      if (lane == 0) red[q][w] = s[q];
+      for (int u = 0; u < UNR; ++u) {
+         const uint32_t bb = b + u * GROUPS * split;
+         sv[u] = (bb < n) ? a.src[off + bb] : INVALID;
+         gv[u] = (bb < n) ? a.gid[off + bb] : 0u;
+      }
+#pragma unroll
+      for (int u = 0; u < UNR; ++u) v[u] = pool_row_t<ST>(a.pool, sv[u], q);
+#pragma unroll
+      for (int u = 0; u < UNR; ++u) {
+         uint32_t x, y, z;
+         gid_xyz(gv[u], a.gs, x, y, z);
+         const double v0 = v[u].x, v1 = v[u].y, v2 = v[u].z, v3 = v[u].w;
+         const double S = (v0 + v1) + (v2 + v3);
+         const double A = fma(3.0, v3, fma(2.0, v2, v1));
+         const double X = fma((double)x, bx, ox), Y = fma((double)y, by, oy), Z = fma((double)z, bz, oz);
+         const double XS = X * S, YS = Y * S, D = fma(h, A, XS);   // D = sum f dx
+         sb += fma(9.0, v3, fma(4.0, v2, v1));
+         s[0] = fma(X, fma(h2, A, XS), s[0]);
+         s[1] = fma(Y, YS, s[1]);
+         s[2] = fma(Z, Z * S, s[2]);
+         s[3] = fma(Z, YS, s[3]);
+         s[4] = fma(Z, D, s[4]);
+         s[5] = fma(Y, D, s[5]);
+      }
+   }
+   s[0] = fma(h * h, sb, s[0]);
+#pragma unroll
+   for (int e = 0; e < 6; ++e) {
+      for (int o = 32; o > 0; o >>= 1) s[e] += __shfl_down(s[e], o, 64);
+      if ((t & 63) == 0) red[e][t >> 6] = s[e];
    }
    __syncthreads();
    if (t < 6) {
-      const double DV3 = a.cell[0] * a.cell[1] * a.cell[2];
       double sum = 0.0;
-      for (int q = 0; q < WG / 64; ++q) sum += red[t][q];
-      out[6 * (size_t)c + t] = mass * (sum * DV3);
+      for (int w = 0; w < WG / 64; ++w) sum += red[t][w];
+      part[6 * (size_t)blockIdx.x + t] = sum;
    }
+}
+
+// out[nv c + e] = scale * sum over the cell's parts, in order: part[(c split + p) nv + e]
+__global__ void k_cell_parts(const double* part, uint32_t split, uint32_t nv, uint32_t n, double scale, double* out) {
+   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+   if (i >= n) return;
+   const uint32_t c = i / nv, e = i - c * nv;
+   const double* p = part + (size_t)c * split * nv + e;
+   double sum = 0.0;
+   for (uint32_t k = 0; k < split; ++k) sum += p[(size_t)k * nv];
+   out[i] = sum * scale;
 }
 
 // spatial_cell_cpu.cpp:699-727
@@ -2067,9 +2114,23 @@ void launch_fill_f64(double* dst, double v, uint32_t n, hipStream_t s) {
    hipLaunchKernelGGL(k_fill_f64, dim3((n + 255) / 256), dim3(256), 0, s, dst, v, n);
 }
 
-void launch_pressure(const MomentArgs& a, const double* pivot, double mass, double* out, hipStream_t s) {
+// Workgroups per cell of the kernels that sum over a cell's blocks: about CELL_PARTS in all, so
+// that a few cells (or a few large ones among many) still fill the chip.
+uint32_t cell_split(uint32_t ncells) {
+   const uint32_t s = CELL_PARTS / std::max(ncells, 1u);
+   return std::min(std::max(s, 1u), CELL_SPLIT_MAX);
+}
+
+void launch_pressure(const MomentArgs& a, const double* pivot, double mass, double* part, double* out, hipStream_t s) {
    if (a.ncells == 0) return;
-   hipLaunchKernelGGL(k_pressure, dim3(a.ncells), dim3(WG), 0, s, a, pivot, mass, out);
+   const uint32_t split = cell_split(a.ncells);
+   const dim3 grid(a.ncells * split);
+   if (a.pool.storage == ST_F32) hipLaunchKernelGGL(k_pressure<ST_F32>, grid, dim3(WG), 0, s, a, pivot, part, split);
+   else if (a.pool.storage == ST_BF16) hipLaunchKernelGGL(k_pressure<ST_BF16>, grid, dim3(WG), 0, s, a, pivot, part, split);
+   else hipLaunchKernelGGL(k_pressure<ST_F16>, grid, dim3(WG), 0, s, a, pivot, part, split);
+   const double dv3 = a.cell[0] * a.cell[1] * a.cell[2];
+   hipLaunchKernelGGL(k_cell_parts, dim3((6 * a.ncells + 255) / 256), dim3(256), 0, s, part, split, 6u, 6 * a.ncells,
+                      mass * dv3, out);
 }
 
 void launch_sparse_min(const SparseArgs& p, const double* moments, const uint32_t* off, double* minval,
