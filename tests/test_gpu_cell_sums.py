@@ -1,4 +1,4 @@
-"""Sums over a cell's blocks (moments, pressure tensor) split over several workgroups per cell,
+"""Sums and flags over a cell's blocks (moments, pressure tensor, content) split over several workgroups per cell,
 against numpy in FP64 on the downloaded f.
 
 The kernels add FP64 products of the stored values; with N terms of one sign the rounding of any
@@ -69,3 +69,30 @@ def test_moments_and_pressure(sizes, store):
                 # the pivot's own rounding moves every velocity difference by about 1e-16 of |v|
                 most = MASS * _dv3() * (f * (np.abs(v[a]) + abs(at[a])) * (np.abs(v[b]) + abs(at[b]))).sum()
                 assert abs(got[k] - want) <= 1e-10 * most, (c, k, got[k], want)
+
+
+@pytest.mark.parametrize("store", [V.STORE_F32, V.STORE_BF16, V.STORE_F16])
+@pytest.mark.parametrize("sizes", sorted(COUNTS))
+def test_content_flags(sizes, store):
+    """The adjust after an upload keeps the blocks with a stored value at or above the threshold
+    and their neighbours; with width 0 it keeps exactly the former.  A fifth of the blocks hold
+    their one value above the threshold in a random cell, some at the threshold itself."""
+    counts = COUNTS[sizes]
+    rng = np.random.default_rng(11)
+    thr = 1e-13
+    cells = []
+    for g, _ in _cells(counts, 7):
+        f = np.full((len(g), 64), 2e-14, np.float32)
+        hit = np.nonzero(rng.random(len(g)) < 0.2)[0]
+        f[hit, rng.integers(0, 64, hit.size)] = rng.choice(np.array([thr, 1.1e-13, 3e-12], np.float32), hit.size)
+        cells.append((g, f))
+    ctx = V.Context(V.make_mesh(LEN, VMIN, VMAX), V.make_species(MASS, CHARGE, thr, 0), V.make_options(V.PPM, storage=store))
+    ctx.upload_cells(cells)
+    before = ctx.download_cells()
+    ctx.adjust(len(counts))
+    after = ctx.download_cells()
+    ctx.close()
+    for c, ((g, f), (g2, f2)) in enumerate(zip(before, after)):
+        keep = (f.astype(np.float64) >= thr).any(1)
+        assert np.array_equal(g2, g[keep]), c
+        assert np.array_equal(f2, f[keep]), c

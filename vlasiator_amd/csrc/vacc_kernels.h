@@ -198,7 +198,6 @@ struct InitArgs {
 
 void launch_init(const InitArgs& a, bool write_phase, hipStream_t s);
 int init_box_words_max();
-void launch_content(const uint32_t* src, const Pool& pool, uint8_t* content, uint32_t n, double mv, hipStream_t s);
 
 void launch_columns(int dim, const ColumnArgs& a, hipStream_t s);
 void launch_scan(const ScanArgs& a, hipStream_t s);
@@ -240,7 +239,7 @@ struct SparseArgs {
 };
 void launch_sparse_min(const SparseArgs& p, const double* moments, const uint32_t* off, double* minval,
                        uint32_t ncells, hipStream_t s);
-// content flag of every block of a list with the cell's threshold (one workgroup per cell)
+// content flag of every block of a list with the cell's threshold
 void launch_content_cells(const uint32_t* off, const uint32_t* src, const Pool& pool, const double* minval,
                           uint8_t* content, uint32_t ncells, hipStream_t s);
 // FP64 sum of f over each cell's blocks
