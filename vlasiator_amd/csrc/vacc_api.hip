@@ -1520,6 +1520,7 @@ static MomentArgs moment_args(const vacc_ctx* c) {
    ma.src = c->src[c->lcur];
    ma.pool = pool(c, c->fcur);
    ma.out = c->moments;
+   ma.part = c->parts;
    ma.ncells = c->ncells;
    for (int d = 0; d < 3; ++d) {
       ma.len[d] = c->mi.len[d];
@@ -2051,7 +2052,7 @@ int vacc_pressure(vacc_ctx* c, const double* pivot, double* out) {
    if (pivot) HIPCHK(hipMemcpyAsync(d_piv, pivot, 3 * n * sizeof(double), hipMemcpyHostToDevice, c->stream));
    else enqueue_moments(c);
    MomentArgs ma = moment_args(c);
-   launch_pressure(ma, pivot ? d_piv : nullptr, c->sp.mass, c->parts, d_out, c->stream);
+   launch_pressure(ma, pivot ? d_piv : nullptr, c->sp.mass, d_out, c->stream);
    HIPCHK(hipGetLastError());
    HIPCHK(hipMemcpyAsync(out, d_out, 6 * n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
    HIPCHK(hipStreamSynchronize(c->stream));

@@ -165,6 +165,8 @@ struct MomentArgs {
    const uint32_t* src;
    Pool pool;
    double* out;                // [ncells*4]
+   double* part;               // partial sums: 4 (moments) or 6 (pressure) doubles per workgroup,
+                               // ncells * cell_split(ncells) workgroups
    uint32_t ncells;
    uint32_t len[3];
    GidSplit gs;                // block coordinates of a GID (from len)
@@ -250,15 +252,14 @@ void launch_cell_sums(const uint32_t* off, const uint32_t* src, const Pool& pool
 void launch_cell_scale(const uint32_t* off, const uint32_t* src, const Pool& pool, const double* pre,
                        const double* post, uint32_t ncells, hipStream_t s);
 void launch_fill_f64(double* dst, double v, uint32_t n, hipStream_t s);
-// Workgroups per cell of the sums over a cell's blocks, and the most workgroups of such a launch
-// (per-workgroup partial sums: at most CELL_PARTS + ncells parts).
+// Workgroups per cell of the kernels that read a cell's blocks, about CELL_PARTS in all and at most
+// CELL_SPLIT_MAX per cell.
 constexpr uint32_t CELL_PARTS = 32768, CELL_SPLIT_MAX = 64;
 uint32_t cell_split(uint32_t ncells);
 // Second moments (arch_moments.h:123-150): out[6c..] = mass * sum f (v - V)_a (v - V)_b DV3 for
 // (a,b) = xx, yy, zz, yz, xz, xy (FP64 sums) about the pivot pivot[3c..], or, for a null pivot,
-// about the population's bulk velocity of a.out (its first moments).  part: 6 doubles per
-// workgroup (ncells * cell_split(ncells)).
-void launch_pressure(const MomentArgs& a, const double* pivot, double mass, double* part, double* out, hipStream_t s);
+// about the population's bulk velocity of a.out (its first moments).
+void launch_pressure(const MomentArgs& a, const double* pivot, double mass, double* out, hipStream_t s);
 // dt_override: [ncells] or null; replaces fields[c].dt.
 void launch_transform(const MeshInfo& m, const TransformIn* fields, const double* dt_override, const double* moments, int use_moments,
                       double mass, double charge, double hall_min_rhoq, int ohm_gradpe, int map_order,

@@ -1482,20 +1482,53 @@ __global__ __launch_bounds__(AWG) void k_adjust(AdjustArgs a) {
    }
 }
 
+// out[nv c + e] = scale * sum over the cell's parts part[(c split + p) nv + e]: 16 lanes per sum,
+// each adding every 16th part, then a fixed tree (one lane per sum waited 10 us for 64 dependent
+// loads, 16 lanes take 4)
+__global__ __launch_bounds__(WG) void k_cell_parts(const double* part, uint32_t split, uint32_t nv, uint32_t n,
+                                                   double scale, double* out) {
+   const uint32_t i = blockIdx.x * (WG / 16) + (threadIdx.x >> 4), l = threadIdx.x & 15;
+   double sum = 0.0;
+   if (i < n) {
+      const uint32_t c = i / nv, e = i - c * nv;
+      const double* p = part + (size_t)c * split * nv + e;
+#pragma unroll
+      for (uint32_t u = 0; u < CELL_SPLIT_MAX / 16; ++u) {
+         const uint32_t k = l + 16 * u;
+         sum += (k < split) ? p[(size_t)k * nv] : 0.0;
+      }
+   }
+   for (int o = 8; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 16);
+   if (l == 0 && i < n) out[i] = sum * scale;
+}
+
+// One workgroup's NV sums (red[e][wave]): the cell's result times scale when the cell has one
+// workgroup, otherwise its part for k_cell_parts.
+template <int NV>
+__device__ inline void put_cell_sums(const double (*red)[WG / 64], double* part, double* out, uint32_t split, double scale) {
+   const int t = threadIdx.x;
+   if (t < NV) {
+      double sum = 0.0;
+      for (int w = 0; w < WG / 64; ++w) sum += red[t][w];
+      if (split == 1) out[(size_t)NV * blockIdx.x + t] = sum * scale;
+      else part[(size_t)NV * blockIdx.x + t] = sum;
+   }
+}
+
 // Second moments of one population about a pivot (arch_moments.h:123-150), split workgroups
 // per cell (blockIdx.x), 16 lanes per block and one float4 row (i = 0..3 at fixed j, k) per
 // lane, UNR blocks per lane group in flight.  With X the offset of the row's first cell from the
 // pivot along x and h the cell size, the row's sums S = sum f, A = sum i f, B = sum i^2 f give
 //   sum f dx = X S + h A,   sum f dx^2 = X (X S + 2 h A) + h^2 B,
 // and dy, dz are the row's: about 30 FP64 operations per row of four cells instead of 15 per
-// cell.  Each workgroup writes its six FP64 sums to part; k_cell_parts adds a cell's parts in
+// cell.  Each workgroup writes its six FP64 sums to a.part; k_cell_parts adds a cell's parts in
 // order, so the result does not depend on the schedule.
 // Bound by HBM reads (256 bytes per block).  The form before it, a wave per block with one
 // lane per cell, one block in flight and one workgroup per cell, was bound by the latency of
 // each block's loads and by the largest cell: 3.92 -> 1.36 ms over 26 million FP32 blocks in
 // 8192 cells (5.0 TB/s), 1.15 -> 0.022 ms over 64 cells of 300 to 20000 blocks.
 template <int ST>
-__global__ __launch_bounds__(WG) void k_pressure(MomentArgs a, const double* pivot, double* part, uint32_t split) {
+__global__ __launch_bounds__(WG) void k_pressure(MomentArgs a, const double* pivot, uint32_t split, double mass, double* out) {
    __shared__ double red[6][WG / 64];
    const int t = threadIdx.x;
    const uint32_t c = blockIdx.x / split, sp = blockIdx.x - c * split;
@@ -1553,22 +1586,7 @@ __global__ __launch_bounds__(WG) void k_pressure(MomentArgs a, const double* piv
       if ((t & 63) == 0) red[e][t >> 6] = s[e];
    }
    __syncthreads();
-   if (t < 6) {
-      double sum = 0.0;
-      for (int w = 0; w < WG / 64; ++w) sum += red[t][w];
-      part[6 * (size_t)blockIdx.x + t] = sum;
-   }
-}
-
-// out[nv c + e] = scale * sum over the cell's parts, in order: part[(c split + p) nv + e]
-__global__ void k_cell_parts(const double* part, uint32_t split, uint32_t nv, uint32_t n, double scale, double* out) {
-   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-   if (i >= n) return;
-   const uint32_t c = i / nv, e = i - c * nv;
-   const double* p = part + (size_t)c * split * nv + e;
-   double sum = 0.0;
-   for (uint32_t k = 0; k < split; ++k) sum += p[(size_t)k * nv];
-   out[i] = sum * scale;
+   put_cell_sums<6>(red, a.part, out, split, mass * (a.cell[0] * a.cell[1] * a.cell[2]));
 }
 
 // spatial_cell_cpu.cpp:699-727
@@ -1666,16 +1684,16 @@ __global__ __launch_bounds__(WG) void k_cell_scale(const uint32_t* off, const ui
 // ---------------------------------------------------------------------------
 
 template <int ST>
-__global__ __launch_bounds__(WG) void k_moments(MomentArgs a) {
-   // One workgroup per cell; 16 lanes per block, each lane one float4 (i = 0..3 at fixed j, k),
-   // UNR blocks per 16-lane group in flight.  Per value the reference adds f*DV3, f*VX*DV3, ...
+__global__ __launch_bounds__(WG) void k_moments(MomentArgs a, uint32_t split) {
+   // split workgroups per cell (their sums to a.part, added in order by k_cell_parts); 16 lanes per
+   // block, each lane one float4 (i = 0..3 at fixed j, k), UNR blocks per 16-lane group in flight.  Per value the reference adds f*DV3, f*VX*DV3, ...
    // (arch_moments.h:98-108); here DV3 is applied once to the cell's FP64 sums.  A lane keeps
    // per row the sum S and the index-weighted sum W = f1 + 2 f2 + 3 f3, and accumulates S, W and
    // S times the block's corner velocity; its fixed offsets within the block (x: 0.5 dv and W dv,
    // y, z: (j, k) + 0.5 cells) are applied once at the end.
    __shared__ double red[4][WG / 64];
    const int t = threadIdx.x;
-   const uint32_t c = blockIdx.x;
+   const uint32_t c = blockIdx.x / split, sp = blockIdx.x - c * split;
    const uint32_t off = a.cell_off[c];
    const uint32_t n = a.cell_off[c + 1] - off;
    const int q = t & 15;
@@ -1684,12 +1702,12 @@ __global__ __launch_bounds__(WG) void k_moments(MomentArgs a) {
    double s0 = 0.0, sw = 0.0, sx = 0.0, sy = 0.0, sz = 0.0;
    constexpr uint32_t GROUPS = WG / 16;
    constexpr int UNR = 4;
-   for (uint32_t b = t >> 4; b < n; b += UNR * GROUPS) {
+   for (uint32_t b = sp * GROUPS + (t >> 4); b < n; b += UNR * GROUPS * split) {
       uint32_t sv[UNR], gv[UNR];
       float4 v[UNR];
 #pragma unroll
       for (int h = 0; h < UNR; ++h) {
-         const uint32_t bb = b + h * GROUPS;
+         const uint32_t bb = b + h * GROUPS * split;
          sv[h] = (bb < n) ? a.src[off + bb] : INVALID;
          gv[h] = (bb < n) ? a.gid[off + bb] : 0u;
       }
@@ -1725,31 +1743,26 @@ __global__ __launch_bounds__(WG) void k_moments(MomentArgs a) {
       red[3][t >> 6] = s3;
    }
    __syncthreads();
-   if (t < 4) {
-      const double DV3 = a.cell[0] * a.cell[1] * a.cell[2];
-      double sum = 0.0;
-      for (int w = 0; w < WG / 64; ++w) sum += red[t][w];
-      a.out[4 * (size_t)c + t] = sum * DV3;
-   }
+   put_cell_sums<4>(red, a.part, a.out, split, a.cell[0] * a.cell[1] * a.cell[2]);
 }
 
-// The same moments from the block sums of the last remap pass (MomentArgs::blk_stats): one
-// workgroup per cell, one lane per block, FP64 sums of S, S times the block's corner velocity
+// The same moments from the block sums of the last remap pass (MomentArgs::blk_stats): split
+// workgroups per cell, one lane per block, FP64 sums of S, S times the block's corner velocity
 // and the in-block index sums; the 0.5-cell offsets and DV3 applied once per cell.
-__global__ __launch_bounds__(WG) void k_moments_sums(MomentArgs a) {
+__global__ __launch_bounds__(WG) void k_moments_sums(MomentArgs a, uint32_t split) {
    __shared__ double red[4][WG / 64];
    const int t = threadIdx.x;
-   const uint32_t c = blockIdx.x;
+   const uint32_t c = blockIdx.x / split, sp = blockIdx.x - c * split;
    const uint32_t off = a.cell_off[c];
    const uint32_t n = a.cell_off[c + 1] - off;
    const double bx = a.cell[0] * WID, by = a.cell[1] * WID, bz = a.cell[2] * WID;
    double s0 = 0.0, sx = 0.0, sy = 0.0, sz = 0.0, wx = 0.0, wy = 0.0, wz = 0.0;
    constexpr int UNR = 4;   // blocks per lane in flight
-   for (uint32_t b0 = t; b0 < n; b0 += UNR * WG) {
+   for (uint32_t b0 = sp * WG + t; b0 < n; b0 += UNR * WG * split) {
       uint32_t sidx[UNR], g[UNR];
 #pragma unroll
       for (int h = 0; h < UNR; ++h) {
-         const uint32_t b = b0 + h * WG;
+         const uint32_t b = b0 + h * WG * split;
          sidx[h] = (b < n) ? a.src[off + b] : INVALID;
          g[h] = (b < n) ? a.gid[off + b] : 0u;
       }
@@ -1787,12 +1800,7 @@ __global__ __launch_bounds__(WG) void k_moments_sums(MomentArgs a) {
       red[3][t >> 6] = s3;
    }
    __syncthreads();
-   if (t < 4) {
-      const double DV3 = a.cell[0] * a.cell[1] * a.cell[2];
-      double sum = 0.0;
-      for (int w = 0; w < WG / 64; ++w) sum += red[t][w];
-      a.out[4 * (size_t)c + t] = sum * DV3;
-   }
+   put_cell_sums<4>(red, a.part, a.out, split, a.cell[0] * a.cell[1] * a.cell[2]);
 }
 
 __global__ void k_transform(MeshInfo m, const TransformIn* fields, const double* dt_override, const double* moments,
@@ -2013,12 +2021,31 @@ static uint32_t launch_waves(uint32_t n) {
    return (uint32_t)std::min<uint64_t>(want, 1u << 20);
 }
 
+// Workgroups per cell of the kernels that read a cell's blocks: about CELL_PARTS in all, so
+// that a few cells (or a few large ones among many) still fill the chip.
+uint32_t cell_split(uint32_t ncells) {
+   const uint32_t s = CELL_PARTS / std::max(ncells, 1u);
+   return std::min(std::max(s, 1u), CELL_SPLIT_MAX);
+}
+
+static void launch_parts(const double* part, uint32_t split, uint32_t nv, uint32_t ncells, double scale, double* out,
+                         hipStream_t s) {
+   const uint32_t n = nv * ncells;
+   if (split > 1)
+      hipLaunchKernelGGL(k_cell_parts, dim3((n + WG / 16 - 1) / (WG / 16)), dim3(WG), 0, s, part, split, nv, n, scale, out);
+}
+
 void launch_moments(const MomentArgs& a, hipStream_t s) {
    if (a.ncells == 0) return;
-   if (a.blk_stats) hipLaunchKernelGGL(k_moments_sums, dim3(a.ncells), dim3(WG), 0, s, a);
-   else if (a.pool.storage == ST_F32) hipLaunchKernelGGL(k_moments<ST_F32>, dim3(a.ncells), dim3(WG), 0, s, a);
-   else if (a.pool.storage == ST_BF16) hipLaunchKernelGGL(k_moments<ST_BF16>, dim3(a.ncells), dim3(WG), 0, s, a);
-   else hipLaunchKernelGGL(k_moments<ST_F16>, dim3(a.ncells), dim3(WG), 0, s, a);
+   // the block sums are 24 bytes per block and one lane per block: a workgroup covers 1024 blocks
+   // per round, so a cell is split only while there are fewer cells than resident workgroups
+   const uint32_t split = a.blk_stats ? std::min(std::max(2048u / a.ncells, 1u), 8u) : cell_split(a.ncells);
+   const dim3 grid(a.ncells * split);
+   if (a.blk_stats) hipLaunchKernelGGL(k_moments_sums, grid, dim3(WG), 0, s, a, split);
+   else if (a.pool.storage == ST_F32) hipLaunchKernelGGL(k_moments<ST_F32>, grid, dim3(WG), 0, s, a, split);
+   else if (a.pool.storage == ST_BF16) hipLaunchKernelGGL(k_moments<ST_BF16>, grid, dim3(WG), 0, s, a, split);
+   else hipLaunchKernelGGL(k_moments<ST_F16>, grid, dim3(WG), 0, s, a, split);
+   launch_parts(a.part, split, 4, a.ncells, a.cell[0] * a.cell[1] * a.cell[2], a.out, s);
 }
 
 void launch_transform(const MeshInfo& m, const TransformIn* fields, const double* dt_override, const double* moments,
@@ -2114,23 +2141,17 @@ void launch_fill_f64(double* dst, double v, uint32_t n, hipStream_t s) {
    hipLaunchKernelGGL(k_fill_f64, dim3((n + 255) / 256), dim3(256), 0, s, dst, v, n);
 }
 
-// Workgroups per cell of the kernels that sum over a cell's blocks: about CELL_PARTS in all, so
-// that a few cells (or a few large ones among many) still fill the chip.
-uint32_t cell_split(uint32_t ncells) {
-   const uint32_t s = CELL_PARTS / std::max(ncells, 1u);
-   return std::min(std::max(s, 1u), CELL_SPLIT_MAX);
-}
-
-void launch_pressure(const MomentArgs& a, const double* pivot, double mass, double* part, double* out, hipStream_t s) {
+void launch_pressure(const MomentArgs& a, const double* pivot, double mass, double* out, hipStream_t s) {
    if (a.ncells == 0) return;
    const uint32_t split = cell_split(a.ncells);
    const dim3 grid(a.ncells * split);
-   if (a.pool.storage == ST_F32) hipLaunchKernelGGL(k_pressure<ST_F32>, grid, dim3(WG), 0, s, a, pivot, part, split);
-   else if (a.pool.storage == ST_BF16) hipLaunchKernelGGL(k_pressure<ST_BF16>, grid, dim3(WG), 0, s, a, pivot, part, split);
-   else hipLaunchKernelGGL(k_pressure<ST_F16>, grid, dim3(WG), 0, s, a, pivot, part, split);
-   const double dv3 = a.cell[0] * a.cell[1] * a.cell[2];
-   hipLaunchKernelGGL(k_cell_parts, dim3((6 * a.ncells + 255) / 256), dim3(256), 0, s, part, split, 6u, 6 * a.ncells,
-                      mass * dv3, out);
+   if (a.pool.storage == ST_F32)
+      hipLaunchKernelGGL(k_pressure<ST_F32>, grid, dim3(WG), 0, s, a, pivot, split, mass, out);
+   else if (a.pool.storage == ST_BF16)
+      hipLaunchKernelGGL(k_pressure<ST_BF16>, grid, dim3(WG), 0, s, a, pivot, split, mass, out);
+   else
+      hipLaunchKernelGGL(k_pressure<ST_F16>, grid, dim3(WG), 0, s, a, pivot, split, mass, out);
+   launch_parts(a.part, split, 6, a.ncells, mass * (a.cell[0] * a.cell[1] * a.cell[2]), out, s);
 }
 
 void launch_sparse_min(const SparseArgs& p, const double* moments, const uint32_t* off, double* minval,
