@@ -74,7 +74,7 @@ struct vacc_ctx {
    uint32_t* n_units = nullptr;
    uint32_t* n_tgt = nullptr;
    uint32_t* unit_base = nullptr;
-   uint32_t* len_hist = nullptr;     // [2*LEN_BINS]: histogram, cursors
+   uint32_t* len_hist = nullptr;     // [LEN_BINS]: work units per length bin
    uint32_t* status = nullptr;
    uint32_t* flags = nullptr;
    double* isect = nullptr;
@@ -283,7 +283,7 @@ static int alloc_cells(vacc_ctx* c, uint32_t n) {
    HIPCHK(hipMalloc(&c->n_units, m * sizeof(uint32_t)));
    HIPCHK(hipMalloc(&c->n_tgt, m * sizeof(uint32_t)));
    HIPCHK(hipMalloc(&c->unit_base, m * sizeof(uint32_t)));
-   HIPCHK(hipMalloc(&c->len_hist, 2 * LEN_BINS * sizeof(uint32_t)));
+   HIPCHK(hipMalloc(&c->len_hist, LEN_BINS * sizeof(uint32_t)));
    HIPCHK(hipMalloc(&c->status, m * sizeof(uint32_t)));
    HIPCHK(hipMemset(c->status, 0, m * sizeof(uint32_t)));
    HIPCHK(hipMalloc(&c->isect, m * 12 * sizeof(double)));
@@ -426,7 +426,6 @@ static int enqueue_pass(vacc_ctx* c, int dim, int grid_mult, int wgs = 0, bool s
    ca.col_rec = c->col_rec;
    ca.n_units = c->n_units;
    ca.n_targets = c->n_tgt;
-   ca.len_hist = c->len_hist;
    ca.status = c->status;
    ca.ncells = c->ncells;
    for (int d = 0; d < 3; ++d) ca.len[d] = c->mi.len[d];
@@ -439,25 +438,23 @@ static int enqueue_pass(vacc_ctx* c, int dim, int grid_mult, int wgs = 0, bool s
    ca.cell_hist = c->cell_hist;
    {
       ProfScope ps(c, 1);
-      launch_fill_u32(c->len_hist, 0u, LEN_BINS, c->stream);
       launch_columns(dim, ca, c->stream);
-      ScanArgs sa{};
-      sa.a = c->n_tgt;
-      sa.b = c->n_units;
-      sa.a_off = c->off[lo];
-      sa.b_off = c->unit_base;
-      sa.n = c->ncells;
-      sa.cap_a = (uint32_t)std::min<size_t>(c->cap, 0xFFFFFFFFull);
-      sa.flags = c->flags;
-      sa.hist = c->len_hist;
-      sa.hist_cursor = c->len_hist + LEN_BINS;
-      launch_scan(sa, c->stream);
-      launch_bin_scan(c->cell_hist, c->ncells, c->stream);
+      BuildScanArgs sa{};
+      sa.s.a = c->n_tgt;
+      sa.s.b = c->n_units;
+      sa.s.a_off = c->off[lo];
+      sa.s.b_off = c->unit_base;
+      sa.s.n = c->ncells;
+      sa.s.cap_a = (uint32_t)std::min<size_t>(c->cap, 0xFFFFFFFFull);
+      sa.s.flags = c->flags;
+      sa.cell_hist = c->cell_hist;
+      sa.len_hist = c->len_hist;
+      launch_build_scan(sa, c->stream);
       OrderArgs oa{};
       oa.cell_off = c->off[li];
       oa.unit_base = c->unit_base;
       oa.unit_rec = c->unit_rec;
-      oa.hist_cursor = c->len_hist + LEN_BINS;
+      oa.len_hist = c->len_hist;
       oa.cell_hist = c->cell_hist;
       oa.perm = c->perm;
       oa.perm_cell = c->perm_cell;
@@ -490,6 +487,7 @@ static int enqueue_pass(vacc_ctx* c, int dim, int grid_mult, int wgs = 0, bool s
    ra.min_value = c->sp.sparse_min_value;
    ra.minval = c->minval;
    ra.len_hist = c->len_hist;
+   ra.nblocks = c->nblocks;
    ra.dv_d = c->mi.cell[dim];
    ra.vmin_d = c->mi.vmin[dim];
    ra.blk_stats = (stats && c->blk_stats) ? c->blk_stats : nullptr;

@@ -34,7 +34,10 @@ constexpr uint32_t EXACT_FLAG = 0x40000000u;
 // wide instance of the exact kernel, in either arithmetic form.
 constexpr uint32_t WIDE_FLAG = 0x20000000u;
 constexpr uint32_t UNIT_NCOL_MASK = 0x1FFFFFFFu;
-constexpr int LEN_BINS = 256;   // length bins of the work-unit ordering
+// Length bins of the work-unit ordering (units of LEN_BINS - 3 blocks and more share a bin: what
+// counts is that long units start first).  The column build writes one word per (bin, cell)
+// with a stride of ncells, so the bins are as few as a mesh of 50 to 100 blocks per axis needs.
+constexpr int LEN_BINS = 64;
 // The last two bins hold the units marked EXACT_FLAG and then those marked WIDE_FLAG, so that
 // the work list ends with them: the tolerance-form kernel takes the list up to EXACT_BIN's
 // start, the exact kernel the EXACT_BIN units (or, in the exact form, everything before
@@ -42,7 +45,7 @@ constexpr int LEN_BINS = 256;   // length bins of the work-unit ordering
 constexpr int EXACT_BIN = LEN_BINS - 2;
 constexpr int WIDE_BIN = LEN_BINS - 1;
 // RemapArgs::range of an exact-kernel launch
-enum { RANGE_ALL = 0, RANGE_EXACT = 1, RANGE_WIDE = 2 };
+enum { RANGE_ALL = 0, RANGE_EXACT = 1 };
 
 struct ColumnArgs {
    const uint32_t* cell_off;   // [ncells+1] input list offsets
@@ -53,7 +56,6 @@ struct ColumnArgs {
    uint4* unit_rec;            // [N] at cell_off
    uint4* col_rec;             // [N] at cell_off
    uint32_t* n_units;          // [ncells]
-   uint32_t* len_hist;         // [LEN_BINS] work units per length bin (zeroed before the launch)
    uint32_t* n_targets;        // [ncells]
    uint32_t* status;           // [ncells + 1] OR-ed status bits; entry ncells ORs all cells
    uint32_t ncells;
@@ -75,15 +77,21 @@ struct ScanArgs {
    uint32_t n;
    uint32_t cap_a;         // capacity check on the a total (0 = none)
    uint32_t* flags;        // device flags word: bit VACC_STATUS_CAPACITY set on overflow
-   const uint32_t* hist;   // [LEN_BINS] optional histogram to scan into hist_cursor
-   uint32_t* hist_cursor;
+};
+
+// The scans of one column build: the cells' target and unit counts, and the units per (bin, cell)
+// over cells within each bin.
+struct BuildScanArgs {
+   ScanArgs s;
+   uint32_t* cell_hist;    // [LEN_BINS * ncells] counts, replaced by their exclusive prefix over cells
+   uint32_t* len_hist;     // [LEN_BINS] total of each bin (written)
 };
 
 struct OrderArgs {
    const uint32_t* cell_off;
    const uint32_t* unit_base;   // [ncells+1]
    const uint4* unit_rec;
-   const uint32_t* hist_cursor; // [LEN_BINS] first list position of each length bin
+   const uint32_t* len_hist;    // [LEN_BINS] units per length bin
    const uint32_t* cell_hist;   // [LEN_BINS * ncells] exclusive prefix over cells of the bin's units
    uint32_t* perm;              // [total units] unit record indices (unit_rec), longest first
    uint32_t* perm_cell;         // [total units] the cell of each perm entry
@@ -114,8 +122,11 @@ struct RemapArgs {
    double min_value;            // content test threshold
    const double* minval;        // [ncells] sparsity threshold per cell (velocityBlockMinValue)
    double dv_d, vmin_d;         // cell size and mesh minimum along the pass axis (FP64)
-   int range;                   // exact kernel: RANGE_ALL (every unit before WIDE_BIN's),
-                                // RANGE_EXACT (EXACT_BIN's units), RANGE_WIDE (WIDE_BIN's units)
+   int range;                   // exact kernel: RANGE_ALL (every unit before WIDE_BIN's) or
+                                // RANGE_EXACT (EXACT_BIN's units)
+   uint32_t main_grid;          // exact kernel: workgroups that take the range; the rest of the grid
+                                // takes WIDE_BIN's units
+   uint64_t nblocks;            // source blocks, about (sizes the grid)
    const uint32_t* len_hist;    // [LEN_BINS] units per length bin; [EXACT_BIN] = EXACT_FLAG units,
                                 // [WIDE_BIN] = WIDE_FLAG units
    float4* blk_stats;           // null, or per output block (at its slot) the sums of its stored
@@ -204,7 +215,7 @@ int init_box_words_max();
 void launch_columns(int dim, const ColumnArgs& a, hipStream_t s);
 void launch_scan(const ScanArgs& a, hipStream_t s);
 void launch_order(const OrderArgs& a, hipStream_t s);
-void launch_bin_scan(uint32_t* cell_hist, uint32_t ncells, hipStream_t s);
+void launch_build_scan(const BuildScanArgs& a, hipStream_t s);
 // grid: grid_mult persistent workgroups per CU
 // grid_mult workgroups per compute unit; wgs: lanes per workgroup of the tolerance-form kernel
 // (64, 128 or 256: 4, 8 or 16 work units); the exact kernel always runs 256-lane workgroups

@@ -1,12 +1,13 @@
 // vacc_kernels.hip -- gfx950 kernels of the velocity-space acceleration step.
 //
-// One 1-D remap pass along a dimension is three launches over all cells:
+// One 1-D remap pass along a dimension is four launches over all cells:
 //   k_columns  one workgroup per cell: LDS bitmap counting sort of the cell's
 //              blocks into column sets / columns along the pass axis, target
 //              extents of every column (cpu_acc_map.cpp:250-353) and the
 //              output slot of every target block.
-//   k_scan2    one workgroup: exclusive scans of per-cell set and target
-//              counts (global work list and output offsets).
+//   k_build_scan  exclusive scans over cells of the target and unit counts (output
+//              offsets, work list) and of the units per length bin, then
+//              k_order: the global work list, longest units first.
 //   k_remap    persistent: 16 lanes per column set, one lane per transverse
 //              pencil, walks the columns of the set sourcing the blocks from
 //              HBM once and writing every target block once, with the PLM,
@@ -486,56 +487,50 @@ __global__ __launch_bounds__(CWG, 8) void k_columns(ColumnArgs a) {
          atomicOr(&a.status[a.ncells], sstat);   // OR over all cells
       }
    }
-   for (int i = t; i < LEN_BINS; i += CWG) {
-      a.cell_hist[(size_t)i * a.ncells + c] = hist[i];
-      if (hist[i]) atomicAdd(&a.len_hist[i], hist[i]);
-   }
+   for (int i = t; i < LEN_BINS; i += CWG) a.cell_hist[(size_t)i * a.ncells + c] = hist[i];
 }
 
-// Per length bin (one workgroup each), the exclusive prefix over cells of the cells' unit
-// counts, in place: cell c's units of bin b take list positions from hist_cursor[b] +
-// cell_hist[b][c] on.
-__global__ __launch_bounds__(1024) void k_bin_scan(uint32_t* cell_hist, uint32_t ncells) {
-   constexpr uint32_t K = 8;
-   __shared__ uint32_t sh[16];
-   uint32_t* row = cell_hist + (size_t)blockIdx.x * ncells;
+// ---------------------------------------------------------------------------
+// scans over cells: one workgroup of 1024 threads per scan, tiles of 1024 x SCAN_K entries,
+// SCAN_K contiguous entries per thread
+// ---------------------------------------------------------------------------
+
+constexpr uint32_t SCAN_K = 8;
+
+// exclusive scan of row[0..n) in place; returns the total (in every thread)
+__device__ inline uint32_t scan_row(uint32_t* row, uint32_t n, uint32_t* sh) {
    uint32_t carry = 0;
-   for (uint32_t base = 0; base < ncells; base += 1024 * K) {
-      const uint32_t i0 = base + threadIdx.x * K;
-      uint32_t v[K];
+   for (uint32_t base = 0; base < n; base += 1024 * SCAN_K) {
+      const uint32_t i0 = base + threadIdx.x * SCAN_K;
+      uint32_t v[SCAN_K];
       uint32_t sum[1] = {0u};
 #pragma unroll
-      for (uint32_t k = 0; k < K; ++k) {
-         v[k] = (i0 + k < ncells) ? row[i0 + k] : 0u;
+      for (uint32_t k = 0; k < SCAN_K; ++k) {
+         v[k] = (i0 + k < n) ? row[i0 + k] : 0u;
          sum[0] += v[k];
       }
       uint32_t ex[1], tot[1];
       block_scan<1>(sum, ex, tot, sh);
       uint32_t r = carry + ex[0];
 #pragma unroll
-      for (uint32_t k = 0; k < K; ++k) {
-         if (i0 + k < ncells) row[i0 + k] = r;
+      for (uint32_t k = 0; k < SCAN_K; ++k) {
+         if (i0 + k < n) row[i0 + k] = r;
          r += v[k];
       }
       carry += tot[0];
    }
+   return carry;
 }
 
-// ---------------------------------------------------------------------------
-// k_scan2: exclusive scans of one or two per-cell count arrays
-// ---------------------------------------------------------------------------
-
-__global__ __launch_bounds__(1024) void k_scan2(ScanArgs a) {
-   // tiles of 1024 x K entries, K contiguous entries per thread (one workgroup scan per tile)
-   constexpr uint32_t K = 8;
-   __shared__ uint32_t sh[16 * 2];
+// exclusive scans of one or two per-cell count arrays, and the capacity check
+__device__ inline void scan_counts(const ScanArgs& a, uint32_t* sh) {
    uint32_t carry0 = 0, carry1 = 0;   // running totals, the same in every thread
-   for (uint32_t base = 0; base < a.n; base += 1024 * K) {
-      const uint32_t i0 = base + threadIdx.x * K;
-      uint32_t va[K], vb[K];
+   for (uint32_t base = 0; base < a.n; base += 1024 * SCAN_K) {
+      const uint32_t i0 = base + threadIdx.x * SCAN_K;
+      uint32_t va[SCAN_K], vb[SCAN_K];
       uint32_t v[2] = {0u, 0u};
 #pragma unroll
-      for (uint32_t k = 0; k < K; ++k) {
+      for (uint32_t k = 0; k < SCAN_K; ++k) {
          const uint32_t i = i0 + k;
          va[k] = (i < a.n) ? a.a[i] : 0u;
          vb[k] = (a.b && i < a.n) ? a.b[i] : 0u;
@@ -546,7 +541,7 @@ __global__ __launch_bounds__(1024) void k_scan2(ScanArgs a) {
       block_scan<2>(v, ex, tot, sh);
       uint32_t r0 = carry0 + ex[0], r1 = carry1 + ex[1];
 #pragma unroll
-      for (uint32_t k = 0; k < K; ++k) {
+      for (uint32_t k = 0; k < SCAN_K; ++k) {
          const uint32_t i = i0 + k;
          if (i < a.n) {
             a.a_off[i] = r0;
@@ -563,32 +558,49 @@ __global__ __launch_bounds__(1024) void k_scan2(ScanArgs a) {
       if (a.b) a.b_off[a.n] = carry1;
       if (a.cap_a && carry0 > a.cap_a && a.flags) atomicOr(a.flags, VACC_STATUS_CAPACITY);
    }
-   if (a.hist) {
-      // exclusive scan of the work-unit length histogram -> insertion cursors of k_order
-      uint32_t v[2] = {threadIdx.x < LEN_BINS ? a.hist[threadIdx.x] : 0u, 0u};
-      uint32_t ex[2], tot[2];
-      block_scan<2>(v, ex, tot, sh);
-      if (threadIdx.x < LEN_BINS) a.hist_cursor[threadIdx.x] = ex[0];
+}
+
+__global__ __launch_bounds__(1024) void k_scan2(ScanArgs a) {
+   __shared__ uint32_t sh[16 * 2];
+   scan_counts(a, sh);
+}
+
+// The scans of a column build in one launch: workgroup b < LEN_BINS turns bin b's unit counts into
+// their exclusive prefix over cells (cell c's units of bin b take the bin's list positions from
+// cell_hist[b][c] on) and stores the bin's total; the last workgroup scans the cells' target
+// and unit counts.  One launch in place of a fill, a scan per kind and their gaps: in a small
+// batch each of them is a launch of about 4.6 us.
+__global__ __launch_bounds__(1024) void k_build_scan(BuildScanArgs a) {
+   __shared__ uint32_t sh[16 * 2];
+   if (blockIdx.x == LEN_BINS) {
+      scan_counts(a.s, sh);
+      return;
    }
+   const uint32_t tot = scan_row(a.cell_hist + (size_t)blockIdx.x * a.s.n, a.s.n, sh);
+   if (threadIdx.x == 0) a.len_hist[blockIdx.x] = tot;
 }
 
 // Global work list of the remap: every unit's global index, ordered by source length
 // (longest first; within a length bin by cell, units are independent).
 __global__ __launch_bounds__(WG) void k_order(OrderArgs a) {
-   // one workgroup per cell: the cell's range in each bin is known (hist_cursor + the bin's
-   // prefix over cells); units take positions in it through an LDS counter per bin
-   __shared__ uint32_t cnt[LEN_BINS];
+   // one workgroup per cell: the cell's range in each bin starts at the units of the bins before it
+   // plus the bin's prefix over cells; units take positions in it through an LDS cursor per bin
+   static_assert(LEN_BINS == 64, "one wave scans the bins");
+   __shared__ uint32_t cursor[LEN_BINS];
    if (*a.flags & VACC_STATUS_CAPACITY) return;
    const uint32_t c = blockIdx.x;
    const uint32_t base = a.unit_base[c];
    const uint32_t nu = a.unit_base[c + 1] - base;
    if (nu == 0) return;
    const uint32_t off = a.cell_off[c];
-   for (int i = threadIdx.x; i < LEN_BINS; i += WG) cnt[i] = 0;
+   if (threadIdx.x < LEN_BINS) {
+      const uint32_t n = a.len_hist[threadIdx.x];
+      cursor[threadIdx.x] = wave_incl_scan(n) - n + a.cell_hist[(size_t)threadIdx.x * a.ncells + c];
+   }
    __syncthreads();
    for (uint32_t u = threadIdx.x; u < nu; u += WG) {
       const uint32_t b = unit_bin(a.unit_rec[off + u]);
-      const uint32_t pos = a.hist_cursor[b] + a.cell_hist[(size_t)b * a.ncells + c] + atomicAdd(&cnt[b], 1u);
+      const uint32_t pos = atomicAdd(&cursor[b], 1u);
       a.perm[pos] = off + u;   // the unit's record
       a.perm_cell[pos] = c;
    }
@@ -814,25 +826,18 @@ __device__ inline void copy_block(const RemapArgs& a, int l16, int setlane0, int
    }
 }
 
-// RN-cell ring per lane in workgroups of WGS lanes: RING / WG for the work list, RING_WIDE /
-// WG_WIDE for the units of wide-span cells (range RANGE_WIDE)
+// Exact remap of the work-list entries [first, total), the workgroup being `block` of `blocks`:
+// RN-cell ring per lane, WGS lanes per workgroup.
 template <int DIM, int METHOD, int ST, int RN, int WGS>
-__global__ __launch_bounds__(WGS) void k_remap(RemapArgs a, double i_dv) {
-   __shared__ float ring[RN][WGS];
-   if (*a.flags & VACC_STATUS_CAPACITY) return;
+__device__ __forceinline__ void remap_units(const RemapArgs& a, double i_dv, float (*ring)[WGS], uint32_t first,
+                                            uint32_t total, uint32_t block, uint32_t blocks) {
    const int tid = threadIdx.x;
    const int l16 = tid & 15;
    const int ip = l16 & 3, jp = l16 >> 2;
    const int setlane0 = (tid & 63) & ~15;
    const int o = (DIM == 0) ? (ip * WID2 + jp * WID) : (DIM == 1) ? (jp * WID2 + ip) : (jp * WID + ip);
-   // the list ends with the EXACT_BIN units and then the WIDE_BIN units
-   const uint32_t all = a.unit_base[a.ncells], nwide = a.len_hist[WIDE_BIN];
-   const uint32_t first = (a.range == RANGE_WIDE)    ? all - nwide
-                          : (a.range == RANGE_EXACT) ? all - nwide - a.len_hist[EXACT_BIN]
-                                                     : 0u;
-   const uint32_t total = (a.range == RANGE_WIDE) ? all : all - nwide;
-   const uint32_t gstride = gridDim.x * (WGS / 16);
-   for (uint32_t gi = first + blockIdx.x * (WGS / 16) + (tid >> 4); gi < total; gi += gstride) {
+   const uint32_t gstride = blocks * (WGS / 16);
+   for (uint32_t gi = first + block * (WGS / 16) + (tid >> 4); gi < total; gi += gstride) {
       const uint32_t c = a.perm_cell[gi];
       const uint4 sr = a.unit_rec[a.perm[gi]];
       const int b0 = (int)(sr.x & 0xFFFFu), b1 = (int)(sr.x >> 16);
@@ -965,6 +970,26 @@ __global__ __launch_bounds__(WGS) void k_remap(RemapArgs a, double i_dv) {
          carry_open = (next_open > nfk) ? next_open : -1;
          prev_end = max(prev_end, lk);
       }
+   }
+}
+
+// The exact remap: workgroups below a.main_grid take the work list up to the WIDE_BIN units (or
+// only the EXACT_BIN units, a.range), the others the units of wide-span cells (the end of the
+// list) with a RING_WIDE-cell ring per lane in their first WG_WIDE lanes.  Most passes have no
+// such units; a launch of their own cost every pass 4.6 us.
+template <int DIM, int METHOD, int ST>
+__global__ __launch_bounds__(WG) void k_remap(RemapArgs a, double i_dv) {
+   __shared__ float lds[RING * WG];
+   static_assert(RING_WIDE * WG_WIDE <= RING * WG, "the wide ring shares the LDS");
+   if (*a.flags & VACC_STATUS_CAPACITY) return;
+   const uint32_t all = a.unit_base[a.ncells], nwide = a.len_hist[WIDE_BIN];
+   if (blockIdx.x < a.main_grid) {
+      const uint32_t first = (a.range == RANGE_EXACT) ? all - nwide - a.len_hist[EXACT_BIN] : 0u;
+      remap_units<DIM, METHOD, ST, RING, WG>(a, i_dv, reinterpret_cast<float(*)[WG]>(lds), first, all - nwide, blockIdx.x,
+                                             a.main_grid);
+   } else if (nwide && threadIdx.x < WG_WIDE) {
+      remap_units<DIM, METHOD, ST, RING_WIDE, WG_WIDE>(a, i_dv, reinterpret_cast<float(*)[WG_WIDE]>(lds), all - nwide, all,
+                                                       blockIdx.x - a.main_grid, gridDim.x - a.main_grid);
    }
 }
 
@@ -1928,9 +1953,9 @@ void launch_order(const OrderArgs& a, hipStream_t s) {
    hipLaunchKernelGGL(k_order, dim3(a.ncells), dim3(WG), 0, s, a);
 }
 
-void launch_bin_scan(uint32_t* cell_hist, uint32_t ncells, hipStream_t s) {
-   if (ncells == 0) return;
-   hipLaunchKernelGGL(k_bin_scan, dim3(LEN_BINS), dim3(1024), 0, s, cell_hist, ncells);
+void launch_build_scan(const BuildScanArgs& a, hipStream_t s) {
+   if (a.s.n == 0) return;
+   hipLaunchKernelGGL(k_build_scan, dim3(LEN_BINS + 1), dim3(1024), 0, s, a);
 }
 
 void launch_scan(const ScanArgs& a, hipStream_t s) {
@@ -1950,10 +1975,10 @@ int device_cus() {
 
 template <int DIM, int METHOD, int ST>
 static void remap_dms(RemapArgs a, uint32_t grid, double i_dv, bool fast, int wgs, hipStream_t s) {
-   if (!fast) {
-      a.range = RANGE_ALL;
-      hipLaunchKernelGGL((k_remap<DIM, METHOD, ST, RING, WG>), dim3(grid), dim3(WG), 0, s, a, i_dv);
-   } else {
+   const uint32_t cus = (uint32_t)device_cus();
+   a.range = RANGE_ALL;
+   a.main_grid = grid;
+   if (fast) {
       // tolerance form: the lean kernel (workgroups of wgs lanes, wgs/16 work units each), then
       // the exact kernel over the few units it leaves
       // (with block sums: their own instance, whose extra registers the other passes do not carry)
@@ -1967,12 +1992,9 @@ static void remap_dms(RemapArgs a, uint32_t grid, double i_dv, bool fast, int wg
          else hipLaunchKernelGGL((k_remap_lean<DIM, METHOD, ST, WG, false>), dim3(grid), dim3(WG), 0, s, a);
       }
       a.range = RANGE_EXACT;
-      hipLaunchKernelGGL((k_remap<DIM, METHOD, ST, RING, WG>), dim3((uint32_t)device_cus()), dim3(WG), 0, s, a, i_dv);
+      a.main_grid = cus;
    }
-   // the units of wide-span cells (none in most passes: the launch then exits at once)
-   a.range = RANGE_WIDE;
-   hipLaunchKernelGGL((k_remap<DIM, METHOD, ST, RING_WIDE, WG_WIDE>), dim3((uint32_t)device_cus()), dim3(WG_WIDE), 0, s,
-                      a, i_dv);
+   hipLaunchKernelGGL((k_remap<DIM, METHOD, ST>), dim3(a.main_grid + cus), dim3(WG), 0, s, a, i_dv);
 }
 
 template <int DIM, int METHOD>
@@ -1993,7 +2015,12 @@ static void remap_d(int method, const RemapArgs& a, uint32_t grid, double i_dv, 
 
 void launch_remap(int dim, int method, bool fast, RemapArgs a, int grid_mult, int wgs, hipStream_t s) {
    if (a.ncells == 0) return;
-   const uint32_t grid = (uint32_t)device_cus() * (uint32_t)std::max(grid_mult, 1);
+   // the kernels walk the list with a grid stride, so any grid is right; units are columns of at
+   // least one block, so workgroups beyond nblocks / (units per workgroup) would find nothing (for
+   // 16 cells of 600 blocks 32768 empty workgroups took longer than the others)
+   const uint32_t cus = (uint32_t)device_cus(), per = (uint32_t)(fast ? wgs : WG) / 16u;
+   const uint64_t most = std::max<uint64_t>(((uint64_t)a.nblocks + per - 1) / per, cus);
+   const uint32_t grid = (uint32_t)std::min<uint64_t>((uint64_t)cus * (uint32_t)std::max(grid_mult, 1), most);
    const double i_dv = 1.0 / (double)a.dv;   // cpu_acc_map.cpp:201, Real i_dv = 1.0/dv
    if (dim == 0) remap_d<0>(method, a, grid, i_dv, fast, wgs, s);
    else if (dim == 1) remap_d<1>(method, a, grid, i_dv, fast, wgs, s);
