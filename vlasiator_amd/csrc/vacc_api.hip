@@ -81,7 +81,7 @@ struct vacc_ctx {
    TransformIn* fields = nullptr;
    double* moments = nullptr;
    double* parts = nullptr;          // [6*parts_max(ncells)] partial sums of the moment kernels
-   double* press = nullptr;          // [9*ncells] pressure tensor, and the caller's pivot
+   double* press = nullptr;          // [3*ncells] the caller's pivot of vacc_pressure
    double* pivot = nullptr;          // [4*ncells] plasma pivot of a multi-population step
    double* rho_loss = nullptr;
    // subcycling (vacc_subcycle_count / vacc_subcycle_step): per cell max_v_dt, subcycle count,
@@ -127,7 +127,13 @@ struct vacc_ctx {
    int remap_wgs[3] = {256, 256, 256};    // lanes per workgroup of the tolerance-form remap (vacc_autotune)
    int remap_mult_s[3] = {128, 128, 128}; // the same for the passes that store block sums (their own
    int remap_wgs_s[3] = {256, 256, 256};  // kernel instance, with more registers in scratch)
-   uint32_t* h_sum = nullptr;        // pinned host words: capacity flag, block total, status OR
+   // Pinned host memory that kernels write results to (the d_ pointers are its device addresses):
+   // h_sum: capacity flag, block total, status OR, subcycle count; h_res: [6*ncells] per-cell
+   // results of a call; stage: small transfers in either direction, allocated on first use
+   uint32_t *h_sum = nullptr, *d_sum = nullptr;
+   double *h_res = nullptr, *d_res = nullptr;
+   uint8_t *stage = nullptr, *d_stage = nullptr;
+   size_t stage_used = 0;            // bytes handed out since the stream was last waited for
    // streamed block transfer (vacc_blocks_io.h): two pinned chunks, their copy events and,
    // for the 16-bit forms, a device FP32 stage of two chunks; allocated on first use
    float* io_pin[2] = {nullptr, nullptr};
@@ -256,6 +262,8 @@ static void free_cells(vacc_ctx* c) {
    c->keep_box = nullptr;
    c->cell_hist = nullptr;
    c->parts = c->press = nullptr;
+   if (c->h_res) (void)hipHostFree(c->h_res);
+   c->h_res = c->d_res = nullptr;
    c->sub_maxdt = c->sub_dt = nullptr;
    c->sub_n = c->sub_nmax = nullptr;
    c->minval = c->csum_pre = c->csum_post = nullptr;
@@ -293,7 +301,9 @@ static int alloc_cells(vacc_ctx* c, uint32_t n) {
    HIPCHK(hipMalloc(&c->pivot, m * 4 * sizeof(double)));
    HIPCHK(hipMalloc(&c->rho_loss, m * sizeof(double)));
    HIPCHK(hipMalloc(&c->parts, 6 * parts_max(n) * sizeof(double)));
-   HIPCHK(hipMalloc(&c->press, 9 * m * sizeof(double)));
+   HIPCHK(hipMalloc(&c->press, 3 * m * sizeof(double)));
+   HIPCHK(hipHostMalloc(&c->h_res, 6 * m * sizeof(double), hipHostMallocDefault));
+   HIPCHK(hipHostGetDevicePointer((void**)&c->d_res, c->h_res, 0));
    HIPCHK(hipMalloc(&c->sub_maxdt, m * sizeof(double)));
    HIPCHK(hipMalloc(&c->sub_dt, m * sizeof(double)));
    HIPCHK(hipMalloc(&c->sub_n, m * sizeof(uint32_t)));
@@ -390,7 +400,9 @@ static int ensure_blocks(vacc_ctx* c, size_t want) {
    return 0;
 }
 
-// Read the total block count of the current list (synchronises the stream).
+// Read the total block count of the current list (synchronises the stream).  Every call that
+// changes the list ends with the count known (finish, a load), so only the synthetic initial
+// state, which sizes its buffers by it, reads it here.
 static int refresh_count(vacc_ctx* c) {
    uint32_t tot = 0;
    HIPCHK(hipMemcpyAsync(&tot, c->off[c->lcur] + c->ncells, sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
@@ -534,7 +546,7 @@ struct SpatialIn {
 // Rebuild the list: add_width >= 0 is the sparsity adjust, add_width < 0 a re-sort by GID.
 // With spatial-neighbour inputs the kept count can exceed the reserve: the total is read back
 // after the count phase and the block storage grown before the write phase.
-static void enqueue_moments(vacc_ctx* c);
+static void enqueue_moments(vacc_ctx* c, double* host = nullptr);
 
 static int do_relist(vacc_ctx* c, int add_width, bool want_loss, const SpatialIn* sp = nullptr) {
    ProfScope ps(c, add_width >= 0 ? 2 : 4);
@@ -622,25 +634,67 @@ static int do_relist(vacc_ctx* c, int add_width, bool want_loss, const SpatialIn
 // Compact the pool so that src is the identity (block i of the list at pool index i).
 static int do_compact(vacc_ctx* c) {
    launch_gather(c->src[c->lcur], pool(c, c->fcur), pool(c, 1 - c->fcur), (uint32_t)c->nblocks, c->stream);
-   launch_iota(c->src[c->lcur], (uint32_t)c->nblocks, c->stream);
    HIPCHK(hipGetLastError());
    c->fcur = 1 - c->fcur;
    c->stats_valid = false;   // the pool was gathered
    return 0;
 }
 
-// The one synchronisation of a work call: reads the capacity flag, the block total of the
-// current list and the OR of the cell status words (kept in status[ncells]) with three small
-// copies into pinned memory.  Returns the status OR or an error.
-static int finish(vacc_ctx* c) {
-   HIPCHK(hipMemcpyAsync(c->h_sum + 0, c->flags, sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
-   HIPCHK(hipMemcpyAsync(c->h_sum + 1, c->off[c->lcur] + c->ncells, sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
-   HIPCHK(hipMemcpyAsync(c->h_sum + 2, c->status + c->ncells, sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
+// The end of a work call: one small kernel writes the capacity flag, the block total of the current
+// list, the OR of the cell status words (kept in status[ncells]) and, when asked for, the removed
+// mass per cell into pinned memory, and the host waits once.  (Three copies and, after the wait, a
+// copy of the removed mass into the caller's pageable array took 4 launches and a second wait,
+// 40 us of every small step.)  Returns the status OR or an error.
+static int finish_enqueue(vacc_ctx* c, bool loss) {
+   launch_finish(c->flags, c->off[c->lcur] + c->ncells, c->status + c->ncells, c->d_sum, loss ? c->rho_loss : nullptr,
+                 c->d_res, c->ncells, c->stream);
+   HIPCHK(hipGetLastError());
+   return 0;
+}
+
+static int finish_wait(vacc_ctx* c, double* rho_loss) {
    HIPCHK(hipStreamSynchronize(c->stream));
+   c->stage_used = 0;
    if (c->h_sum[0] & VACC_STATUS_CAPACITY)
       return set_err(VACC_E_STATE, "block pool capacity exceeded; state is undefined");
    c->nblocks = c->h_sum[1];
+   if (rho_loss) std::memcpy(rho_loss, c->h_res, c->ncells * sizeof(double));
    return (int)(c->h_sum[2] & 0x7FFFFFFFu);
+}
+
+static int finish(vacc_ctx* c, double* rho_loss = nullptr) {
+   const int rc = finish_enqueue(c, rho_loss != nullptr);
+   return rc ? rc : finish_wait(c, rho_loss);
+}
+
+// Staging of small transfers: `bytes` of pinned memory (host address; *dev the device address),
+// or null when they don't fit.  What was handed out stays in use until the stream has been waited
+// for (stage_used = 0 after a wait); a call that failed in between is waited for here.
+constexpr size_t STAGE_BYTES = 1u << 20;
+static uint8_t* stage_take(vacc_ctx* c, size_t bytes, uint8_t** dev) {
+   const size_t want = (bytes + 255) & ~(size_t)255;
+   if (want > STAGE_BYTES) return nullptr;
+   if (!c->stage) {
+      if (hipHostMalloc(&c->stage, STAGE_BYTES, hipHostMallocDefault) != hipSuccess ||
+          hipHostGetDevicePointer((void**)&c->d_stage, c->stage, 0) != hipSuccess) {
+         (void)hipGetLastError();
+         if (c->stage) (void)hipHostFree(c->stage);
+         c->stage = nullptr;
+         return nullptr;
+      }
+   }
+   if (c->stage_used + want > STAGE_BYTES) return nullptr;
+   uint8_t* h = c->stage + c->stage_used;
+   *dev = c->d_stage + c->stage_used;
+   c->stage_used += want;
+   return h;
+}
+
+// Waits for what an earlier call left in the staging (nothing unless that call failed).
+static int stage_begin(vacc_ctx* c) {
+   if (c->stage_used) HIPCHK(hipStreamSynchronize(c->stream));
+   c->stage_used = 0;
+   return 0;
 }
 
 // OR of the per-cell status words (synchronises the stream).
@@ -712,15 +766,11 @@ static void abort_load(vacc_ctx* c) {
    c->content_valid = c->moments_valid = c->fields_valid = c->sub_valid = c->stats_valid = false;
 }
 
-// First half of a load of new cells: checks the lists, sizes the buffers and copies the
-// offsets and GIDs; the caller then fills pool F[0] and calls end_load, or abort_load when
-// that fails.
-static int begin_load(vacc_ctx* c, uint32_t ncells, const uint64_t* offsets, const uint32_t* gids) {
+// First part of a load of new cells: checks the lists and sizes the buffers.
+static int prepare_load(vacc_ctx* c, uint32_t ncells, const uint64_t* offsets, const uint32_t* gids) {
    int rc = check_load(c, ncells, offsets, gids);
    if (rc) return rc;
    const uint64_t total = offsets[ncells];
-   std::vector<uint32_t> off32(ncells + 1);
-   for (uint32_t i = 0; i <= ncells; ++i) off32[i] = (uint32_t)offsets[i];
    // from here on a failure empties the context
    c->content_valid = c->moments_valid = c->fields_valid = c->sub_valid = c->stats_valid = false;
    rc = alloc_cells(c, ncells);
@@ -741,6 +791,17 @@ static int begin_load(vacc_ctx* c, uint32_t ncells, const uint64_t* offsets, con
    c->fcur = 0;
    c->sorted = false;
    c->cell_epoch++;
+   return 0;
+}
+
+// First half of a load: checks, buffers, and the copy of the offsets and GIDs; the caller then
+// fills pool F[0] and calls end_load, or abort_load when that fails.
+static int begin_load(vacc_ctx* c, uint32_t ncells, const uint64_t* offsets, const uint32_t* gids) {
+   const int rc = prepare_load(c, ncells, offsets, gids);
+   if (rc) return rc;
+   const uint64_t total = offsets[ncells];
+   std::vector<uint32_t> off32(ncells + 1);
+   for (uint32_t i = 0; i <= ncells; ++i) off32[i] = (uint32_t)offsets[i];
    hipError_t e = hipMemcpyAsync(c->off[0], off32.data(), (ncells + 1) * sizeof(uint32_t), hipMemcpyHostToDevice,
                                  c->stream);
    if (e == hipSuccess && total)
@@ -751,6 +812,11 @@ static int begin_load(vacc_ctx* c, uint32_t ncells, const uint64_t* offsets, con
       return set_err(VACC_E_HIP, std::string("load of the block lists: ") + hipGetErrorString(e));
    }
    return 0;
+}
+
+static void loaded(vacc_ctx* c, uint64_t total) {
+   c->nblocks = total;
+   c->content_valid = c->moments_valid = c->stats_valid = c->fields_valid = c->sub_valid = false;
 }
 
 static int end_load(vacc_ctx* c, uint64_t total) {
@@ -765,12 +831,57 @@ static int end_load(vacc_ctx* c, uint64_t total) {
       abort_load(c);
       return set_err(VACC_E_HIP, std::string("end of load: ") + hipGetErrorString(e));
    }
-   c->nblocks = total;
-   c->content_valid = false;
-   c->moments_valid = false;
-   c->stats_valid = false;
-   c->fields_valid = false;
-   c->sub_valid = false;
+   loaded(c, total);
+   return 0;
+}
+
+// A small FP32 load (lists and f fit the staging): one kernel reads the staging over the bus and
+// fills the lists, the pool, the thresholds and the status words, with one wait.  1: not taken.
+static int load_staged(vacc_ctx* c, uint32_t ncells, const uint64_t* offsets, const uint32_t* gids, const float* f) {
+   const uint64_t total = offsets[ncells];
+   if (c->opt.storage != VACC_STORE_F32 || total * (WID3 + 1) * sizeof(float) > STAGE_BYTES) return 1;
+   int rc = stage_begin(c);
+   if (rc) return rc;
+   uint8_t *d_off = nullptr, *d_gid = nullptr, *d_f = nullptr;
+   uint32_t* h_off = reinterpret_cast<uint32_t*>(stage_take(c, (ncells + 1) * sizeof(uint32_t), &d_off));
+   uint8_t* h_gid = stage_take(c, total * sizeof(uint32_t), &d_gid);
+   uint8_t* h_f = stage_take(c, total * WID3 * sizeof(float), &d_f);
+   if (!h_off || !h_gid || !h_f) {
+      c->stage_used = 0;   // nothing was enqueued
+      return 1;
+   }
+   if ((rc = prepare_load(c, ncells, offsets, gids))) {
+      c->stage_used = 0;
+      return rc;
+   }
+   for (uint32_t i = 0; i <= ncells; ++i) h_off[i] = (uint32_t)offsets[i];
+   if (total) {
+      std::memcpy(h_gid, gids, total * sizeof(uint32_t));
+      std::memcpy(h_f, f, total * WID3 * sizeof(float));
+   }
+   LoadArgs la{};
+   la.off_in = reinterpret_cast<const uint32_t*>(d_off);
+   la.gid_in = reinterpret_cast<const uint32_t*>(d_gid);
+   la.f_in = reinterpret_cast<const float4*>(d_f);
+   la.off = c->off[0];
+   la.gid = c->gid[0];
+   la.src = c->src[0];
+   la.f = static_cast<float4*>(c->f[0]);
+   la.minval = c->minval;
+   la.min_value = c->sp.sparse_min_value;
+   la.status = c->status;
+   la.flags = c->flags;
+   la.n = (uint32_t)total;
+   la.ncells = ncells;
+   launch_load(la, c->stream);
+   hipError_t e = hipGetLastError();
+   if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+   c->stage_used = 0;
+   if (e != hipSuccess) {
+      abort_load(c);
+      return set_err(VACC_E_HIP, std::string("upload: ") + hipGetErrorString(e));
+   }
+   loaded(c, total);
    return 0;
 }
 
@@ -1355,6 +1466,7 @@ int vacc_create(const vacc_mesh* mesh, const vacc_species* species, const vacc_o
    if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess ||
        hipMalloc(&c->flags, sizeof(uint32_t)) != hipSuccess || hipMemset(c->flags, 0, sizeof(uint32_t)) != hipSuccess ||
        hipHostMalloc(&c->h_sum, 4 * sizeof(uint32_t), hipHostMallocDefault) != hipSuccess ||
+       hipHostGetDevicePointer((void**)&c->d_sum, c->h_sum, 0) != hipSuccess ||
        hipEventCreateWithFlags(&c->mom_ev, hipEventDisableTiming) != hipSuccess) {
       delete c;
       return set_err(VACC_E_HIP, "stream/flag allocation failed");
@@ -1377,6 +1489,7 @@ int vacc_destroy(vacc_ctx* c) {
    if (c->prof_counts) (void)hipFree(c->prof_counts);
    if (c->flags) (void)hipFree(c->flags);
    if (c->h_sum) (void)hipHostFree(c->h_sum);
+   if (c->stage) (void)hipHostFree(c->stage);
    if (c->mom_ev) (void)hipEventDestroy(c->mom_ev);
    for (int i = 0; i < 2; ++i) {
       if (c->io_pin[i]) (void)hipHostFree(c->io_pin[i]);
@@ -1398,7 +1511,9 @@ int vacc_destroy(vacc_ctx* c) {
 
 int vacc_upload_cells(vacc_ctx* c, uint32_t ncells, const uint64_t* offsets, const uint32_t* gids, const float* f) {
    if (!c || !offsets || (ncells && (!gids || !f))) return set_err(VACC_E_ARG, "null argument");
-   int rc = begin_load(c, ncells, offsets, gids);
+   int rc = load_staged(c, ncells, offsets, gids, f);
+   if (rc <= 0) return rc;
+   rc = begin_load(c, ncells, offsets, gids);
    if (rc) return rc;
    const uint64_t total = offsets[ncells];
    if (total) {
@@ -1452,17 +1567,39 @@ int vacc_get_counts(vacc_ctx* c, uint32_t* ncells, uint32_t* counts) {
 
 int vacc_download_cells(vacc_ctx* c, uint64_t* offsets, uint32_t* gids, float* f) {
    if (!c || !offsets) return set_err(VACC_E_ARG, "null argument");
-   int rc = refresh_count(c);
+   if (!c->off[0]) return set_err(VACC_E_HIP, "the context holds no lists: nothing was loaded");
+   int rc = stage_begin(c);
    if (rc) return rc;
    rc = do_relist(c, -1, false);    // ascending GID order, same blocks
    if (rc) return rc;
    rc = do_compact(c);
    if (rc) return rc;
+   const size_t n = c->nblocks;
+   const size_t f_bytes = (n && f) ? n * WID3 * sizeof(float) : 0, g_bytes = (n && gids) ? n * sizeof(uint32_t) : 0;
+   uint8_t *d_off = nullptr, *d_gid = nullptr, *d_f = nullptr;
+   uint8_t* h_off = stage_take(c, (c->ncells + 1) * sizeof(uint32_t), &d_off);
+   uint8_t* h_gid = h_off ? stage_take(c, g_bytes, &d_gid) : nullptr;
+   uint8_t* h_f = h_gid ? stage_take(c, f_bytes, &d_f) : nullptr;
+   if (h_f) {
+      // everything fits the staging: the kernels write it there, one wait, then host copies
+      const bool f32 = c->opt.storage == VACC_STORE_F32;
+      launch_unload(c->off[c->lcur], c->gid[c->lcur], (f32 && f_bytes) ? static_cast<const float4*>(c->f[c->fcur]) : nullptr,
+                    reinterpret_cast<uint32_t*>(d_off), g_bytes ? reinterpret_cast<uint32_t*>(d_gid) : nullptr,
+                    reinterpret_cast<float4*>(d_f), c->ncells, (uint32_t)n, c->stream);
+      if (!f32 && f_bytes) launch_decode(pool(c, c->fcur), reinterpret_cast<float*>(d_f), (uint32_t)n, c->stream);
+      HIPCHK(hipGetLastError());
+      HIPCHK(hipStreamSynchronize(c->stream));
+      c->stage_used = 0;
+      for (uint32_t i = 0; i <= c->ncells; ++i) offsets[i] = reinterpret_cast<const uint32_t*>(h_off)[i];
+      if (g_bytes) std::memcpy(gids, h_gid, g_bytes);
+      if (f_bytes) std::memcpy(f, h_f, f_bytes);
+      return 0;
+   }
    std::vector<uint32_t> off(c->ncells + 1);
    HIPCHK(hipMemcpyAsync(off.data(), c->off[c->lcur], (c->ncells + 1) * sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
    HIPCHK(hipStreamSynchronize(c->stream));
+   c->stage_used = 0;
    for (uint32_t i = 0; i <= c->ncells; ++i) offsets[i] = off[i];
-   const size_t n = off[c->ncells];
    if (n && gids) HIPCHK(hipMemcpy(gids, c->gid[c->lcur], n * sizeof(uint32_t), hipMemcpyDeviceToHost));
    if (n && f) {
       if (c->opt.storage == VACC_STORE_F32) {
@@ -1529,12 +1666,14 @@ static MomentArgs moment_args(const vacc_ctx* c) {
    return ma;
 }
 
-// Enqueue the moments of the current list unless they are resident.
-static void enqueue_moments(vacc_ctx* c) {
+// Enqueue the moments of the current list unless they are resident; host: also written there
+// (device address of pinned memory).
+static void enqueue_moments(vacc_ctx* c, double* host) {
    if (c->moments_valid) return;
    ProfScope ps(c, 3);
    MomentArgs ma = moment_args(c);
    ma.blk_stats = c->stats_valid ? c->blk_stats : nullptr;
+   ma.host = host;
    launch_moments(ma, c->stream);
    c->moments_valid = true;
 }
@@ -1550,11 +1689,18 @@ static void enqueue_transform(vacc_ctx* c, uint32_t map_order, int mode) {
                     c->opt.ohm_gradpe_term, (int)map_order, c->isect, c->ncells, c->stream);
 }
 
+// Copies the fields to the device; the caller waits for the stream before it returns.
 static int upload_fields(vacc_ctx* c, const vacc_cell_fields* fields) {
-   std::vector<TransformIn> tin(c->ncells);
-   for (uint32_t i = 0; i < c->ncells; ++i) to_tin(fields[i], tin[i]);
-   HIPCHK(hipMemcpyAsync(c->fields, tin.data(), tin.size() * sizeof(TransformIn), hipMemcpyHostToDevice, c->stream));
-   HIPCHK(hipStreamSynchronize(c->stream));   // tin is released on return
+   int rc = stage_begin(c);
+   if (rc) return rc;
+   const size_t bytes = c->ncells * sizeof(TransformIn);
+   uint8_t* dev = nullptr;
+   TransformIn* t = reinterpret_cast<TransformIn*>(stage_take(c, bytes, &dev));
+   std::vector<TransformIn> big(t ? 0 : c->ncells);
+   if (!t) t = big.data();
+   for (uint32_t i = 0; i < c->ncells; ++i) to_tin(fields[i], t[i]);
+   HIPCHK(hipMemcpyAsync(c->fields, t, bytes, hipMemcpyHostToDevice, c->stream));
+   if (!big.empty()) HIPCHK(hipStreamSynchronize(c->stream));   // big is released on return
    c->fields_valid = true;
    c->sub_valid = false;
    return 0;
@@ -1563,7 +1709,11 @@ static int upload_fields(vacc_ctx* c, const vacc_cell_fields* fields) {
 int vacc_set_fields(vacc_ctx* c, const vacc_cell_fields* fields) {
    if (!c || (!fields && c->ncells)) return set_err(VACC_E_ARG, "null argument");
    if (!c->ncells) return 0;
-   return upload_fields(c, fields);
+   const int rc = upload_fields(c, fields);
+   if (rc) return rc;
+   HIPCHK(hipStreamSynchronize(c->stream));
+   c->stage_used = 0;
+   return 0;
 }
 
 int vacc_compute_cell_intersections(vacc_ctx* c, const vacc_cell_fields* fields, uint32_t map_order, int32_t use_moments) {
@@ -1578,6 +1728,7 @@ int vacc_compute_cell_intersections(vacc_ctx* c, const vacc_cell_fields* fields,
    enqueue_transform(c, map_order, use_moments ? 1 : 0);
    HIPCHK(hipGetLastError());
    HIPCHK(hipStreamSynchronize(c->stream));
+   c->stage_used = 0;
    return 0;
 }
 
@@ -1632,10 +1783,7 @@ int vacc_adjust_blocks(vacc_ctx* c, double* rho_loss) {
    if (rc) return rc;
    rc = do_relist(c, c->sp.sparse_add_width_v, true);
    if (rc) return rc;
-   rc = finish(c);
-   if (rc < 0) return rc;
-   if (rho_loss) HIPCHK(hipMemcpy(rho_loss, c->rho_loss, c->ncells * sizeof(double), hipMemcpyDeviceToHost));
-   return rc;
+   return finish(c, rho_loss);
 }
 
 // grow a device buffer to hold n elements of size es
@@ -1688,10 +1836,7 @@ int vacc_adjust_blocks_spatial(vacc_ctx* c, const uint32_t* nbr_off, const uint3
    if (rc) return rc;
    rc = do_relist(c, c->sp.sparse_add_width_v, true, &sp);
    if (rc) return rc;
-   rc = finish(c);
-   if (rc < 0) return rc;
-   if (rho_loss) HIPCHK(hipMemcpy(rho_loss, c->rho_loss, c->ncells * sizeof(double), hipMemcpyDeviceToHost));
-   return rc;
+   return finish(c, rho_loss);
 }
 
 int vacc_autotune(vacc_ctx* c, uint32_t* mult_out) {
@@ -1846,10 +1991,7 @@ int vacc_step(vacc_ctx* c, uint32_t map_order, int32_t use_moments, int32_t adju
    rc = (c->opt.use_graph && !c->prof) ? graph_step(c, map_order, use_moments, adjust)
                                        : enqueue_step(c, map_order, use_moments, adjust);
    if (rc) return rc;
-   rc = finish(c);
-   if (rc < 0) return rc;
-   if (adjust && rho_loss) HIPCHK(hipMemcpy(rho_loss, c->rho_loss, c->ncells * sizeof(double), hipMemcpyDeviceToHost));
-   return rc;
+   return finish(c, adjust ? rho_loss : nullptr);
 }
 
 int vacc_subcycle_count(vacc_ctx* c, double dt, uint32_t* nmax) {
@@ -1885,10 +2027,7 @@ int vacc_subcycle_step(vacc_ctx* c, uint32_t step, uint32_t map_order, int32_t u
    rc = enqueue_step(c, map_order, use_moments, adjust);
    c->subcycling = false;
    if (rc) return rc;
-   rc = finish(c);
-   if (rc < 0) return rc;
-   if (adjust && rho_loss) HIPCHK(hipMemcpy(rho_loss, c->rho_loss, c->ncells * sizeof(double), hipMemcpyDeviceToHost));
-   return rc;
+   return finish(c, adjust ? rho_loss : nullptr);
 }
 
 int vacc_accelerate_subcycled(vacc_ctx* c, double dt, uint32_t map_order, int32_t use_moments, uint32_t* nsub,
@@ -1964,16 +2103,17 @@ int vacc_accelerate_populations(vacc_ctx* const* ctxs, uint32_t npop, uint32_t m
       }
       HIPCHK(hipGetLastError());
    }
+   const bool loss = adjust && rho_loss;
+   for (uint32_t p = 0; p < npop; ++p) {
+      const int rc = finish_enqueue(ctxs[p], loss && rho_loss[p]);
+      if (rc) return rc;
+   }
    int st = 0;
    for (uint32_t p = 0; p < npop; ++p) {
-      const int rc = finish(ctxs[p]);
+      const int rc = finish_wait(ctxs[p], loss ? rho_loss[p] : nullptr);
       if (rc < 0) return rc;
       st |= rc;
    }
-   if (adjust && rho_loss)
-      for (uint32_t p = 0; p < npop; ++p)
-         if (rho_loss[p])
-            HIPCHK(hipMemcpy(rho_loss[p], ctxs[p]->rho_loss, ctxs[p]->ncells * sizeof(double), hipMemcpyDeviceToHost));
    return st;
 }
 
@@ -2034,10 +2174,11 @@ int vacc_find_blocks_noalloc(vacc_ctx* c, uint64_t nq, const uint32_t* cells, co
 int vacc_moments(vacc_ctx* c, double* out) {
    if (!c || (!out && c->ncells)) return set_err(VACC_E_ARG, "null argument");
    if (!c->ncells) return 0;
-   enqueue_moments(c);
+   if (c->moments_valid) launch_copy_f64(c->d_res, c->moments, 4 * c->ncells, c->stream);
+   else enqueue_moments(c, c->d_res);
    HIPCHK(hipGetLastError());
-   HIPCHK(hipMemcpyAsync(out, c->moments, (size_t)c->ncells * 4 * sizeof(double), hipMemcpyDeviceToHost, c->stream));
    HIPCHK(hipStreamSynchronize(c->stream));
+   std::memcpy(out, c->h_res, (size_t)c->ncells * 4 * sizeof(double));
    return 0;
 }
 
@@ -2046,14 +2187,12 @@ int vacc_pressure(vacc_ctx* c, const double* pivot, double* out) {
    if (!c->ncells) return 0;
    const size_t n = c->ncells;
    // without a pivot the kernel takes the population's own bulk velocity from its first moments
-   double *d_out = c->press, *d_piv = c->press + 6 * n;
-   if (pivot) HIPCHK(hipMemcpyAsync(d_piv, pivot, 3 * n * sizeof(double), hipMemcpyHostToDevice, c->stream));
+   if (pivot) HIPCHK(hipMemcpyAsync(c->press, pivot, 3 * n * sizeof(double), hipMemcpyHostToDevice, c->stream));
    else enqueue_moments(c);
-   MomentArgs ma = moment_args(c);
-   launch_pressure(ma, pivot ? d_piv : nullptr, c->sp.mass, d_out, c->stream);
+   launch_pressure(moment_args(c), pivot ? c->press : nullptr, c->sp.mass, c->d_res, c->stream);
    HIPCHK(hipGetLastError());
-   HIPCHK(hipMemcpyAsync(out, d_out, 6 * n * sizeof(double), hipMemcpyDeviceToHost, c->stream));
    HIPCHK(hipStreamSynchronize(c->stream));
+   std::memcpy(out, c->h_res, 6 * n * sizeof(double));
    return 0;
 }
 
@@ -2212,7 +2351,6 @@ int vacc_trans_map_1d(vacc_ctx* c, uint32_t dim, double dt) {
    // that select a captured variant are updated below
    int rc = 0;
    if (!c->sorted && (rc = do_relist(c, -1, false))) return rc;   // ascending GIDs, same blocks
-   if ((rc = refresh_count(c))) return rc;
    TransArgs ta{};
    ta.off = c->off[c->lcur];
    ta.gid = c->gid[c->lcur];

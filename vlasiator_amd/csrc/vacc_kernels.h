@@ -178,6 +178,7 @@ struct MomentArgs {
    double* out;                // [ncells*4]
    double* part;               // partial sums: 4 (moments) or 6 (pressure) doubles per workgroup,
                                // ncells * cell_split(ncells) workgroups
+   double* host;               // null, or where the moments also go (device address of pinned memory)
    uint32_t ncells;
    uint32_t len[3];
    GidSplit gs;                // block coordinates of a GID (from len)
@@ -275,7 +276,30 @@ void launch_pressure(const MomentArgs& a, const double* pivot, double mass, doub
 void launch_transform(const MeshInfo& m, const TransformIn* fields, const double* dt_override, const double* moments, int use_moments,
                       double mass, double charge, double hall_min_rhoq, int ohm_gradpe, int map_order,
                       double* isect_out, uint32_t ncells, hipStream_t s);
-void launch_gather(const uint32_t* src, const Pool& in, const Pool& out, uint32_t n, hipStream_t s);
+// out block i = in block src[i] (zero for INVALID); then src[i] = i
+void launch_gather(uint32_t* src, const Pool& in, const Pool& out, uint32_t n, hipStream_t s);
+// The end of a work call: sum[0..2] = capacity flag, block total, status OR, and the removed mass
+// of n cells (loss null: none), into pinned memory
+void launch_finish(const uint32_t* flags, const uint32_t* total, const uint32_t* status, uint32_t* sum, const double* loss,
+                   double* loss_out, uint32_t n, hipStream_t s);
+void launch_copy_f64(double* dst, const double* src, uint32_t n, hipStream_t s);
+// A load from staged lists and FP32 blocks (pinned memory): lists, identity src, pool, thresholds,
+// cleared status words and flags
+struct LoadArgs {
+   const uint32_t *off_in, *gid_in;
+   const float4* f_in;
+   uint32_t *off, *gid, *src;
+   float4* f;
+   double* minval;
+   double min_value;
+   uint32_t *status, *flags;   // [ncells + 1], one word
+   uint32_t n, ncells;         // blocks, cells
+};
+void launch_load(const LoadArgs& a, hipStream_t s);
+// Offsets, GIDs (null: not wanted) and FP32 blocks (f null: not wanted) of a compact list into
+// staged memory
+void launch_unload(const uint32_t* off, const uint32_t* gid, const float4* f, uint32_t* off_out, uint32_t* gid_out,
+                   float4* f_out, uint32_t ncells, uint32_t n, hipStream_t s);
 // FP32 blocks <-> 16-bit pool (one wave per block)
 void launch_encode(const float* f, const Pool& out, uint32_t n, hipStream_t s);
 void launch_decode(const Pool& in, float* f, uint32_t n, hipStream_t s);

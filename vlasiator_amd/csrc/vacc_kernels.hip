@@ -1511,7 +1511,7 @@ __global__ __launch_bounds__(AWG) void k_adjust(AdjustArgs a) {
 // each adding every 16th part, then a fixed tree (one lane per sum waited 10 us for 64 dependent
 // loads, 16 lanes take 4)
 __global__ __launch_bounds__(WG) void k_cell_parts(const double* part, uint32_t split, uint32_t nv, uint32_t n,
-                                                   double scale, double* out) {
+                                                   double scale, double* out, double* host) {
    const uint32_t i = blockIdx.x * (WG / 16) + (threadIdx.x >> 4), l = threadIdx.x & 15;
    double sum = 0.0;
    if (i < n) {
@@ -1524,19 +1524,28 @@ __global__ __launch_bounds__(WG) void k_cell_parts(const double* part, uint32_t 
       }
    }
    for (int o = 8; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 16);
-   if (l == 0 && i < n) out[i] = sum * scale;
+   if (l == 0 && i < n) {
+      out[i] = sum * scale;
+      if (host) host[i] = sum * scale;
+   }
 }
 
 // One workgroup's NV sums (red[e][wave]): the cell's result times scale when the cell has one
 // workgroup, otherwise its part for k_cell_parts.
 template <int NV>
-__device__ inline void put_cell_sums(const double (*red)[WG / 64], double* part, double* out, uint32_t split, double scale) {
+__device__ inline void put_cell_sums(const double (*red)[WG / 64], double* part, double* out, double* host, uint32_t split,
+                                     double scale) {
    const int t = threadIdx.x;
    if (t < NV) {
       double sum = 0.0;
       for (int w = 0; w < WG / 64; ++w) sum += red[t][w];
-      if (split == 1) out[(size_t)NV * blockIdx.x + t] = sum * scale;
-      else part[(size_t)NV * blockIdx.x + t] = sum;
+      const size_t i = (size_t)NV * blockIdx.x + t;
+      if (split > 1) {
+         part[i] = sum;
+      } else {
+         out[i] = sum * scale;
+         if (host) host[i] = sum * scale;
+      }
    }
 }
 
@@ -1611,7 +1620,7 @@ __global__ __launch_bounds__(WG) void k_pressure(MomentArgs a, const double* piv
       if ((t & 63) == 0) red[e][t >> 6] = s[e];
    }
    __syncthreads();
-   put_cell_sums<6>(red, a.part, out, split, mass * (a.cell[0] * a.cell[1] * a.cell[2]));
+   put_cell_sums<6>(red, a.part, out, nullptr, split, mass * (a.cell[0] * a.cell[1] * a.cell[2]));
 }
 
 // spatial_cell_cpu.cpp:699-727
@@ -1768,7 +1777,7 @@ __global__ __launch_bounds__(WG) void k_moments(MomentArgs a, uint32_t split) {
       red[3][t >> 6] = s3;
    }
    __syncthreads();
-   put_cell_sums<4>(red, a.part, a.out, split, a.cell[0] * a.cell[1] * a.cell[2]);
+   put_cell_sums<4>(red, a.part, a.out, a.host, split, a.cell[0] * a.cell[1] * a.cell[2]);
 }
 
 // The same moments from the block sums of the last remap pass (MomentArgs::blk_stats): split
@@ -1825,7 +1834,7 @@ __global__ __launch_bounds__(WG) void k_moments_sums(MomentArgs a, uint32_t spli
       red[3][t >> 6] = s3;
    }
    __syncthreads();
-   put_cell_sums<4>(red, a.part, a.out, split, a.cell[0] * a.cell[1] * a.cell[2]);
+   put_cell_sums<4>(red, a.part, a.out, a.host, split, a.cell[0] * a.cell[1] * a.cell[2]);
 }
 
 __global__ void k_transform(MeshInfo m, const TransformIn* fields, const double* dt_override, const double* moments,
@@ -1883,26 +1892,91 @@ void launch_plasma(const PlasmaArgs& a, hipStream_t s) {
    hipLaunchKernelGGL(k_plasma, dim3((a.ncells + 255) / 256), dim3(256), 0, s, a);
 }
 
-// 16 lanes per block, grid-stride (capped grid, see launch_gather)
-__global__ void k_gather(const uint32_t* src, const float4* f_in, float4* f_out, uint32_t n) {
+// 16 lanes per block, grid-stride (capped grid, see launch_gather).  The lanes of a block are in
+// one wave and read its index together before lane 0 replaces it by the identity.
+__global__ void k_gather(uint32_t* src, const float4* f_in, float4* f_out, uint32_t n) {
    const size_t stride = (size_t)gridDim.x * blockDim.x;
    for (size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x; q < (size_t)n * 16; q += stride) {
       const uint32_t b = (uint32_t)(q >> 4);
       const uint32_t s = src[b];
       f_out[q] = (s == INVALID) ? make_float4(0.f, 0.f, 0.f, 0.f) : f_in[(size_t)s * 16 + (q & 15)];
+      if ((q & 15) == 0) src[b] = b;
    }
 }
 
 // 16-bit pools: 16 lanes per block, 8 bytes of codes each, lane 0 the scale.
-__global__ void k_gather16(const uint32_t* src, const uint2* q_in, const float* s_in, uint2* q_out, float* s_out,
-                           uint32_t n) {
+__global__ void k_gather16(uint32_t* src, const uint2* q_in, const float* s_in, uint2* q_out, float* s_out, uint32_t n) {
    const size_t stride = (size_t)gridDim.x * blockDim.x;
    for (size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x; q < (size_t)n * 16; q += stride) {
       const uint32_t b = (uint32_t)(q >> 4);
       const uint32_t s = src[b];
       q_out[q] = (s == INVALID) ? make_uint2(0u, 0u) : q_in[(size_t)s * 16 + (q & 15)];
-      if ((q & 15) == 0) s_out[b] = (s == INVALID) ? 0.0f : s_in[s];
+      if ((q & 15) == 0) {
+         s_out[b] = (s == INVALID) ? 0.0f : s_in[s];
+         src[b] = b;
+      }
    }
+}
+
+__global__ void k_finish(const uint32_t* flags, const uint32_t* total, const uint32_t* status, uint32_t* sum,
+                         const double* loss, double* loss_out, uint32_t n) {
+   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+   if (i == 0) {
+      sum[0] = *flags;
+      sum[1] = *total;
+      sum[2] = *status;
+   }
+   if (loss && i < n) loss_out[i] = loss[i];
+}
+
+void launch_finish(const uint32_t* flags, const uint32_t* total, const uint32_t* status, uint32_t* sum, const double* loss,
+                   double* loss_out, uint32_t n, hipStream_t s) {
+   const uint32_t grid = loss ? (n + 255) / 256 : 1;
+   hipLaunchKernelGGL(k_finish, dim3(std::max(grid, 1u)), dim3(256), 0, s, flags, total, status, sum, loss, loss_out, n);
+}
+
+__global__ void k_copy_f64(double* dst, const double* src, uint32_t n) {
+   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+   if (i < n) dst[i] = src[i];
+}
+
+void launch_copy_f64(double* dst, const double* src, uint32_t n, hipStream_t s) {
+   if (n) hipLaunchKernelGGL(k_copy_f64, dim3((n + 255) / 256), dim3(256), 0, s, dst, src, n);
+}
+
+// One thread per float4 of f (at least one per cell word); bound by the bus.
+__global__ void k_load(LoadArgs a) {
+   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+   if (i < 16 * a.n) a.f[i] = a.f_in[i];
+   if (i < a.n) {
+      a.gid[i] = a.gid_in[i];
+      a.src[i] = i;
+   }
+   if (i <= a.ncells) {
+      a.off[i] = a.off_in[i];
+      a.status[i] = 0u;
+   }
+   if (i < a.ncells) a.minval[i] = a.min_value;
+   if (i == 0) *a.flags = 0u;
+}
+
+void launch_load(const LoadArgs& a, hipStream_t s) {
+   const uint32_t n = std::max(16 * a.n, a.ncells + 1);   // a staged load holds less than 2^20 bytes
+   hipLaunchKernelGGL(k_load, dim3((n + 255) / 256), dim3(256), 0, s, a);
+}
+
+__global__ void k_unload(const uint32_t* off, const uint32_t* gid, const float4* f, uint32_t* off_out, uint32_t* gid_out,
+                         float4* f_out, uint32_t ncells, uint32_t n) {
+   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+   if (f && i < 16 * n) f_out[i] = f[i];
+   if (gid_out && i < n) gid_out[i] = gid[i];
+   if (i <= ncells) off_out[i] = off[i];
+}
+
+void launch_unload(const uint32_t* off, const uint32_t* gid, const float4* f, uint32_t* off_out, uint32_t* gid_out,
+                   float4* f_out, uint32_t ncells, uint32_t n, hipStream_t s) {
+   const uint32_t m = std::max(f ? 16 * n : n, ncells + 1);
+   hipLaunchKernelGGL(k_unload, dim3((m + 255) / 256), dim3(256), 0, s, off, gid, f, off_out, gid_out, f_out, ncells, n);
 }
 
 // FP32 blocks -> 16-bit pool, one wave per block.
@@ -2056,10 +2130,11 @@ uint32_t cell_split(uint32_t ncells) {
 }
 
 static void launch_parts(const double* part, uint32_t split, uint32_t nv, uint32_t ncells, double scale, double* out,
-                         hipStream_t s) {
+                         double* host, hipStream_t s) {
    const uint32_t n = nv * ncells;
    if (split > 1)
-      hipLaunchKernelGGL(k_cell_parts, dim3((n + WG / 16 - 1) / (WG / 16)), dim3(WG), 0, s, part, split, nv, n, scale, out);
+      hipLaunchKernelGGL(k_cell_parts, dim3((n + WG / 16 - 1) / (WG / 16)), dim3(WG), 0, s, part, split, nv, n, scale, out,
+                         host);
 }
 
 void launch_moments(const MomentArgs& a, hipStream_t s) {
@@ -2072,7 +2147,7 @@ void launch_moments(const MomentArgs& a, hipStream_t s) {
    else if (a.pool.storage == ST_F32) hipLaunchKernelGGL(k_moments<ST_F32>, grid, dim3(WG), 0, s, a, split);
    else if (a.pool.storage == ST_BF16) hipLaunchKernelGGL(k_moments<ST_BF16>, grid, dim3(WG), 0, s, a, split);
    else hipLaunchKernelGGL(k_moments<ST_F16>, grid, dim3(WG), 0, s, a, split);
-   launch_parts(a.part, split, 4, a.ncells, a.cell[0] * a.cell[1] * a.cell[2], a.out, s);
+   launch_parts(a.part, split, 4, a.ncells, a.cell[0] * a.cell[1] * a.cell[2], a.out, a.host, s);
 }
 
 void launch_transform(const MeshInfo& m, const TransformIn* fields, const double* dt_override, const double* moments,
@@ -2127,7 +2202,7 @@ void launch_subcycle_step(const double* maxdt, const uint32_t* nsub, uint32_t nc
                       subdt, active);
 }
 
-void launch_gather(const uint32_t* src, const Pool& in, const Pool& out, uint32_t n, hipStream_t s) {
+void launch_gather(uint32_t* src, const Pool& in, const Pool& out, uint32_t n, hipStream_t s) {
    if (n == 0) return;
    const uint32_t grid = (uint32_t)std::min<uint64_t>(((uint64_t)n * 16 + 255) / 256, 1u << 20);
    if (in.storage == ST_F32)
@@ -2178,7 +2253,7 @@ void launch_pressure(const MomentArgs& a, const double* pivot, double mass, doub
       hipLaunchKernelGGL(k_pressure<ST_BF16>, grid, dim3(WG), 0, s, a, pivot, split, mass, out);
    else
       hipLaunchKernelGGL(k_pressure<ST_F16>, grid, dim3(WG), 0, s, a, pivot, split, mass, out);
-   launch_parts(a.part, split, 6, a.ncells, mass * (a.cell[0] * a.cell[1] * a.cell[2]), out, s);
+   launch_parts(a.part, split, 6, a.ncells, mass * (a.cell[0] * a.cell[1] * a.cell[2]), out, nullptr, s);
 }
 
 void launch_sparse_min(const SparseArgs& p, const double* moments, const uint32_t* off, double* minval,
