@@ -1029,18 +1029,19 @@ __device__ inline int row_min16(int x) {
 }
 
 // At least five waves per SIMD (at most 96 VGPRs).  The values that no longer fit are kept in
-// scratch across the per-unit setup and the column ends, not in the block loop: 12 to 20
-// bytes per lane for FP32 storage (36 to 44 with block sums), 44 to 64 for the 16-bit forms
+// scratch across the per-unit setup and the column ends, not in the block loop: none to 8
+// bytes per lane for FP32 storage (PQM; up to 16 with block sums), 32 to 84 for the 16-bit forms
 // (their codec alone would need 111 to 116 VGPRs).  Five waves issue about 7 % more per pass
-// than four on the PQM workloads for FP32 and make the 16-bit forms' step 3 % faster; six and
-// eight are slower.
+// than four on the PQM workloads for FP32 and make the 16-bit forms' step 3 % faster.
+// Bound by VALU issue and latency: with limiters and face tests as medians of three, halved
+// derivatives and the short quartic (vacc_lean.h), and targets placed by a minimum in place of
+// a range test, a PQM cell without a second boundary takes 65 VALU instructions instead of 87;
+// x, y, z passes over 26 million blocks 4.88, 5.31, 5.05 -> 4.32, 5.09, 4.60 ms (PQM, FP32).
 template <int DIM, int METHOD, int ST, int WGS, bool STATS>
 __global__ __launch_bounds__(WGS, 5) void k_remap_lean(RemapArgs a) {
    using R = ReconLean<METHOD>;
    constexpr int NC = R::NC;
-   // rows 0 .. LEAN_RING - 1: the target ring; row LEAN_RING: sink of deposits outside the
-   // column's target range
-   __shared__ float ring[LEAN_RING + 1][WGS];
+   __shared__ float ring[LEAN_RING][WGS];
    if (*a.flags & VACC_STATUS_CAPACITY) return;
    const int tid = threadIdx.x;
    const int l16 = tid & 15;
@@ -1084,17 +1085,21 @@ __global__ __launch_bounds__(WGS, 5) void k_remap_lean(RemapArgs a) {
             prev_end = max(prev_end, lk);
             continue;
          }
-         const int lo = WID * fk, hi = WID * lk + WID - 1;
+         const int hi = WID * lk + WID - 1;
          // Each target cell ends with its whole mass in one store: the deposit closes a target
          // once (the shares of earlier source cells ride in the running sum), the partial sum a
          // cell without a boundary stores into the open target is overwritten when it closes,
          // and the columns of a unit reach distinct target cells (dk <= 3 dv, checked in the
-         // column build).  Ring cells that no deposit reaches keep the zero of their opening.  A target
-         // outside the column's range goes to the sink row (no branch).
-         auto emit = [&](int gt, float m) {
-            const bool in = (uint32_t)(gt - lo) <= (uint32_t)(hi - lo);
-            ring[in ? (gt & (LEAN_RING - 1)) : LEAN_RING][tid] = m;
-         };
+         // column build).  Ring cells that no deposit reaches keep the zero of their opening.
+         // Targets outside [WID fk, hi] (mesh walls, rounding at the ends) need no test.  Every
+         // target that a source block's cells reach lies within spread + 4 dv/dk + 3 <= 10 cells of
+         // the lowest target any lane had open at the previous block (spread <= 3 (|di| + |dj|)/dk
+         // + 1, and LEAN_SPAN bounds the sum): no block that is still to be stored, and none opened
+         // ahead, is 13 or more cells away, so the rows of targets below the range alias none of
+         // theirs.  Above the range (up to a whole mesh of them at a wall, while the last block
+         // stays open for the next column) they are moved to hi + 1, the row of a block three
+         // below the last one.
+         auto emit = [&](int gt, float m) { ring[min(gt, hi + 1) & (LEAN_RING - 1)][tid] = m; };
          Flux<NC> fx;
          fx.begin((a.vmin_d + (double)(WID * ks) * a.dv_d - imin) * rdk, r);
          float w0[4] = {0.0f, 0.0f, 0.0f, 0.0f}, w1[4], w2[4];
