@@ -129,11 +129,13 @@ struct vacc_ctx {
    int remap_wgs_s[3] = {256, 256, 256};  // kernel instance, with more registers in scratch)
    // Pinned host memory that kernels write results to (the d_ pointers are its device addresses):
    // h_sum: capacity flag, block total, status OR, subcycle count; h_res: [6*ncells] per-cell
-   // results of a call; stage: small transfers in either direction, allocated on first use
+   // results of a call, in the same page for a few cells; stage: small transfers in either
+   // direction, allocated for a context's second one
    uint32_t *h_sum = nullptr, *d_sum = nullptr;
    double *h_res = nullptr, *d_res = nullptr;
    uint8_t *stage = nullptr, *d_stage = nullptr;
    size_t stage_used = 0;            // bytes handed out since the stream was last waited for
+   bool stage_wanted = false;        // a small transfer came before
    // streamed block transfer (vacc_blocks_io.h): two pinned chunks, their copy events and,
    // for the 16-bit forms, a device FP32 stage of two chunks; allocated on first use
    float* io_pin[2] = {nullptr, nullptr};
@@ -239,6 +241,13 @@ static void free_blocks(vacc_ctx* c) {
    c->cap = 0;
 }
 
+// The pinned page of h_sum: the words, and from RES_OFFSET on the results of up to 84 cells (a
+// pinned allocation takes about 0.1 ms, more than the call of a small context).
+constexpr size_t SUM_PAGE = 4096, RES_OFFSET = 16;
+static bool results_in_page(const vacc_ctx* c) {
+   return reinterpret_cast<const uint8_t*>(c->h_res) == reinterpret_cast<const uint8_t*>(c->h_sum) + RES_OFFSET;
+}
+
 static void free_cells(vacc_ctx* c) {
    for (int i = 0; i < 2; ++i) {
       if (c->off[i]) (void)hipFree(c->off[i]);
@@ -262,7 +271,7 @@ static void free_cells(vacc_ctx* c) {
    c->keep_box = nullptr;
    c->cell_hist = nullptr;
    c->parts = c->press = nullptr;
-   if (c->h_res) (void)hipHostFree(c->h_res);
+   if (c->h_res && !results_in_page(c)) (void)hipHostFree(c->h_res);
    c->h_res = c->d_res = nullptr;
    c->sub_maxdt = c->sub_dt = nullptr;
    c->sub_n = c->sub_nmax = nullptr;
@@ -302,8 +311,13 @@ static int alloc_cells(vacc_ctx* c, uint32_t n) {
    HIPCHK(hipMalloc(&c->rho_loss, m * sizeof(double)));
    HIPCHK(hipMalloc(&c->parts, 6 * parts_max(n) * sizeof(double)));
    HIPCHK(hipMalloc(&c->press, 3 * m * sizeof(double)));
-   HIPCHK(hipHostMalloc(&c->h_res, 6 * m * sizeof(double), hipHostMallocDefault));
-   HIPCHK(hipHostGetDevicePointer((void**)&c->d_res, c->h_res, 0));
+   if (6 * m * sizeof(double) <= SUM_PAGE - RES_OFFSET) {
+      c->h_res = reinterpret_cast<double*>(reinterpret_cast<uint8_t*>(c->h_sum) + RES_OFFSET);
+      c->d_res = reinterpret_cast<double*>(reinterpret_cast<uint8_t*>(c->d_sum) + RES_OFFSET);
+   } else {
+      HIPCHK(hipHostMalloc(&c->h_res, 6 * m * sizeof(double), hipHostMallocDefault));
+      HIPCHK(hipHostGetDevicePointer((void**)&c->d_res, c->h_res, 0));
+   }
    HIPCHK(hipMalloc(&c->sub_maxdt, m * sizeof(double)));
    HIPCHK(hipMalloc(&c->sub_dt, m * sizeof(double)));
    HIPCHK(hipMalloc(&c->sub_n, m * sizeof(uint32_t)));
@@ -668,13 +682,18 @@ static int finish(vacc_ctx* c, double* rho_loss = nullptr) {
 }
 
 // Staging of small transfers: `bytes` of pinned memory (host address; *dev the device address),
-// or null when they don't fit.  What was handed out stays in use until the stream has been waited
+// or null when they don't fit or the context has made no small transfer before (its allocation
+// would cost a context used once more than it saves).  What was handed out stays in use until the stream has been waited
 // for (stage_used = 0 after a wait); a call that failed in between is waited for here.
 constexpr size_t STAGE_BYTES = 1u << 20;
 static uint8_t* stage_take(vacc_ctx* c, size_t bytes, uint8_t** dev) {
    const size_t want = (bytes + 255) & ~(size_t)255;
    if (want > STAGE_BYTES) return nullptr;
    if (!c->stage) {
+      if (!c->stage_wanted) {
+         c->stage_wanted = true;
+         return nullptr;
+      }
       if (hipHostMalloc(&c->stage, STAGE_BYTES, hipHostMallocDefault) != hipSuccess ||
           hipHostGetDevicePointer((void**)&c->d_stage, c->stage, 0) != hipSuccess) {
          (void)hipGetLastError();
@@ -844,9 +863,9 @@ static int load_staged(vacc_ctx* c, uint32_t ncells, const uint64_t* offsets, co
    if (rc) return rc;
    uint8_t *d_off = nullptr, *d_gid = nullptr, *d_f = nullptr;
    uint32_t* h_off = reinterpret_cast<uint32_t*>(stage_take(c, (ncells + 1) * sizeof(uint32_t), &d_off));
-   uint8_t* h_gid = stage_take(c, total * sizeof(uint32_t), &d_gid);
-   uint8_t* h_f = stage_take(c, total * WID3 * sizeof(float), &d_f);
-   if (!h_off || !h_gid || !h_f) {
+   uint8_t* h_gid = h_off ? stage_take(c, total * sizeof(uint32_t), &d_gid) : nullptr;
+   uint8_t* h_f = h_gid ? stage_take(c, total * WID3 * sizeof(float), &d_f) : nullptr;
+   if (!h_f) {
       c->stage_used = 0;   // nothing was enqueued
       return 1;
    }
@@ -1465,7 +1484,7 @@ int vacc_create(const vacc_mesh* mesh, const vacc_species* species, const vacc_o
    }
    if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess ||
        hipMalloc(&c->flags, sizeof(uint32_t)) != hipSuccess || hipMemset(c->flags, 0, sizeof(uint32_t)) != hipSuccess ||
-       hipHostMalloc(&c->h_sum, 4 * sizeof(uint32_t), hipHostMallocDefault) != hipSuccess ||
+       hipHostMalloc(&c->h_sum, SUM_PAGE, hipHostMallocDefault) != hipSuccess ||
        hipHostGetDevicePointer((void**)&c->d_sum, c->h_sum, 0) != hipSuccess ||
        hipEventCreateWithFlags(&c->mom_ev, hipEventDisableTiming) != hipSuccess) {
       delete c;
