@@ -69,8 +69,8 @@ struct vacc_ctx {
    uint32_t* sorted_src = nullptr;
    uint4* unit_rec = nullptr;
    uint4* col_rec = nullptr;
-   uint32_t* perm = nullptr;
-   uint32_t* perm_cell = nullptr;
+   uint4* units = nullptr;           // remap work list, two words of 16 bytes per unit
+   PassCell* pass_cell = nullptr;    // [ncells]
    uint32_t* n_units = nullptr;
    uint32_t* n_tgt = nullptr;
    uint32_t* unit_base = nullptr;
@@ -231,13 +231,11 @@ static void free_blocks(vacc_ctx* c) {
    if (c->sorted_src) (void)hipFree(c->sorted_src);
    if (c->unit_rec) (void)hipFree(c->unit_rec);
    if (c->col_rec) (void)hipFree(c->col_rec);
-   if (c->perm) (void)hipFree(c->perm);
-   if (c->perm_cell) (void)hipFree(c->perm_cell);
-   c->perm_cell = nullptr;
+   if (c->units) (void)hipFree(c->units);
    c->content = nullptr;
    c->sorted_src = nullptr;
    c->unit_rec = c->col_rec = nullptr;
-   c->perm = nullptr;
+   c->units = nullptr;
    c->cap = 0;
 }
 
@@ -264,13 +262,14 @@ static void free_cells(vacc_ctx* c) {
    if (c->pivot) (void)hipFree(c->pivot);
    if (c->rho_loss) (void)hipFree(c->rho_loss);
    void* subs[] = {c->sub_maxdt, c->sub_dt, c->sub_n, c->active, c->sub_nmax, c->minval, c->csum_pre, c->csum_post,
-                   c->keep_bm, c->keep_box, c->cell_hist, c->parts, c->press};
+                   c->keep_bm, c->keep_box, c->cell_hist, c->parts, c->press, c->pass_cell};
    for (void* p : subs)
       if (p) (void)hipFree(p);
    c->keep_bm = nullptr;
    c->keep_box = nullptr;
    c->cell_hist = nullptr;
    c->parts = c->press = nullptr;
+   c->pass_cell = nullptr;
    if (c->h_res && !results_in_page(c)) (void)hipHostFree(c->h_res);
    c->h_res = c->d_res = nullptr;
    c->sub_maxdt = c->sub_dt = nullptr;
@@ -328,6 +327,7 @@ static int alloc_cells(vacc_ctx* c, uint32_t n) {
    HIPCHK(hipMalloc(&c->csum_post, m * sizeof(double)));
    HIPCHK(hipMalloc(&c->keep_bm, (size_t)n * ADJ_BM_WORDS * sizeof(uint32_t)));
    HIPCHK(hipMalloc(&c->keep_box, m * 8 * sizeof(int)));
+   HIPCHK(hipMalloc(&c->pass_cell, m * sizeof(PassCell)));
    HIPCHK(hipMalloc(&c->cell_hist, (size_t)LEN_BINS * n * sizeof(uint32_t)));
    c->cell_cap = n;
    return 0;
@@ -350,11 +350,11 @@ static int ensure_blocks(vacc_ctx* c, size_t want) {
    void* f[2] = {nullptr, nullptr};
    float* sc[2] = {nullptr, nullptr};
    uint8_t* ct = nullptr;
-   uint32_t *ss = nullptr, *pm = nullptr, *pc = nullptr;
-   uint4 *sr = nullptr, *cr = nullptr;
+   uint32_t* ss = nullptr;
+   uint4 *sr = nullptr, *cr = nullptr, *un = nullptr;
    float4* bs = nullptr;
    auto release = [&]() {
-      void* all[] = {g[0], g[1], s[0], s[1], f[0], f[1], sc[0], sc[1], ct, ss, pm, pc, sr, cr, bs};
+      void* all[] = {g[0], g[1], s[0], s[1], f[0], f[1], sc[0], sc[1], ct, ss, un, sr, cr, bs};
       for (void* p : all)
          if (p) (void)hipFree(p);
    };
@@ -369,8 +369,7 @@ static int ensure_blocks(vacc_ctx* c, size_t want) {
    if (e == hipSuccess) e = hipMalloc(&ss, ncap * sizeof(uint32_t));
    if (e == hipSuccess) e = hipMalloc(&sr, ncap * sizeof(uint4));
    if (e == hipSuccess) e = hipMalloc(&cr, ncap * sizeof(uint4));
-   if (e == hipSuccess) e = hipMalloc(&pm, ncap * sizeof(uint32_t));
-   if (e == hipSuccess) e = hipMalloc(&pc, ncap * sizeof(uint32_t));
+   if (e == hipSuccess) e = hipMalloc(&un, 2 * ncap * sizeof(uint4));
    if (e == hipSuccess && use_block_sums(c)) e = hipMalloc(&bs, ncap * sizeof(float4));
    if (e == hipSuccess && c->cap && c->nblocks) {
       // carry the current state: list entries and the whole current pool extent
@@ -406,8 +405,7 @@ static int ensure_blocks(vacc_ctx* c, size_t want) {
    c->sorted_src = ss;
    c->unit_rec = sr;
    c->col_rec = cr;
-   c->perm = pm;
-   c->perm_cell = pc;
+   c->units = un;
    c->blk_stats = bs;
    c->stats_valid = keep_stats;   // carried with the pool
    c->cap = ncap;
@@ -479,25 +477,27 @@ static int enqueue_pass(vacc_ctx* c, int dim, int grid_mult, int wgs = 0, bool s
       OrderArgs oa{};
       oa.cell_off = c->off[li];
       oa.unit_base = c->unit_base;
+      oa.out_off = c->off[lo];
       oa.unit_rec = c->unit_rec;
+      oa.col_rec = c->col_rec;
+      oa.isect = c->isect;
+      oa.minval = c->minval;
+      oa.dv_d = c->mi.cell[dim];
       oa.len_hist = c->len_hist;
       oa.cell_hist = c->cell_hist;
-      oa.perm = c->perm;
-      oa.perm_cell = c->perm_cell;
+      oa.units = c->units;
+      oa.pass_cell = c->pass_cell;
       oa.flags = c->flags;
       oa.ncells = c->ncells;
-      launch_order(oa, c->stream);
+      launch_order(dim, oa, c->stream);
    }
    RemapArgs ra{};
-   ra.cell_off = c->off[li];
    ra.unit_base = c->unit_base;
    ra.out_off = c->off[lo];
-   ra.perm = c->perm;
-   ra.perm_cell = c->perm_cell;
-   ra.unit_rec = c->unit_rec;
+   ra.units = c->units;
+   ra.pass_cell = c->pass_cell;
    ra.col_rec = c->col_rec;
    ra.sorted_src = c->sorted_src;
-   ra.isect = c->isect;
    ra.in = pool(c, fi);
    ra.out = pool(c, fo);
    ra.gid_out = c->gid[lo];
@@ -509,9 +509,6 @@ static int enqueue_pass(vacc_ctx* c, int dim, int grid_mult, int wgs = 0, bool s
    for (int d = 0; d < 3; ++d) ra.len[d] = c->mi.len[d];
    ra.dv = ca.dv;
    ra.vmin = ca.vmin;
-   ra.threshold = (float)c->sp.sparse_min_value;   // Realf threshold argument of compute_*_coeff
-   ra.min_value = c->sp.sparse_min_value;
-   ra.minval = c->minval;
    ra.len_hist = c->len_hist;
    ra.nblocks = c->nblocks;
    ra.dv_d = c->mi.cell[dim];

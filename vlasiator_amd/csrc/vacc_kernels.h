@@ -87,28 +87,44 @@ struct BuildScanArgs {
    uint32_t* len_hist;     // [LEN_BINS] total of each bin (written)
 };
 
+// What every unit of a cell needs of it in one pass: the intersections in the pass frame (FP64 for
+// the tolerance form, FP32 for the exact one) and the values derived from them and from the
+// sparsity threshold, computed once per cell instead of once per unit.
+struct PassCell {
+   double I, di, dj, rdk;        // rdk = 1 / dk
+   float r, inv_r;               // dk / dv, dv / dk
+   float thc;                    // content threshold (smallest float not below the FP64 one)
+   float thr, scale;             // reconstruction threshold and (float)(1 / thr)
+   float fI, fdi, fdj, fdk, frdk;
+   float pad[2];
+};
+
 struct OrderArgs {
    const uint32_t* cell_off;
    const uint32_t* unit_base;   // [ncells+1]
+   const uint32_t* out_off;     // [ncells+1]
    const uint4* unit_rec;
+   const uint4* col_rec;
+   const double* isect;
+   const double* minval;
+   double dv_d;                 // cell size along the pass axis
    const uint32_t* len_hist;    // [LEN_BINS] units per length bin
    const uint32_t* cell_hist;   // [LEN_BINS * ncells] exclusive prefix over cells of the bin's units
-   uint32_t* perm;              // [total units] unit record indices (unit_rec), longest first
-   uint32_t* perm_cell;         // [total units] the cell of each perm entry
+   uint4* units;                // [2 * total units] the work list, longest first; per unit
+                                //   {b0 | b1 << 16, cell, columns and flags (unit_rec.z), first column}
+                                //   {the first column's record, its output slot absolute}
+   PassCell* pass_cell;         // [ncells]
    const uint32_t* flags;
    uint32_t ncells;
 };
 
 struct RemapArgs {
-   const uint32_t* cell_off;    // input list offsets (record base of each cell)
    const uint32_t* unit_base;   // [ncells+1] global work-unit index base
    const uint32_t* out_off;     // [ncells+1] output block offsets
-   const uint32_t* perm;        // [total units] unit record indices in processing order
-   const uint32_t* perm_cell;   // [total units] cell of each entry of perm
-   const uint4* unit_rec;
+   const uint4* units;          // [2 * total units] the work list (OrderArgs)
+   const PassCell* pass_cell;   // [ncells]
    const uint4* col_rec;
    const uint32_t* sorted_src;
-   const double* isect;
    Pool in, out;                // source and target pools
    uint32_t* gid_out;
    uint32_t* src_out;
@@ -118,9 +134,6 @@ struct RemapArgs {
    uint32_t ncells;
    uint32_t len[3];
    float dv, vmin;
-   float threshold;             // (float) sparse min value, reconstruction threshold
-   double min_value;            // content test threshold
-   const double* minval;        // [ncells] sparsity threshold per cell (velocityBlockMinValue)
    double dv_d, vmin_d;         // cell size and mesh minimum along the pass axis (FP64)
    int range;                   // exact kernel: RANGE_ALL (every unit before WIDE_BIN's) or
                                 // RANGE_EXACT (EXACT_BIN's units)
@@ -215,7 +228,7 @@ int init_box_words_max();
 
 void launch_columns(int dim, const ColumnArgs& a, hipStream_t s);
 void launch_scan(const ScanArgs& a, hipStream_t s);
-void launch_order(const OrderArgs& a, hipStream_t s);
+void launch_order(int dim, const OrderArgs& a, hipStream_t s);
 void launch_build_scan(const BuildScanArgs& a, hipStream_t s);
 // grid: grid_mult persistent workgroups per CU
 // grid_mult workgroups per compute unit; wgs: lanes per workgroup of the tolerance-form kernel

@@ -621,8 +621,29 @@ __global__ __launch_bounds__(1024) void k_build_scan(BuildScanArgs a) {
    if (threadIdx.x == 0) a.len_hist[blockIdx.x] = tot;
 }
 
-// Global work list of the remap: every unit's global index, ordered by source length
-// (longest first; within a length bin by cell, units are independent).
+// The content test (double)x >= mv of an FP32 value x, as x >= content_threshold(mv): the
+// smallest float whose double value is >= mv (x >= it exactly when (double)x >= mv).
+__device__ inline float content_threshold(double mv) {
+   const float f = (float)mv;   // nearest float: the answer, or the float just below mv
+   return ((double)f < mv) ? nextafterf(f, INFINITY) : f;
+}
+
+template <int DIM>
+__device__ inline void pass_isect_d(const double* is, double& I, double& di, double& dj, double& dk) {
+   I = is[4 * DIM + 0];
+   const double a = is[4 * DIM + 1], b = is[4 * DIM + 2], c = is[4 * DIM + 3];
+   if (DIM == 0) { di = c; dj = b; dk = a; }
+   else if (DIM == 1) { di = a; dj = c; dk = b; }
+   else { di = a; dj = b; dk = c; }
+}
+
+// Global work list of the remap, ordered by source length (longest first; within a length bin by
+// cell, units are independent), with everything a unit starts from: its record, its first
+// column's record and, per cell, PassCell.  A remap unit then waits for one record, then for its
+// cell and source indices together, then for f; an index list waited for index, unit record,
+// column record and source indices one after another, and derived the cell's values (two FP64
+// divisions) per unit.
+template <int DIM>
 __global__ __launch_bounds__(WG) void k_order(OrderArgs a) {
    // one workgroup per cell: the cell's range in each bin starts at the units of the bins before it
    // plus the bin's prefix over cells; units take positions in it through an LDS cursor per bin
@@ -633,17 +654,35 @@ __global__ __launch_bounds__(WG) void k_order(OrderArgs a) {
    const uint32_t base = a.unit_base[c];
    const uint32_t nu = a.unit_base[c + 1] - base;
    if (nu == 0) return;
-   const uint32_t off = a.cell_off[c];
+   const uint32_t off = a.cell_off[c], obase = a.out_off[c];
    if (threadIdx.x < LEN_BINS) {
       const uint32_t n = a.len_hist[threadIdx.x];
       cursor[threadIdx.x] = wave_incl_scan(n) - n + a.cell_hist[(size_t)threadIdx.x * a.ncells + c];
+   } else if (threadIdx.x == LEN_BINS) {
+      PassCell p;
+      double dk;
+      pass_isect_d<DIM>(a.isect + 12 * (size_t)c, p.I, p.di, p.dj, dk);
+      p.rdk = 1.0 / dk;
+      p.r = (float)(dk / a.dv_d);
+      p.inv_r = (float)(a.dv_d * p.rdk);
+      // the content test, and the reconstruction threshold as the Realf argument of
+      // compute_*_coeff (cpu_acc_map.cpp:539-547)
+      const double mv = a.minval[c];
+      p.thc = content_threshold(mv);
+      p.thr = (float)mv;
+      p.scale = (float)(1.0 / (double)p.thr);
+      pass_isect<DIM>(a.isect + 12 * (size_t)c, p.fI, p.fdi, p.fdj, p.fdk);
+      p.frdk = 1.0f / p.fdk;
+      p.pad[0] = p.pad[1] = 0.0f;
+      a.pass_cell[c] = p;
    }
    __syncthreads();
    for (uint32_t u = threadIdx.x; u < nu; u += WG) {
-      const uint32_t b = unit_bin(a.unit_rec[off + u]);
-      const uint32_t pos = atomicAdd(&cursor[b], 1u);
-      a.perm[pos] = off + u;   // the unit's record
-      a.perm_cell[pos] = c;
+      const uint4 r = a.unit_rec[off + u];
+      const uint4 col = a.col_rec[r.y];
+      const size_t pos = atomicAdd(&cursor[unit_bin(r)], 1u);
+      a.units[2 * pos] = make_uint4(r.x, c, r.z, r.y);
+      a.units[2 * pos + 1] = make_uint4(col.x, col.y, col.z, obase + col.w);
    }
 }
 
@@ -732,13 +771,6 @@ __device__ inline void store_pencil(float* __restrict__ f, size_t slot, int o, c
       constexpr int st = Pencil<DIM>::st;
       p[0] = w[0]; p[st] = w[1]; p[2 * st] = w[2]; p[3 * st] = w[3];
    }
-}
-
-// The content test (double)x >= mv of an FP32 value x, as x >= content_threshold(mv): the
-// smallest float whose double value is >= mv (x >= it exactly when (double)x >= mv).
-__device__ inline float content_threshold(double mv) {
-   const float f = (float)mv;   // nearest float: the answer, or the float just below mv
-   return ((double)f < mv) ? nextafterf(f, INFINITY) : f;
 }
 
 __device__ inline void set_content_flag(uint8_t* content, size_t slot, bool has, int setlane0, int l16) {
@@ -879,21 +911,15 @@ __device__ __forceinline__ void remap_units(const RemapArgs& a, double i_dv, flo
    const int o = (DIM == 0) ? (ip * WID2 + jp * WID) : (DIM == 1) ? (jp * WID2 + ip) : (jp * WID + ip);
    const uint32_t gstride = blocks * (WGS / 16);
    for (uint32_t gi = first + block * (WGS / 16) + (tid >> 4); gi < total; gi += gstride) {
-      const uint32_t c = a.perm_cell[gi];
-      const uint4 sr = a.unit_rec[a.perm[gi]];
+      const uint4 sr = a.units[2 * (size_t)gi], first_col = a.units[2 * (size_t)gi + 1];
+      const uint32_t c = sr.y;
+      const PassCell& pc = a.pass_cell[c];
       const int b0 = (int)(sr.x & 0xFFFFu), b1 = (int)(sr.x >> 16);
-      const uint32_t col0 = sr.y;
-      // the cell's sparsity threshold: the content test, and the reconstruction threshold as
-      // the Realf argument of compute_*_coeff (cpu_acc_map.cpp:539-547)
-      const double mv = a.minval[c];
-      const float thc = content_threshold(mv);
-      const float thr = (float)mv;
-      const float scale = (float)(1.0 / (double)thr);
+      const uint32_t col0 = sr.w;
+      const float thc = pc.thc, thr = pc.thr, scale = pc.scale;
       const uint32_t ncol = sr.z & UNIT_NCOL_MASK;
       const bool copy = (sr.z & COPY_FLAG) != 0u;
-      const uint32_t obase = a.out_off[c];
-      float I, di, dj, dk;
-      pass_isect<DIM>(a.isect + 12 * (size_t)c, I, di, dj, dk);
+      const float I = pc.fI, di = pc.fdi, dj = pc.fdj, dk = pc.fdk, rdk = pc.frdk;
       // Lagrangian base of this lane's pencil, cpu_acc_map.cpp:493-496
       const float Imin = (I + (float)(uint32_t)(b0 * WID + ip) * di) + (float)(uint32_t)(b1 * WID + jp) * dj;
       // Columns of a unit have non-decreasing target ranges that overlap only where one ends
@@ -903,12 +929,16 @@ __device__ __forceinline__ void remap_units(const RemapArgs& a, double i_dv, flo
       int prev_end = -1;
       int carry_open = -1;
       for (uint32_t ci = 0; ci < ncol; ++ci) {
-         const uint4 cr = a.col_rec[col0 + ci];
+         uint4 cr = first_col;
+         if (ci) {
+            cr = a.col_rec[col0 + ci];
+            cr.w += a.out_off[c];
+         }
          const int ks = (int)(cr.x & 0xFFFFu), len = (int)(cr.x >> 16);
          const int fk = (int)(cr.z & 0xFFFFu), lk = (int)(cr.z >> 16);
          const int nfk = (ci + 1 < ncol) ? (int)(a.col_rec[col0 + ci + 1].z & 0xFFFFu) : INT_MAX;
          const uint32_t* srcs = a.sorted_src + cr.y;
-         const size_t slotb = (size_t)obase + cr.w;   // output slot of block fk
+         const size_t slotb = cr.w;   // output slot of block fk
          for (int tb = max(fk, prev_end + 1) + l16; tb <= lk; tb += 16) {
             const size_t slot = slotb + (size_t)(tb - fk);
             a.gid_out[slot] = pass_gid<DIM>(b0, b1, tb, a.len);
@@ -922,7 +952,6 @@ __device__ __forceinline__ void remap_units(const RemapArgs& a, double i_dv, flo
          float v_r = (float)(uint32_t)(WID * ks) * a.dv + a.vmin;
          const float lvr = (v_r - Imin) / dk;
          int gkr = (int)lvr;
-         const float rdk = 1.0f / dk;
          // lanes of min/max Lagrangian index within the 8-lane vector (cpu_acc_map.cpp:515-529)
          int minL = 0, maxL = 0;
          {
@@ -1045,15 +1074,6 @@ __global__ __launch_bounds__(WG) void k_remap(RemapArgs a, double i_dv) {
 // row).  Units marked EXACT_FLAG are left to k_remap (range RANGE_EXACT), and those marked
 // WIDE_FLAG to its wide instance.
 
-template <int DIM>
-__device__ inline void pass_isect_d(const double* is, double& I, double& di, double& dj, double& dk) {
-   I = is[4 * DIM + 0];
-   const double a = is[4 * DIM + 1], b = is[4 * DIM + 2], c = is[4 * DIM + 3];
-   if (DIM == 0) { di = c; dj = b; dk = a; }
-   else if (DIM == 1) { di = a; dj = c; dk = b; }
-   else { di = a; dj = b; dk = c; }
-}
-
 // maximum / minimum over the 16 lanes of the caller's DPP row (all active), in every lane of
 // the row (rotations folded into v_max_i32_dpp / v_min_i32_dpp)
 __device__ inline int row_max16(int x) {
@@ -1093,29 +1113,31 @@ __global__ __launch_bounds__(WGS, 5) void k_remap_lean(RemapArgs a) {
    const uint32_t total = a.unit_base[a.ncells] - a.len_hist[EXACT_BIN] - a.len_hist[WIDE_BIN];
    const uint32_t gstride = gridDim.x * (WGS / 16);
    for (uint32_t gi = blockIdx.x * (WGS / 16) + (tid >> 4); gi < total; gi += gstride) {
-      const uint32_t c = a.perm_cell[gi];
-      const uint4 sr = a.unit_rec[a.perm[gi]];
-      const float thc = content_threshold(a.minval[c]);
+      const uint4 sr = a.units[2 * (size_t)gi], first_col = a.units[2 * (size_t)gi + 1];
+      const uint32_t c = sr.y;
+      const PassCell& pc = a.pass_cell[c];
+      const float thc = pc.thc;
       const int b0 = (int)(sr.x & 0xFFFFu), b1 = (int)(sr.x >> 16);
-      const uint32_t col0 = sr.y;
+      const uint32_t col0 = sr.w;
       const uint32_t ncol = sr.z & UNIT_NCOL_MASK;
       const bool copy = (sr.z & COPY_FLAG) != 0u;
-      const uint32_t obase = a.out_off[c];
-      double I, di, dj, dk;
-      pass_isect_d<DIM>(a.isect + 12 * (size_t)c, I, di, dj, dk);
       // Lagrangian base of this lane's pencil and the boundary spacing in cells
-      const double imin = I + (double)(b0 * WID + ip) * di + (double)(b1 * WID + jp) * dj;
-      const double rdk = 1.0 / dk;
-      const float r = (float)(dk / a.dv_d), inv_r = (float)(a.dv_d * rdk);
+      const double imin = pc.I + (double)(b0 * WID + ip) * pc.di + (double)(b1 * WID + jp) * pc.dj;
+      const double rdk = pc.rdk;
+      const float r = pc.r, inv_r = pc.inv_r;
       int prev_end = -1;
       int carry_open = -1;
       for (uint32_t ci = 0; ci < ncol; ++ci) {
-         const uint4 cr = a.col_rec[col0 + ci];
+         uint4 cr = first_col;
+         if (ci) {
+            cr = a.col_rec[col0 + ci];
+            cr.w += a.out_off[c];
+         }
          const int ks = (int)(cr.x & 0xFFFFu), len = (int)(cr.x >> 16);
          const int fk = (int)(cr.z & 0xFFFFu), lk = (int)(cr.z >> 16);
          const int nfk = (ci + 1 < ncol) ? (int)(a.col_rec[col0 + ci + 1].z & 0xFFFFu) : INT_MAX;
          const uint32_t* srcs = a.sorted_src + cr.y;
-         const size_t slotb = (size_t)obase + cr.w;   // output slot of block fk
+         const size_t slotb = cr.w;   // output slot of block fk
          for (int tb = max(fk, prev_end + 1) + l16; tb <= lk; tb += 16) {
             const size_t slot = slotb + (size_t)(tb - fk);
             a.gid_out[slot] = pass_gid<DIM>(b0, b1, tb, a.len);
@@ -2067,9 +2089,11 @@ void launch_columns(int dim, const ColumnArgs& a, hipStream_t s) {
    else hipLaunchKernelGGL(k_columns<2>, dim3(a.ncells), dim3(CWG), 0, s, a);
 }
 
-void launch_order(const OrderArgs& a, hipStream_t s) {
+void launch_order(int dim, const OrderArgs& a, hipStream_t s) {
    if (a.ncells == 0) return;
-   hipLaunchKernelGGL(k_order, dim3(a.ncells), dim3(WG), 0, s, a);
+   if (dim == 0) hipLaunchKernelGGL(k_order<0>, dim3(a.ncells), dim3(WG), 0, s, a);
+   else if (dim == 1) hipLaunchKernelGGL(k_order<1>, dim3(a.ncells), dim3(WG), 0, s, a);
+   else hipLaunchKernelGGL(k_order<2>, dim3(a.ncells), dim3(WG), 0, s, a);
 }
 
 void launch_build_scan(const BuildScanArgs& a, hipStream_t s) {
