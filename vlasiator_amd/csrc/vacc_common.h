@@ -61,6 +61,15 @@ VACC_HD void gid_xyz(uint32_t g, const GidSplit& s, uint32_t& x, uint32_t& y, ui
    x = r - y * s.nx.d;
 }
 
+// Median of three finite values.
+VACC_HD float med3(float x, float y, float z) {
+#if defined(__HIP_DEVICE_COMPILE__)
+   return __builtin_amdgcn_fmed3f(x, y, z);
+#else
+   return fmaxf(fminf(x, y), fminf(fmaxf(x, y), z));
+#endif
+}
+
 // physical constants (common.h physicalconstants)
 constexpr double MU_0 = 1.25663706e-6;
 constexpr double PI = 3.14159265358979323846;

@@ -44,14 +44,6 @@ VACC_HD float lean_rcp(float x) {
    return 1.0f / x;
 #endif
 }
-// median of three finite values
-VACC_HD float lean_med3(float x, float y, float z) {
-#if defined(__HIP_DEVICE_COMPILE__)
-   return __builtin_amdgcn_fmed3f(x, y, z);
-#else
-   return fmaxf(fminf(x, y), fminf(fmaxf(x, y), z));
-#endif
-}
 VACC_HD float lean_sqrt(float x) {
 #if defined(__HIP_DEVICE_COMPILE__)
    return __builtin_amdgcn_sqrtf(x);
@@ -84,10 +76,10 @@ VACC_HD float lean_h7h(const float* v) {
 // one, or 0 when the signs differ (the outer median is then 0 as well).  Two instructions with
 // the halves carried from cell to cell, in place of ten.
 VACC_HD float lean_half_superbee(float a, float b, float ha, float hb) {
-   return lean_med3(ha, hb, lean_med3(a, b, 0.0f));
+   return med3(ha, hb, med3(a, b, 0.0f));
 }
 // u lies outside the closed interval between 0 and a (a face outside its two cells' averages)
-VACC_HD bool lean_outside(float u, float a) { return lean_med3(u, 0.0f, a) != u; }
+VACC_HD bool lean_outside(float u, float a) { return med3(u, 0.0f, a) != u; }
 
 template <int METHOD>
 struct ReconLean;
@@ -137,8 +129,8 @@ struct ReconLean<VACC_PPM> {
       // Colella-Woodward: (p - m)(v - (m + p)/2) > (p - m)^2 / 6  <=>  (u_r - u_l)(u_l + 2 u_r) < 0.
       // After the face checks u_l and u_r have opposite signs (or are 0), so this is |u_l| > 2 |u_r|,
       // and u_l becomes the smaller of u_l and -2 u_r; the right test likewise.
-      ul = lean_med3(ul, -2.0f * ur, 0.0f);
-      ur = lean_med3(ur, -2.0f * ul, 0.0f);
+      ul = med3(ul, -2.0f * ur, 0.0f);
+      ur = med3(ur, -2.0f * ul, 0.0f);
       fl = fr;
       b = a;
       hb = ha;
