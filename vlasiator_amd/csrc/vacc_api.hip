@@ -2381,6 +2381,7 @@ int vacc_trans_map_1d(vacc_ctx* c, uint32_t dim, double dt) {
    ta.nblocks = (uint32_t)c->nblocks;
    ta.dim = (int)dim;
    for (int d = 0; d < 3; ++d) ta.len[d] = c->mi.len[d];
+   ta.gs = make_gid_split(c->mi.len);
    ta.dvz = (float)c->mi.cell[dim];
    ta.vz_min = (float)c->mi.vmin[dim];
    ta.dt = (float)dt;

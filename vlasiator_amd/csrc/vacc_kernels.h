@@ -397,6 +397,7 @@ struct TransArgs {
    uint32_t nblocks;
    int dim;
    uint32_t len[3];
+   GidSplit gs;            // block coordinates of a GID (from len)
    float dvz, vz_min;      // (float) cell size and mesh minimum along dim
    float dt;
    float thr;              // reconstruction threshold

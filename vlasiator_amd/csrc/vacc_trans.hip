@@ -52,26 +52,17 @@ __device__ inline float face_nu(const TransFace& F, float um2, float um1, float 
 }
 
 // Filter and monotonicity of PPM on non-uniform widths (cpu_face_estimates.hpp:327-372,
-// cpu_1d_ppm_nonuniform.hpp:40-62) from the raw h4 faces m, p of the source cell u0 with
-// neighbours um1, up1.
-__device__ inline void ppm_nu_coeffs(float m, float p, float um1, float u0, float up1, float thr, float scale,
-                                     float& c0, float& c1, float& c2) {
-   float sl, sabs;
-   if (thr > 0.0f) {
-      const float sm = um1 * scale, s0 = u0 * scale, sp = up1 * scale;
-      sl = superbee_ab(sp - s0, s0 - sm);
-      sabs = fabsf(sl) * thr;
-   } else {
-      sl = superbee_ab(up1 - u0, u0 - um1);
-      sabs = fabsf(sl);
-   }
-   const float ssgn = (sl > 0.0f) ? 1.0f : -1.0f;
-   if (sabs == 0.0f) {
-      p = u0;
-      m = u0;
-   }
-   if ((um1 - m) * (m - u0) < 0.0f) m = u0 - (0.5f * ssgn) * sabs;
-   if ((up1 - p) * (p - u0) < 0.0f) p = u0 + (0.5f * ssgn) * sabs;
+// cpu_1d_ppm_nonuniform.hpp:40-62) from the raw h4 faces m, p of the source cell u0.  sl: the signed
+// limited slope (the reference's sign |slope|); mout, pout: the raw faces' tests
+// (um1 - m)(m - u0) < 0 and (up1 - p)(p - u0) < 0.
+__device__ inline void ppm_nu_limit(float m, float p, float u0, float sl, bool mout, bool pout, float& c0, float& c1,
+                                    float& c2) {
+   const float hs = 0.5f * sl;
+   const bool flat = sl == 0.0f;   // both faces at u0; their tests are then products with 0
+   m = mout ? u0 - hs : m;
+   p = pout ? u0 + hs : p;
+   m = flat ? u0 : m;
+   p = flat ? u0 : p;
    const float one_sixth = (float)(1.0 / 6.0);
    {
       const float d = p - m;
@@ -88,20 +79,29 @@ __device__ inline void ppm_nu_coeffs(float m, float p, float um1, float u0, floa
    c2 = (m + p) - 2.0f * u0;
 }
 
+// The limiter works on values times scale = 1 / threshold when the threshold is positive.
+__device__ inline float limiter_scale(float thr, float scale) { return (thr > 0.0f) ? scale : 1.0f; }
+__device__ inline float limiter_unscale(float thr) { return (thr > 0.0f) ? thr : 1.0f; }
+
 // PPM of the source with stencil u[0..4] = values at k-2..k+2.
 __device__ inline void ppm_nu(const TransEntry& E, const float (&u)[5], float thr, float scale, float& c0, float& c1,
                               float& c2) {
    const float m = face_nu(E.fl, u[0], u[1], u[2], u[3]);
    const float p = face_nu(E.fr, u[1], u[2], u[3], u[4]);
-   ppm_nu_coeffs(m, p, u[1], u[2], u[3], thr, scale, c0, c1, c2);
+   const float sc = limiter_scale(thr, scale);
+   const float sm = u[1] * sc, s0 = u[2] * sc, sp = u[3] * sc;
+   const float sl = superbee_ab(sp - s0, s0 - sm) * limiter_unscale(thr);
+   ppm_nu_limit(m, p, u[2], sl, (u[1] - m) * (m - u[2]) < 0.0f, (u[3] - p) * (p - u[2]) < 0.0f, c0, c1, c2);
 }
 
 // Integral of the reconstruction over the part of the cell that leaves it
-// (cpu_trans_map_amr.cpp:75-106): ng for a Courant number zt.
-__device__ inline float leaving(float zt, float c0, float c1, float c2) {
+// (cpu_trans_map_amr.cpp:75-106): ng between z1 and z2, those of a Courant number zt.
+__device__ inline void leaving_range(float zt, float& z1, float& z2) {
    const bool pos = zt > 0.0f;
-   const float z1 = pos ? (float)(1.0 - (double)zt) : 0.0f;
-   const float z2 = pos ? 1.0f : -zt;
+   z1 = pos ? (float)(1.0 - (double)zt) : 0.0f;
+   z2 = pos ? 1.0f : -zt;
+}
+__device__ inline float leaving(float z1, float z2, float c0, float c1, float c2) {
    return z2 * (c0 + z2 * (c1 + z2 * c2)) - z1 * (c0 + z1 * (c1 + z1 * c2));
 }
 
@@ -151,7 +151,9 @@ __device__ inline void copy_block(const Pool& in, const Pool& out, uint32_t sb, 
 // v dt of the lane's velocity cell along dim for block g (cpu_trans_map_amr.cpp:74-75): the
 // cell-centre velocity in double, rounded to Realf, times the Realf dt.
 __device__ inline float cell_vdt(const TransArgs& a, uint32_t g, int tk) {
-   const uint32_t bz = (a.dim == 0) ? g % a.len[0] : (a.dim == 1) ? (g / a.len[0]) % a.len[1] : g / (a.len[0] * a.len[1]);
+   uint32_t bx, by, bzz;
+   gid_xyz(g, a.gs, bx, by, bzz);
+   const uint32_t bz = (a.dim == 0) ? bx : (a.dim == 1) ? by : bzz;
    const float cell_vz = (float)(((double)(bz * 4u + (uint32_t)tk) + 0.5) * (double)a.dvz + (double)a.vz_min);
    return cell_vz * a.dt;
 }
@@ -279,7 +281,9 @@ __global__ __launch_bounds__(TWG) void k_trans(TransArgs a) {
                if (E.kind != 1 && __ballot(take) == 0ull) continue;
                float c0, c1, c2;
                ppm_nu(E, u, a.thr, a.scale, c0, c1, c2);
-               const float ng = leaving(zt, c0, c1, c2);
+               float z1, z2;
+               leaving_range(zt, z1, z2);
+               const float ng = leaving(z1, z2, c0, c1, c2);
                float contrib;
                if (E.kind == 1) {
                   contrib = (u[2] - ng) * E.ratio;
@@ -294,16 +298,25 @@ __global__ __launch_bounds__(TWG) void k_trans(TransArgs a) {
    }
 }
 
-// Minimum and maximum over the wave (uniform results).
+// Minimum over the wave (all lanes active, uniform result): DPP rotations within the rows of 16
+// lanes, then the rows' minima in scalar registers.
 __device__ inline uint32_t wave_min(uint32_t x) {
-#pragma unroll
-   for (int o = 32; o > 0; o >>= 1) x = min(x, (uint32_t)__shfl_xor((int)x, o, 64));
-   return (uint32_t)__builtin_amdgcn_readfirstlane((int)x);
+   x = min(x, row_ror_u<8>(x));
+   x = min(x, row_ror_u<4>(x));
+   x = min(x, row_ror_u<2>(x));
+   x = min(x, row_ror_u<1>(x));
+   const uint32_t a = (uint32_t)__builtin_amdgcn_readlane((int)x, 0), b = (uint32_t)__builtin_amdgcn_readlane((int)x, 16);
+   const uint32_t c = (uint32_t)__builtin_amdgcn_readlane((int)x, 32), d = (uint32_t)__builtin_amdgcn_readlane((int)x, 48);
+   return min(min(a, b), min(c, d));
 }
-__device__ inline uint32_t wave_max(uint32_t x) {
-#pragma unroll
-   for (int o = 32; o > 0; o >>= 1) x = max(x, (uint32_t)__shfl_xor((int)x, o, 64));
-   return (uint32_t)__builtin_amdgcn_readfirstlane((int)x);
+
+// The groups of 8 lanes with a bit in m, all their bits set (check_skip_remapping's groups).
+__device__ inline unsigned long long group8(unsigned long long m) {
+   m |= m >> 4;
+   m |= m >> 2;
+   m |= m >> 1;
+   m &= 0x0101010101010101ull;
+   return (m << 8) - m;
 }
 
 // Work split of the pencil walk: for each segment, the walked cells' blocks (pairs of a walked
@@ -385,11 +398,17 @@ __global__ __launch_bounds__(TWG) void k_walk_bounds(WalkArgs w, uint32_t* bound
 // A cell that several pencils write (one run position each), or whose two positions lie in
 // different segments of one pencil, is walked in launch levels in the reference's order; a
 // later level's sum starts from the block the earlier one stored (FP32).
-// Waves per SIMD: seven for FP32 (72 VGPRs with 12 bytes per lane spilled, 5 % faster than
-// six waves at 80 VGPRs without a spill) and six for the 16-bit forms (80 VGPRs instead of 85,
-// no spill).
+// Bound by the latency of its loads and by its scalar work per source (window bits, branches,
+// addresses), less by VALU issue: 20 % fewer VALU instructions alone gained nothing, while runs with
+// a shifting window mask, one test per finished position, a path without the 8-lane groups and
+// pool indices fetched with the GIDs took a call over 7.3 million blocks (1024 cells, PQM
+// workload, 16 x 8 x 8 periodic) from 3.35 to 2.89 ms.  Faces through scalar loads instead of LDS
+// (3.03 ms), values two sources ahead (no change) and a shared reciprocal for the widths' quotients
+// (3 % slower: its range test costs a branch) were measured and not kept.
+// Waves per SIMD: eight for FP32 (64 VGPRs, 8 bytes per lane spilled; 2 % faster than seven) and
+// seven for the 16-bit forms.
 template <int ST>
-__global__ __launch_bounds__(TWG) __attribute__((amdgpu_waves_per_eu(ST == ST_F32 ? 7 : 6))) void k_trans_walk(
+__global__ __launch_bounds__(TWG) __attribute__((amdgpu_waves_per_eu(ST == ST_F32 ? 8 : 7))) void k_trans_walk(
     WalkArgs w) {
    // per wave: the current segment's faces (window positions 0..n-1)
    __shared__ TransFace s_face[TWG / 64][WALK_MAXN];
@@ -399,6 +418,7 @@ __global__ __launch_bounds__(TWG) __attribute__((amdgpu_waves_per_eu(ST == ST_F3
    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)((blockIdx.x * (uint32_t)TWG + threadIdx.x) >> 6));
    const uint32_t nwaves = (gridDim.x * (uint32_t)TWG) >> 6;
    const uint32_t nunits = w.nseg * w.wps;
+   const float lsc = limiter_scale(a.thr, a.scale), lus = limiter_unscale(a.thr);
    const int ti = lane & 3, tj = (lane >> 2) & 3, tk = lane >> 4;
    const int ab = (a.dim == 0) ? ti * 16 + tj * 4 + tk : (a.dim == 1) ? ti + tj * 16 + tk * 4 : lane;
    for (uint32_t u = wave; u < nunits; u += nwaves) {
@@ -409,7 +429,7 @@ __global__ __launch_bounds__(TWG) __attribute__((amdgpu_waves_per_eu(ST == ST_F3
       const TransFace* F = s_face[wv];
       bool faces = false;   // F holds this segment's faces
       // lane q < n: window position q, its list [cur, hi) from the first GID >= glo
-      uint32_t cur = 0, hi = 0, cg = VACC_INVALID_ID, pf = 0;
+      uint32_t cur = 0, hi = 0, cg = VACC_INVALID_ID, cs = VACC_INVALID_ID, pf = 0;
       float dzl = 0.0f, rl = 0.0f;
       if ((uint32_t)lane < S.n) {
          const WalkPos P = w.pos[S.pos0 + lane];
@@ -427,6 +447,7 @@ __global__ __launch_bounds__(TWG) __attribute__((amdgpu_waves_per_eu(ST == ST_F3
             }
             cur = lo;
             cg = (cur < hi) ? a.gid[cur] : VACC_INVALID_ID;
+            cs = (cur < hi) ? a.src[cur] : VACC_INVALID_ID;
          }
       }
       const bool walked = (pf & WALK_W) != 0u;
@@ -447,17 +468,19 @@ __global__ __launch_bounds__(TWG) __attribute__((amdgpu_waves_per_eu(ST == ST_F3
             if (cg < g) {
                ++cur;
                cg = (cur < hi) ? a.gid[cur] : VACC_INVALID_ID;
+               cs = (cur < hi) ? a.src[cur] : VACC_INVALID_ID;
             }
          }
          const bool have = cg == g;
          const unsigned long long tmask = wmask & __ballot(have);   // positions written for g
-         const uint32_t pidx = have ? a.src[cur] : VACC_INVALID_ID;
+         const uint32_t pidx = have ? cs : VACC_INVALID_ID;
          const uint32_t ob = cur;                                    // output block where have
          // the cursors that hold g move on now, so that the next GID's lookup is in flight
          // during the walk
          if (have) {
             ++cur;
             cg = (cur < hi) ? a.gid[cur] : VACC_INVALID_ID;
+            cs = (cur < hi) ? a.src[cur] : VACC_INVALID_ID;
          }
          if (!faces) {
             const uint32_t* src = (const uint32_t*)(w.face + S.pos0);
@@ -470,19 +493,20 @@ __global__ __launch_bounds__(TWG) __attribute__((amdgpu_waves_per_eu(ST == ST_F3
             faces = true;
          }
          const float vdt = cell_vdt(a, g, tk);
-         // value at window position min(q, n-1) (uniform q); the load is not conditional (block
-         // 0 stands in for a missing block, whose value is then 0), so that it can be in
-         // flight while earlier work runs
+         // value at window position q (uniform q); the load is not conditional (block 0 stands in
+         // for a missing block, whose value is then 0), so that it can be in flight while earlier
+         // work runs.  Positions at or above n are only asked for ahead of use, by the last source.
+         const unsigned long long vmask = __ballot(pidx != VACC_INVALID_ID);
+         const uint32_t vidx = (pidx != VACC_INVALID_ID) ? pidx : 0u;
          auto val = [&](int q) -> float {
-            const uint32_t idx = (uint32_t)__builtin_amdgcn_readlane((int)pidx, min(q, n - 1));
-            const float x = pool_val<ST>(a.in, (idx != VACC_INVALID_ID) ? idx : 0u, ab);
-            return (idx != VACC_INVALID_ID) ? x : 0.0f;
+            const float x = pool_val<ST>(a.in, (uint32_t)__builtin_amdgcn_readlane((int)vidx, q & 63), ab);
+            return (vmask & (1ull << (q & 63))) ? x : 0.0f;
          };
          float c1 = 0.0f, c2 = 0.0f;   // carry registers
          // start of window position q's sum: zero or a carry register
          const unsigned long long inited = init1 | init2 | inits;
          auto start = [&](int q) -> float {
-            if (!((inited >> q) & 1ull)) return 0.0f;   // the common case, a uniform branch
+            if (!(inited & (1ull << q))) return 0.0f;   // the common case, a uniform branch
             if constexpr (ST == ST_F32) {
                // the sum an earlier launch level stored into this block
                if (((inits & tmask) >> q) & 1ull)
@@ -491,11 +515,11 @@ __global__ __launch_bounds__(TWG) __attribute__((amdgpu_waves_per_eu(ST == ST_F3
             return ((init1 >> q) & 1ull) ? c1 : ((init2 >> q) & 1ull) ? c2 : 0.0f;
          };
          // end of window position q's sum x: into a carry register or the block
+         const unsigned long long plain = tmask & ~(save1 | save2);
          auto retire = [&](int q, float x) {
-            if (!((tmask >> q) & 1ull)) return;
-            if ((save1 >> q) & 1ull) c1 = x;
-            else if ((save2 >> q) & 1ull) c2 = x;
-            else store_block<ST>(a.out, (uint32_t)__builtin_amdgcn_readlane((int)ob, q), x, ab, a.dim, lane);
+            if (plain & (1ull << q)) store_block<ST>(a.out, (uint32_t)__builtin_amdgcn_readlane((int)ob, q), x, ab, a.dim, lane);
+            else if (save1 & tmask & (1ull << q)) c1 = x;
+            else if (save2 & tmask & (1ull << q)) c2 = x;
          };
          // sources next to a written position.  Where every lane moves up (v dt > 0) each m1 is
          // +-0 (zt > 0 or, if zt underflows, a leaving integral of +-0), and where none does
@@ -509,28 +533,78 @@ __global__ __launch_bounds__(TWG) __attribute__((amdgpu_waves_per_eu(ST == ST_F3
          // they receive nothing
          unsigned long long rel = (reach & smask) | (((tmask >> (je + 1)) & 1ull) << je) |
                                   (((tmask >> (js - 1)) & 1ull) << js);
-         float u0 = 0.0f, u1 = 0.0f, u2 = 0.0f, u3 = 0.0f, u4 = 0.0f, nx = 0.0f, fl = 0.0f;
-         float am = 0.0f, a0 = 0.0f;   // sums of positions j-1, j
-         float dzc = __builtin_nanf(""), zt = 0.0f;   // zt = vdt / dzc
-         int prev = -2;
+         float dzc = __builtin_nanf("");
+         float z1 = 0.0f, z2 = 0.0f;   // the leaving part's range for zt = vdt / dzc
+         bool pos = false;             // zt > 0
+         // runs of consecutive sources; within a run a source is a shift of the stencil, one new
+         // value (loaded a source ahead) and one new face
          while (rel) {
-            const int j = __builtin_ctzll(rel);
-            rel &= rel - 1ull;
-            if (j != prev + 1) {   // a new run: the previous one ends, the stencil is loaded
-               if (prev >= 0) {
-                  retire(prev, am);
-                  retire(prev + 1, a0);
+            int j = __builtin_ctzll(rel);
+            const int jend = j + __builtin_ctzll(~(rel >> j));   // j >= 2, so the shifted mask ends in zeros
+            rel &= ~0ull << (jend & 63);
+            if (jend > 63) rel = 0ull;
+            float u0 = val(j - 2), u1 = val(j - 1), u2 = val(j), u3 = val(j + 1), u4 = val(j + 2), nx = val(j + 3);
+            float fl = face_nu(F[j], u0, u1, u2, u3);
+            // carried from source to source: the scaled value and its difference to the one before
+            // (limiter), and the left face's test
+            float s0 = u2 * lsc, sb = s0 - u1 * lsc;
+            bool lout = (u1 - fl) * (fl - u2) < 0.0f;
+            float am = start(j - 1), a0 = start(j);   // sums of positions j-1, j
+            unsigned long long tm = tmask >> (j - 1);   // bits 0, 1, 2: positions j-1, j, j+1 are written
+            for (;;) {
+               float ap = start(j + 1);   // sum of position j+1
+               const float fr = face_nu(F[j + 1], u1, u2, u3, u4);
+               const float sp = u3 * lsc, sa = sp - s0;
+               // the right face's test, the next source's left one (the same product, both factors negated)
+               const bool rout = (u3 - fr) * (fr - u2) < 0.0f;
+               // check_skip_remapping (cpu_trans_map_amr.cpp:18-25) per group of 8 lanes
+               const bool any = (u0 > 0.0f) || (u1 > 0.0f) || (u2 > 0.0f) || (u3 > 0.0f) || (u4 > 0.0f);
+               const unsigned long long amask = __ballot(any);
+               if (amask) {
+                  float k0, k1, k2;
+                  ppm_nu_limit(fl, fr, u2, superbee_ab(sa, sb) * lus, lout, rout, k0, k1, k2);
+                  const float dzj = lanef(dzl, j);
+                  if (!(dzj == dzc)) {
+                     dzc = dzj;
+                     const float zt = vdt / dzj;
+                     leaving_range(zt, z1, z2);
+                     pos = zt > 0.0f;
+                  }
+                  const float ng = leaving(z1, z2, k0, k1, k2);
+                  // a contribution that is +-0 in every lane leaves a sum unchanged (sums start
+                  // at +0 or at a sum, and x + (+-0) = x for x != 0, +0 + (+-0) = +0)
+                  if (amask == ~0ull) {   // no group is left out, the common case
+                     if (tm & 2ull) a0 = a0 + (u2 - ng) * lanef(rl, j);
+                     if ((tm & 4ull) && __ballot(pos)) {
+                        const float x = (ng * dzj) / lanef(dzl, j + 1);
+                        ap = ap + (pos ? x : 0.0f) * lanef(rl, j + 1);
+                     }
+                     if ((tm & 1ull) && __ballot(!pos)) {
+                        const float x = (ng * dzj) / lanef(dzl, j - 1);
+                        am = am + (!pos ? x : 0.0f) * lanef(rl, j - 1);
+                     }
+                  } else {
+                     const bool act = ((amask >> (lane & 56)) & 0xFFull) != 0ull;
+                     if ((tm & 2ull) && act) a0 = a0 + (u2 - ng) * lanef(rl, j);
+                     if ((tm & 4ull) && __ballot(pos && act)) {
+                        const float x = (ng * dzj) / lanef(dzl, j + 1);
+                        if (act) ap = ap + (pos ? x : 0.0f) * lanef(rl, j + 1);
+                     }
+                     if ((tm & 1ull) && __ballot(!pos && act)) {
+                        const float x = (ng * dzj) / lanef(dzl, j - 1);
+                        if (act) am = am + (!pos ? x : 0.0f) * lanef(rl, j - 1);
+                     }
+                  }
                }
-               u0 = val(j - 2);
-               u1 = val(j - 1);
-               u2 = val(j);
-               u3 = val(j + 1);
-               u4 = val(j + 2);
-               nx = val(j + 3);
-               fl = face_nu(F[j], u0, u1, u2, u3);
-               am = start(j - 1);
-               a0 = start(j);
-            } else {
+               retire(j - 1, am);
+               am = a0;
+               a0 = ap;
+               fl = fr;
+               s0 = sp;
+               sb = sa;
+               lout = rout;
+               if (++j == jend) break;
+               tm >>= 1;
                u0 = u1;
                u1 = u2;
                u2 = u3;
@@ -538,44 +612,8 @@ __global__ __launch_bounds__(TWG) __attribute__((amdgpu_waves_per_eu(ST == ST_F3
                u4 = nx;
                nx = val(j + 3);
             }
-            prev = j;
-            float ap = start(j + 1);   // sum of position j+1
-            const float fr = face_nu(F[j + 1], u1, u2, u3, u4);
-            const bool wm = (tmask >> (j - 1)) & 1ull, ws = (tmask >> j) & 1ull, wp = (tmask >> (j + 1)) & 1ull;
-            // check_skip_remapping (cpu_trans_map_amr.cpp:18-25) per group of 8 lanes
-            const bool any = (u0 > 0.0f) || (u1 > 0.0f) || (u2 > 0.0f) || (u3 > 0.0f) || (u4 > 0.0f);
-            const unsigned long long amask = __ballot(any);
-            const bool act = ((amask >> (lane & 56)) & 0xFFull) != 0ull;
-            if (amask) {
-               float k0, k1, k2;
-               ppm_nu_coeffs(fl, fr, u1, u2, u3, a.thr, a.scale, k0, k1, k2);
-               const float dzj = lanef(dzl, j);
-               if (!(dzj == dzc)) {
-                  dzc = dzj;
-                  zt = vdt / dzj;
-               }
-               const float ng = leaving(zt, k0, k1, k2);
-               const bool pos = zt > 0.0f;
-               if (ws && act) a0 = a0 + (u2 - ng) * lanef(rl, j);
-               // a contribution that is +-0 in every lane leaves a sum unchanged (sums start
-               // at +0 or at a sum, and x + (+-0) = x for x != 0, +0 + (+-0) = +0)
-               if (wp && __ballot(pos && act)) {
-                  const float x = (ng * dzj) / lanef(dzl, j + 1);
-                  if (act) ap = ap + (pos ? x : 0.0f) * lanef(rl, j + 1);
-               }
-               if (wm && __ballot(!pos && act)) {
-                  const float x = (ng * dzj) / lanef(dzl, j - 1);
-                  if (act) am = am + (!pos ? x : 0.0f) * lanef(rl, j - 1);
-               }
-            }
             retire(j - 1, am);
-            am = a0;
-            a0 = ap;
-            fl = fr;
-         }
-         if (prev >= 0) {
-            retire(prev, am);
-            retire(prev + 1, a0);
+            retire(j, a0);
          }
       }
    }
