@@ -725,52 +725,129 @@ __device__ inline float4 pool_row(const Pool& pl, uint32_t b, int q) {
                       sc * dec16(pl.storage, r.y & 0xFFFFu), sc * dec16(pl.storage, r.y >> 16));
 }
 
-template <int DIM>
-struct Pencil {
-   int o;   // offset of the pencil's first cell in a block
-   static constexpr int st = (DIM == 0) ? 1 : (DIM == 1) ? 4 : 16;   // stride along the pass axis
+// 4 x 4 transpose over the lanes of a quad: lane q gets element q of the quad's four lanes, in
+// lane order.  Two stages of exchanges, lane ^ 1 and then lane ^ 2, each a select between the
+// lane's own value and its partner's folded into one v_cndmask_b32_dpp: eight instructions (the
+// compiler's form of the same is a DPP move and a select each).  A DPP operand has to be two wait
+// states old: the leading and trailing s_nop see to that for what stands before and after, and
+// inside the block every value is read two or more instructions after it is written.
+__device__ inline void quad_transpose(float (&w)[4]) {
+   float t0, t1, a = w[0], b = w[1], c = w[2], d = w[3];
+   asm("s_mov_b64 vcc, %[even]\n\t"
+       "s_nop 0\n\t"
+       "v_cndmask_b32_dpp %[t0], %[b], %[a], vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+       "v_cndmask_b32_dpp %[t1], %[d], %[c], vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+       "s_not_b64 vcc, vcc\n\t"
+       "v_cndmask_b32_dpp %[b], %[a], %[b], vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+       "v_cndmask_b32_dpp %[d], %[c], %[d], vcc quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+       "s_mov_b64 vcc, %[low]\n\t"
+       "v_cndmask_b32_dpp %[a], %[t1], %[t0], vcc quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+       "v_cndmask_b32_dpp %[c], %[d], %[b], vcc quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+       "s_not_b64 vcc, vcc\n\t"
+       "v_cndmask_b32_dpp %[t1], %[t0], %[t1], vcc quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+       "v_cndmask_b32_dpp %[d], %[b], %[d], vcc quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+       "s_nop 1"
+       : [t0] "=&v"(t0), [t1] "=&v"(t1), [a] "+&v"(a), [b] "+&v"(b), [c] "+&v"(c), [d] "+&v"(d)
+       : [even] "s"(0x5555555555555555ull), [low] "s"(0x3333333333333333ull)
+       : "vcc", "scc");
+   w[0] = a;
+   w[1] = c;
+   w[2] = t1;
+   w[3] = d;
+}
+
+// The same for the quad's rows of four 16-bit codes (two per word): halves exchanged with lane ^ 1,
+// then words with lane ^ 2.
+__device__ inline uint2 quad_transpose16(uint2 q) {
+   const uint32_t sel = (threadIdx.x & 1) ? 0x03020706u : 0x05040100u;
+   const uint32_t x1 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)q.x, 0xB1, 0xF, 0xF, true);   // quad_perm [1,0,3,2]
+   const uint32_t y1 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)q.y, 0xB1, 0xF, 0xF, true);
+   const uint32_t n0 = __builtin_amdgcn_perm(x1, q.x, sel), n1 = __builtin_amdgcn_perm(y1, q.y, sel);
+   uint32_t m0, m1;
+   asm("s_mov_b64 vcc, %[low]\n\t"
+       "s_nop 0\n\t"
+       "v_cndmask_b32_dpp %[m0], %[n1], %[n0], vcc quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+       "s_not_b64 vcc, vcc\n\t"
+       "v_cndmask_b32_dpp %[m1], %[n0], %[n1], vcc quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf\n\t"
+       "s_nop 1"
+       : [m0] "=&v"(m0), [m1] "=&v"(m1)
+       : [n0] "v"(n0), [n1] "v"(n1), [low] "s"(0x3333333333333333ull)
+       : "vcc", "scc");
+   return make_uint2(m0, m1);
+}
+
+// How lane (ip, jp) of a unit reads and writes its share of a block.  Its pencil runs along the pass
+// axis at (j, k) = (jp, ip) for DIM 0, (i, k) = (ip, jp) for DIM 1 and (i, j) = (ip, jp) for DIM 2.
+//   ROW: a row of 4 cells along i, 16 bytes (FP32) or 8 in one access.  For DIM 1 and 2 the quad's four
+//   rows, which differ in the pass axis, are transposed.
+//   otherwise the pencil's four values, 16 cells apart (DIM 2, FP32): each access is then 64
+//   contiguous bytes per unit, and the transposes cost more than the accesses saved.
+// By values, DIM 1 took four accesses of four 16-byte pieces per unit each, and the 16-bit forms four
+// of 2 bytes per lane.  Rows: y pass over 26 million blocks 4.88 -> 4.63 ms (PQM, FP32; z the other
+// way, 4.32 -> 4.77), step 18.7 -> 18.0 ms (8192 cells, BF16), 1.51 -> 1.42 ms (517 cells, FP16).
+template <int DIM, int ST>
+struct Access {
+   static constexpr bool ROW = !(DIM == 2 && ST == ST_F32);
+   __device__ static inline int offset(int ip, int jp) {   // first cell of the lane's share
+      if (!ROW) return jp * WID + ip;
+      return (DIM == 1) ? (jp * WID2 + ip * WID) : (ip * WID2 + jp * WID);
+   }
 };
 
-// Load the lane's pencil (4 cells along the pass axis) of source block sidx, decoded to FP32.
+// A lane's share of a source block as stored, and its pencil of the same block, decoded to FP32.
+// The two are apart so that the wait for the load stands where the values are first needed.
+template <int ST>
+struct Share {
+   uint2 q;
+   float sc;
+};
+template <>
+struct Share<ST_F32> {
+   float4 v;
+};
 template <int DIM, int ST>
-__device__ inline void load_pencil(const Pool& pl, uint32_t sidx, int o, float (&w)[4]) {
-   if (sidx == INVALID) {
-      w[0] = w[1] = w[2] = w[3] = 0.0f;
-      return;
-   }
-   constexpr int st = Pencil<DIM>::st;
+__device__ inline Share<ST> load_share(const Pool& pl, uint32_t sidx, int o) {
+   Share<ST> r{};   // zeros for no block
+   if (sidx == INVALID) return r;
    if constexpr (ST == ST_F32) {
       const float* p = static_cast<const float*>(pl.f) + (size_t)sidx * WID3 + o;
-      if (DIM == 0) {
-         const float4 q = *reinterpret_cast<const float4*>(p);
-         w[0] = q.x; w[1] = q.y; w[2] = q.z; w[3] = q.w;
-      } else {
-         w[0] = p[0]; w[1] = p[st]; w[2] = p[2 * st]; w[3] = p[3 * st];
-      }
+      if (Access<DIM, ST>::ROW) r.v = *reinterpret_cast<const float4*>(p);
+      else r.v = make_float4(p[0], p[WID2], p[2 * WID2], p[3 * WID2]);
    } else {
-      const uint16_t* p = static_cast<const uint16_t*>(pl.f) + (size_t)sidx * WID3 + o;
-      const float sc = pl.scale[sidx];
-      uint32_t u[4];
-      if (DIM == 0) {
-         const uint2 q = *reinterpret_cast<const uint2*>(p);
-         u[0] = q.x & 0xFFFFu; u[1] = q.x >> 16; u[2] = q.y & 0xFFFFu; u[3] = q.y >> 16;
-      } else {
-         u[0] = p[0]; u[1] = p[st]; u[2] = p[2 * st]; u[3] = p[3 * st];
-      }
-#pragma unroll
-      for (int e = 0; e < 4; ++e) w[e] = sc * Codec<ST>::dec(u[e]);
+      r.q = *reinterpret_cast<const uint2*>(static_cast<const uint16_t*>(pl.f) + (size_t)sidx * WID3 + o);
+      r.sc = pl.scale[sidx];
+   }
+   return r;
+}
+template <int DIM, int ST>
+__device__ inline void share_to_pencil(const Share<ST>& r, float (&w)[4]) {
+   if constexpr (ST == ST_F32) {
+      w[0] = r.v.x; w[1] = r.v.y; w[2] = r.v.z; w[3] = r.v.w;
+      if (DIM != 0 && Access<DIM, ST>::ROW) quad_transpose(w);
+   } else {
+      const uint2 q = (DIM != 0) ? quad_transpose16(r.q) : r.q;
+      w[0] = r.sc * Pack2<ST>::lo(q.x);
+      w[1] = r.sc * Pack2<ST>::hi(q.x);
+      w[2] = r.sc * Pack2<ST>::lo(q.y);
+      w[3] = r.sc * Pack2<ST>::hi(q.y);
    }
 }
 
+// An FP32 share, as read
+template <int DIM>
+__device__ inline void store_share(float* __restrict__ f, size_t slot, int o, const float4& v) {
+   float* p = f + slot * WID3 + o;
+   if (Access<DIM, ST_F32>::ROW) {
+      *reinterpret_cast<float4*>(p) = v;
+   } else {
+      p[0] = v.x; p[WID2] = v.y; p[2 * WID2] = v.z; p[3 * WID2] = v.w;
+   }
+}
 template <int DIM>
 __device__ inline void store_pencil(float* __restrict__ f, size_t slot, int o, const float (&w)[4]) {
-   float* p = f + slot * WID3 + o;
-   if (DIM == 0) {
-      *reinterpret_cast<float4*>(p) = make_float4(w[0], w[1], w[2], w[3]);
-   } else {
-      constexpr int st = Pencil<DIM>::st;
-      p[0] = w[0]; p[st] = w[1]; p[2 * st] = w[2]; p[3 * st] = w[3];
-   }
+   float x[4] = {w[0], w[1], w[2], w[3]};
+   if (DIM != 0 && Access<DIM, ST_F32>::ROW) quad_transpose(x);
+   store_share<DIM>(f, slot, o, make_float4(x[0], x[1], x[2], x[3]));
 }
 
 __device__ inline void set_content_flag(uint8_t* content, size_t slot, bool has, int setlane0, int l16) {
@@ -862,7 +939,7 @@ template <int DIM, int ST, bool STATS = true>
 __device__ inline void zero_block(const RemapArgs& a, int l16, int setlane0, int o, size_t slot, float thc) {
    const float q[4] = {0.0f, 0.0f, 0.0f, 0.0f};
    if constexpr (ST == ST_F32) {
-      store_pencil<DIM>(static_cast<float*>(a.out.f), slot, o, q);
+      store_share<DIM>(static_cast<float*>(a.out.f), slot, o, make_float4(0.0f, 0.0f, 0.0f, 0.0f));
    } else {
       uint16_t* p = static_cast<uint16_t*>(a.out.f) + slot * WID3 + 4 * l16;
       *reinterpret_cast<uint2*>(p) = make_uint2(0u, 0u);
@@ -877,11 +954,14 @@ template <int DIM, int ST, bool STATS = true>
 __device__ inline void copy_block(const RemapArgs& a, int l16, int setlane0, int o, uint32_t sidx, size_t slot,
                                   float thc) {
    if constexpr (ST == ST_F32) {
-      float w[4];
-      load_pencil<DIM, ST>(a.in, sidx, o, w);
-      store_pencil<DIM>(static_cast<float*>(a.out.f), slot, o, w);
+      const Share<ST> r = load_share<DIM, ST>(a.in, sidx, o);
+      store_share<DIM>(static_cast<float*>(a.out.f), slot, o, r.v);
+      float w[4] = {r.v.x, r.v.y, r.v.z, r.v.w};
       set_content(a.content_out, slot, w, thc, setlane0, l16);
-      if (STATS && a.blk_stats) put_pencil_stats<DIM>(a.blk_stats, slot, l16, w);
+      if (STATS && a.blk_stats) {
+         share_to_pencil<DIM, ST>(r, w);
+         put_pencil_stats<DIM>(a.blk_stats, slot, l16, w);
+      }
    } else {
       uint2 raw = make_uint2(0u, 0u);
       float sc = 0.0f;
@@ -908,7 +988,7 @@ __device__ __forceinline__ void remap_units(const RemapArgs& a, double i_dv, flo
    const int l16 = tid & 15;
    const int ip = l16 & 3, jp = l16 >> 2;
    const int setlane0 = (tid & 63) & ~15;
-   const int o = (DIM == 0) ? (ip * WID2 + jp * WID) : (DIM == 1) ? (jp * WID2 + ip) : (jp * WID + ip);
+   const int o = Access<DIM, ST>::offset(ip, jp);
    const uint32_t gstride = blocks * (WGS / 16);
    for (uint32_t gi = first + block * (WGS / 16) + (tid >> 4); gi < total; gi += gstride) {
       const uint4 sr = a.units[2 * (size_t)gi], first_col = a.units[2 * (size_t)gi + 1];
@@ -963,24 +1043,26 @@ __device__ __forceinline__ void remap_units(const RemapArgs& a, double i_dv, flo
                if ((double)x < minV) { minV = (double)x; minL = L; }
             }
          }
-         float w0[4] = {0.0f, 0.0f, 0.0f, 0.0f}, w1[4], w2[4];
+         float w0[4] = {0.0f, 0.0f, 0.0f, 0.0f}, w1[4];
          // source indices are read one block ahead of the block data they locate, so that no
          // block waits for an index load and then for the data load behind it
          uint32_t s_next = (len > 2) ? srcs[2] : INVALID;   // index of block b + 2
-         load_pencil<DIM, ST>(a.in, srcs[0], o, w1);
-         load_pencil<DIM, ST>(a.in, (len > 1) ? srcs[1] : INVALID, o, w2);
+         const Share<ST> first = load_share<DIM, ST>(a.in, srcs[0], o);
+         Share<ST> next = load_share<DIM, ST>(a.in, (len > 1) ? srcs[1] : INVALID, o);   // block b + 1
+         share_to_pencil<DIM, ST>(first, w1);
          int next_flush = fk;
          int next_open = (carry_open >= 0) ? carry_open : fk;
          const int lo_gk = WID * fk, hi_gk = WID * lk + WID - 1;
          Recon<METHOD> rc;
          {
-            const float v0[12] = {w0[0], w0[1], w0[2], w0[3], w1[0], w1[1], w1[2], w1[3], w2[0], w2[1], w2[2], w2[3]};
+            const float v0[8] = {w0[0], w0[1], w0[2], w0[3], w1[0], w1[1], w1[2], w1[3]};
             rc.start(v0 + 4, scale);
          }
          for (int b = 0; b < len; ++b) {
             const uint32_t s_after = (b + 3 < len) ? srcs[b + 3] : INVALID;
-            float w3[4];
-            load_pencil<DIM, ST>(a.in, s_next, o, w3);   // zeros past the column's end
+            float w2[4];
+            share_to_pencil<DIM, ST>(next, w2);
+            next = load_share<DIM, ST>(a.in, s_next, o);   // zeros past the column's end
             s_next = s_after;
             const float v[12] = {w0[0], w0[1], w0[2], w0[3], w1[0], w1[1], w1[2], w1[3], w2[0], w2[1], w2[2], w2[3]};
 #pragma unroll
@@ -1029,7 +1111,6 @@ __device__ __forceinline__ void remap_units(const RemapArgs& a, double i_dv, flo
             for (int e = 0; e < 4; ++e) {
                w0[e] = w1[e];
                w1[e] = w2[e];
-               w2[e] = w3[e];
             }
          }
          while (next_flush < next_open && next_flush < nfk) {
@@ -1108,7 +1189,7 @@ __global__ __launch_bounds__(WGS, 5) void k_remap_lean(RemapArgs a) {
    const int l16 = tid & 15;
    const int ip = l16 & 3, jp = l16 >> 2;
    const int setlane0 = (tid & 63) & ~15;
-   const int o = (DIM == 0) ? (ip * WID2 + jp * WID) : (DIM == 1) ? (jp * WID2 + ip) : (jp * WID + ip);
+   const int o = Access<DIM, ST>::offset(ip, jp);
    // the units before EXACT_BIN's; k_remap takes the EXACT_BIN and WIDE_BIN units
    const uint32_t total = a.unit_base[a.ncells] - a.len_hist[EXACT_BIN] - a.len_hist[WIDE_BIN];
    const uint32_t gstride = gridDim.x * (WGS / 16);
@@ -1165,17 +1246,18 @@ __global__ __launch_bounds__(WGS, 5) void k_remap_lean(RemapArgs a) {
          auto emit = [&](int gt, float m) { ring[min(gt, hi + 1) & (LEAN_RING - 1)][tid] = m; };
          Flux<NC> fx;
          fx.begin((a.vmin_d + (double)(WID * ks) * a.dv_d - imin) * rdk, r);
-         float w0[4] = {0.0f, 0.0f, 0.0f, 0.0f}, w1[4], w2[4];
+         float w0[4] = {0.0f, 0.0f, 0.0f, 0.0f}, w1[4];
          // source indices are read one block ahead of the block data they locate, so that no
          // block waits for an index load and then for the data load behind it
          uint32_t s_next = (len > 2) ? srcs[2] : INVALID;   // index of block b + 2
-         load_pencil<DIM, ST>(a.in, srcs[0], o, w1);
-         load_pencil<DIM, ST>(a.in, (len > 1) ? srcs[1] : INVALID, o, w2);
+         const Share<ST> first = load_share<DIM, ST>(a.in, srcs[0], o);
+         Share<ST> next = load_share<DIM, ST>(a.in, (len > 1) ? srcs[1] : INVALID, o);   // block b + 1
+         share_to_pencil<DIM, ST>(first, w1);
          int next_flush = fk;
          int next_open = (carry_open >= 0) ? carry_open : fk;
          R rc;
          {
-            const float v0[12] = {w0[0], w0[1], w0[2], w0[3], w1[0], w1[1], w1[2], w1[3], w2[0], w2[1], w2[2], w2[3]};
+            const float v0[8] = {w0[0], w0[1], w0[2], w0[3], w1[0], w1[1], w1[2], w1[3]};
             rc.start(v0 + 4);
          }
          for (int b = 0; b < len; ++b) {
@@ -1200,6 +1282,8 @@ __global__ __launch_bounds__(WGS, 5) void k_remap_lean(RemapArgs a) {
             // in number; only then are block b + 2 read and the finished target blocks (all below
             // flushLim, which no deposit of this block reaches) stored, so that cells 1..3 cover
             // their latency.  The scheduling barriers keep that order.
+            float w2[4];
+            share_to_pencil<DIM, ST>(next, w2);
             const float v[12] = {w0[0], w0[1], w0[2], w0[3], w1[0], w1[1], w1[2], w1[3], w2[0], w2[1], w2[2], w2[3]};
             {
                float cf[NC];
@@ -1208,8 +1292,7 @@ __global__ __launch_bounds__(WGS, 5) void k_remap_lean(RemapArgs a) {
             }
             __builtin_amdgcn_sched_barrier(0);
             const uint32_t s_after = (b + 3 < len) ? srcs[b + 3] : INVALID;
-            float w3[4];
-            load_pencil<DIM, ST>(a.in, s_next, o, w3);   // zeros past the column's end
+            next = load_share<DIM, ST>(a.in, s_next, o);   // zeros past the column's end
             s_next = s_after;
             while (next_flush < next_open && next_flush < nfk && WID * next_flush + WID - 1 < flushLim) {
                flush_block<DIM, ST, LEAN_RING, WGS, true, STATS>(a, ring, tid, l16, setlane0, o, next_flush, slotb + (next_flush - fk), thc);
@@ -1226,7 +1309,6 @@ __global__ __launch_bounds__(WGS, 5) void k_remap_lean(RemapArgs a) {
             for (int e = 0; e < 4; ++e) {
                w0[e] = w1[e];
                w1[e] = w2[e];
-               w2[e] = w3[e];
             }
          }
          fx.end(emit);
