@@ -129,8 +129,14 @@ struct TransformIn {
    double dt;
 };
 
-VACC_HD Affine acceleration_transform(const TransformIn& in, double mass, double charge,
-                                      double hall_min_rhoq, int ohm_gradpe) {
+// What every substep of the transform uses: the substeps' count and length, the rotation of one and
+// the velocity of the Hall term.
+struct AccelStep {
+   unsigned int substeps;
+   double sdt, R[9], h[3], qm;
+};
+VACC_HD AccelStep acceleration_step(const TransformIn& in, double mass, double charge, double hall_min_rhoq) {
+   AccelStep o;
    const double n2 = in.B[0] * in.B[0] + in.B[1] * in.B[1] + in.B[2] * in.B[2];
    const double nrm = sqrt(n2);
    double u[3] = {in.B[0], in.B[1], in.B[2]};
@@ -150,22 +156,28 @@ VACC_HD Affine acceleration_transform(const TransformIn& in, double mass, double
    const double rhoq = in.rhoq + eps;
    const double hall_rhoq = (rhoq <= hall_min_rhoq) ? hall_min_rhoq : rhoq;
    const double hall = 1.0 / (MU_0 * hall_rhoq);
-   unsigned int substeps = (unsigned int)(fabs(in.dt) / fabs(gyro_period * (0.1 / 360.0)));
-   if (substeps < 1) substeps = 1;
-   const double rad = -(2.0 * PI * in.dt / gyro_period) / substeps;
-   const double sdt = in.dt / substeps;
-   double R[9];
-   axis_rotation(u, rad, R);
-   const double hx = hall * (in.dB[5] - in.dB[3]);
-   const double hy = hall * (in.dB[1] - in.dB[4]);
-   const double hz = hall * (in.dB[2] - in.dB[0]);
+   o.substeps = (unsigned int)(fabs(in.dt) / fabs(gyro_period * (0.1 / 360.0)));
+   if (o.substeps < 1) o.substeps = 1;
+   const double rad = -(2.0 * PI * in.dt / gyro_period) / o.substeps;
+   o.sdt = in.dt / o.substeps;
+   axis_rotation(u, rad, o.R);
+   o.h[0] = hall * (in.dB[5] - in.dB[3]);
+   o.h[1] = hall * (in.dB[1] - in.dB[4]);
+   o.h[2] = hall * (in.dB[2] - in.dB[0]);
+   o.qm = fabs(charge) / mass;
+   return o;
+}
+
+// The host's form; k_transform does the same operations with a lane per element of T.
+VACC_HD Affine acceleration_transform(const TransformIn& in, double mass, double charge,
+                                      double hall_min_rhoq, int ohm_gradpe) {
+   const AccelStep st = acceleration_step(in, mass, charge, hall_min_rhoq);
+   const double* R = st.R;
    Affine T = {{1, 0, 0, 0, 0, 1, 0, 0, 0, 0, 1, 0}};
-   for (unsigned int s = 0; s < substeps; ++s) {
+   for (unsigned int s = 0; s < st.substeps; ++s) {
       double p[3];
       affine_point(T, in.V, p);
-      p[0] -= hx;
-      p[1] -= hy;
-      p[2] -= hz;
+      for (int r = 0; r < 3; ++r) p[r] -= st.h[r];
       for (int r = 0; r < 3; ++r) T.m[4 * r + 3] = -p[r] + T.m[4 * r + 3];
       Affine N;
       for (int r = 0; r < 3; ++r)
@@ -173,10 +185,8 @@ VACC_HD Affine acceleration_transform(const TransformIn& in, double mass, double
             N.m[4 * r + q] = (R[3 * r] * T.m[q] + R[3 * r + 1] * T.m[4 + q]) + R[3 * r + 2] * T.m[8 + q];
       T = N;
       for (int r = 0; r < 3; ++r) T.m[4 * r + 3] = p[r] + T.m[4 * r + 3];
-      if (ohm_gradpe > 0) {
-         const double qm = fabs(charge) / mass;
-         for (int r = 0; r < 3; ++r) T.m[4 * r + 3] = (qm * in.EgradPe[r]) * sdt + T.m[4 * r + 3];
-      }
+      if (ohm_gradpe > 0)
+         for (int r = 0; r < 3; ++r) T.m[4 * r + 3] = (st.qm * in.EgradPe[r]) * st.sdt + T.m[4 * r + 3];
    }
    return T;
 }

@@ -1986,33 +1986,77 @@ __global__ __launch_bounds__(WG) void k_moments_sums(MomentArgs a, uint32_t spli
    put_cell_sums<4>(red, a.part, a.out, a.host, split, a.cell[0] * a.cell[1] * a.cell[2]);
 }
 
-__global__ void k_transform(MeshInfo m, const TransformIn* fields, const double* dt_override, const double* moments,
-                            int use_moments, double mass, double charge, double hall_min_rhoq, int ohm_gradpe,
-                            int map_order, double* isect_out, uint32_t ncells) {
-   const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
-   if (c >= ncells) return;
-   TransformIn in = fields[c];
-   if (dt_override) in.dt = dt_override[c];
-   if (use_moments == 1) {
-      // one population: VX_V = (nVx * m) / (n * m), RHOQ_V = n * q (arch_moments.cpp:419-440)
-      const double* mo = moments + 4 * (size_t)c;
-      const double rhom = mo[0] * mass;
-      if (rhom != 0.0) {
-         in.V[0] = (mo[1] * mass) / rhom;
-         in.V[1] = (mo[2] * mass) / rhom;
-         in.V[2] = (mo[3] * mass) / rhom;
+// DPP move of a double within the row; lanes without a source get 0
+template <int CTRL>
+__device__ inline double dpp_f64(double x) {
+   const uint2 u = __builtin_bit_cast(uint2, x);
+   const uint2 v = make_uint2((uint32_t)__builtin_amdgcn_update_dpp(0, (int)u.x, CTRL, 0xF, 0xF, true),
+                              (uint32_t)__builtin_amdgcn_update_dpp(0, (int)u.y, CTRL, 0xF, 0xF, true));
+   return __builtin_bit_cast(double, v);
+}
+
+// FP64 transform and intersections.  Bound by the chain of substeps (0.1 degrees each, 100 for a
+// rotation of 10 degrees): one lane per cell did the 87 FP64 operations of a substep in series.  Here
+// a row of 16 lanes holds a cell, lane 4q + r the element (r, q) of T (r = 3 idle), so a substep is
+// 13 dependent operations, in acceleration_transform's order and with its results.  Then the three
+// passes' intersections of the workgroup's cells are taken by one wave each.  18 -> 10 us for 16
+// cells, 26 -> 15 us for 300.
+constexpr int TR_CELLS = WG / 16;
+__global__ __launch_bounds__(WG) void k_transform(MeshInfo m, const TransformIn* fields, const double* dt_override,
+                                                  const double* moments, int use_moments, double mass, double charge,
+                                                  double hall_min_rhoq, int ohm_gradpe, int map_order, double* isect_out,
+                                                  uint32_t ncells) {
+   __shared__ Affine fwd[TR_CELLS];
+   const uint32_t c0 = blockIdx.x * TR_CELLS, c = c0 + (threadIdx.x >> 4);
+   if (c < ncells) {
+      TransformIn in = fields[c];
+      if (dt_override) in.dt = dt_override[c];
+      if (use_moments == 1) {
+         // one population: VX_V = (nVx * m) / (n * m), RHOQ_V = n * q (arch_moments.cpp:419-440)
+         const double* mo = moments + 4 * (size_t)c;
+         const double rhom = mo[0] * mass;
+         if (rhom != 0.0) {
+            in.V[0] = (mo[1] * mass) / rhom;
+            in.V[1] = (mo[2] * mass) / rhom;
+            in.V[2] = (mo[3] * mass) / rhom;
+         }
+         in.rhoq = mo[0] * charge;
+      } else if (use_moments == 2) {
+         // plasma pivot of several populations (k_plasma): {VX_V, VY_V, VZ_V, RHOQ_V}
+         const double* pv = moments + 4 * (size_t)c;
+         in.V[0] = pv[0];
+         in.V[1] = pv[1];
+         in.V[2] = pv[2];
+         in.rhoq = pv[3];
       }
-      in.rhoq = mo[0] * charge;
-   } else if (use_moments == 2) {
-      // plasma pivot of several populations (k_plasma): {VX_V, VY_V, VZ_V, RHOQ_V}
-      const double* pv = moments + 4 * (size_t)c;
-      in.V[0] = pv[0];
-      in.V[1] = pv[1];
-      in.V[2] = pv[2];
-      in.rhoq = pv[3];
+      const AccelStep st = acceleration_step(in, mass, charge, hall_min_rhoq);
+      const int r = threadIdx.x & 3, q = (threadIdx.x >> 2) & 3;
+      const bool trans = (q == 3);
+      auto at = [](int i, double x, double y, double z) { return i == 0 ? x : i == 1 ? y : i == 2 ? z : 0.0; };
+      const double R0 = at(r, st.R[0], st.R[3], st.R[6]), R1 = at(r, st.R[1], st.R[4], st.R[7]),
+                   R2 = at(r, st.R[2], st.R[5], st.R[8]);
+      const double V = at(q, in.V[0], in.V[1], in.V[2]), h = at(r, st.h[0], st.h[1], st.h[2]);
+      const double E = (st.qm * at(r, in.EgradPe[0], in.EgradPe[1], in.EgradPe[2])) * st.sdt;
+      double T = (r == q) ? 1.0 : 0.0;
+      for (unsigned int s = 0; s < st.substeps; ++s) {
+         // in the lanes of the translation (q = 3): p = T V + t - h from the products of columns 0..2
+         const double pr = T * V;
+         double p = ((dpp_f64<0x11C>(pr) + dpp_f64<0x118>(pr)) + dpp_f64<0x114>(pr)) + T;   // row_shr 12, 8, 4
+         p -= h;
+         const double x = trans ? -p + T : T;
+         const double n = (R0 * dpp_f64<0x00>(x) + R1 * dpp_f64<0x55>(x)) + R2 * dpp_f64<0xAA>(x);   // quad broadcasts
+         T = trans ? p + n : n;
+         if (ohm_gradpe > 0 && trans) T = E + T;
+      }
+      if (r < 3) fwd[threadIdx.x >> 4].m[4 * r + q] = T;
    }
-   const Affine fwd = acceleration_transform(in, mass, charge, hall_min_rhoq, ohm_gradpe);
-   cell_intersections(m, fwd, map_order, isect_out + 12 * (size_t)c);
+   __syncthreads();
+   const uint32_t l = threadIdx.x & 63;
+   const int pass = (int)(threadIdx.x >> 6);
+   if (pass < 3 && l < TR_CELLS && c0 + l < ncells) {
+      const int d = pass_dim(map_order, pass);
+      pass_intersections(m, affine_inverse(fwd[l]), pass, d, isect_out + 12 * (size_t)(c0 + l) + 4 * d);
+   }
 }
 
 // Plasma moments of several populations (arch_moments.cpp:406-440): RHOM_V = sum n*m,
@@ -2305,7 +2349,7 @@ void launch_transform(const MeshInfo& m, const TransformIn* fields, const double
                       int use_moments, double mass, double charge, double hall_min_rhoq, int ohm_gradpe, int map_order,
                       double* isect_out, uint32_t ncells, hipStream_t s) {
    if (ncells == 0) return;
-   hipLaunchKernelGGL(k_transform, dim3((ncells + 127) / 128), dim3(128), 0, s, m, fields, dt_override, moments,
+   hipLaunchKernelGGL(k_transform, dim3((ncells + TR_CELLS - 1) / TR_CELLS), dim3(WG), 0, s, m, fields, dt_override, moments,
                       use_moments, mass, charge, hall_min_rhoq, ohm_gradpe, map_order, isect_out, ncells);
 }
 
