@@ -13,10 +13,10 @@
 //                  of long pencils in the 16-bit forms, and cells that are not written
 //                  (copied).
 //
-// In both writing kernels lane l holds the block's velocity cell of transposed index
-// l = i + 4j + 16k, k along the translation dimension (cpu_trans_map_amr.cpp:224-285), so
-// the reference's 8-lane groups of check_skip_remapping (VECL = 8, planes of 16 cells) are
-// aligned groups of 8 lanes; values are accumulated in FP32 in the reference's order.
+// In both writing kernels lane e holds the block's velocity cell of in-block index e.  The reference
+// transposes a block to l = i + 4j + 16k, k along the translation dimension
+// (cpu_trans_map_amr.cpp:224-285); the 8-lane groups of its check_skip_remapping (VECL = 8, planes of
+// 16 cells) are lane masks here (LaneGroup).  Values are accumulated in FP32 in its order.
 //
 // k_trans: for each of its cells the host lists every contribution the cell receives (source
 // position of a pencil, kind, widths, ratio) in the reference's accumulation order, and the
@@ -115,21 +115,35 @@ __device__ inline float pool_val(const Pool& p, uint32_t idx, int e) {
    }
 }
 
-// Writes block b: lane l holds the value of in-block index ab.  The 16-bit forms encode the
-// block with the canonical lane order (lane e = in-block index e), so the values are first
-// moved there: lane e reads the lane whose transposed index maps to e.
+// Lane layout of the translation kernels: lane e holds the block's value of in-block index e whatever the
+// dimension, so that blocks are read, written and encoded contiguously.  In the reference's order, with the
+// translated axis moved last, the x walk read pieces 64 bytes apart and the 16-bit forms moved every
+// written block through the LDS crossbar: calls over 3.6 million blocks 3.1 -> 3.0 ms in 16 bits, the x
+// walk over 7.3 million 3.07 -> 2.98 ms in FP32 (y and z unchanged within 1 %).  The
+// reference's order only shows in its groups of 8 lanes: those of the lane are (lanes >> shift) & base.
+struct LaneGroup {
+   unsigned long long base;
+   int shift;
+   __device__ inline bool any(unsigned long long lanes) const { return ((lanes >> shift) & base) != 0ull; }
+};
+__device__ inline LaneGroup lane_group(int dim, int e) {
+   // transposed index t = ti + 4 tj + 16 tk of e = 16 ti + 4 tj + tk (dim 0), ti + 16 tj + 4 tk (1), t (2);
+   // a group shares tk and the upper bit of tj
+   if (dim == 0) return {0x0011001100110011ull, e & 11};
+   if (dim == 1) return {0x000F000Full, e & 44};
+   return {0xFFull, e & 56};
+}
+// coordinate of in-block index e along dim
+__device__ inline int lane_coord(int dim, int e) { return (dim == 0) ? e & 3 : (dim == 1) ? (e >> 2) & 3 : e >> 4; }
+
+// Writes block b: lane e holds the value of in-block index e.
 template <int ST>
-__device__ inline void store_block(const Pool& p, uint32_t b, float x, int ab, int dim, int lane) {
+__device__ inline void store_block(const Pool& p, uint32_t b, float x, int e) {
    if constexpr (ST == ST_F32) {
-      static_cast<float*>(p.f)[(size_t)b * 64 + ab] = x;
+      static_cast<float*>(p.f)[(size_t)b * 64 + e] = x;
    } else {
-      const int e = lane;
-      const int from = (dim == 0) ? (e >> 4) + 4 * ((e >> 2) & 3) + 16 * (e & 3)
-                       : (dim == 1) ? (e & 3) + 4 * (e >> 4) + 16 * ((e >> 2) & 3)
-                                    : e;
-      const float xe = __shfl(x, from, 64);
       uint32_t code;
-      const float sc = encode_wave64<ST>(xe, code);
+      const float sc = encode_wave64<ST>(x, code);
       static_cast<uint16_t*>(p.f)[(size_t)b * 64 + e] = (uint16_t)code;
       if (e == 0) p.scale[b] = sc;
    }
@@ -172,9 +186,8 @@ __global__ __launch_bounds__(TWG) void k_trans(TransArgs a) {
    static_assert(sizeof(TransFace) == 64 && sizeof(TransEntry) == 160 && sizeof(TransCell) == 64, "layouts");
    const int lane = threadIdx.x & 63;
    const int wv = threadIdx.x >> 6;
-   const int ti = lane & 3, tj = (lane >> 2) & 3, tk = lane >> 4;
-   // vcell_transpose: in-block index of transposed cell (ti, tj, tk)
-   const int ab = (a.dim == 0) ? ti * 16 + tj * 4 + tk : (a.dim == 1) ? ti + tj * 16 + tk * 4 : lane;
+   const LaneGroup group = lane_group(a.dim, lane);
+   const int tk = lane_coord(a.dim, lane);
    // work item = (cell of the rest list, one of TSPLIT workgroups); its waves take the
    // cell's chunks of TCHUNK blocks in turn
    const uint32_t items = a.nrest * (uint32_t)TSPLIT;
@@ -251,7 +264,7 @@ __global__ __launch_bounds__(TWG) void k_trans(TransArgs a) {
                   const unsigned long long hit = __ballot(s_gid[wv][j][lane] == g);
                   if (hit) {
                      const uint32_t idx = s_src[wv][j][__builtin_ctzll(hit)];
-                     if (idx != VACC_INVALID_ID) v[j] = pool_val<ST>(a.in, idx, ab);
+                     if (idx != VACC_INVALID_ID) v[j] = pool_val<ST>(a.in, idx, lane);
                   }
                }
             }
@@ -272,7 +285,7 @@ __global__ __launch_bounds__(TWG) void k_trans(TransArgs a) {
                // when none of its stencil values is positive
                const bool any = (u[0] > 0.0f) || (u[1] > 0.0f) || (u[2] > 0.0f) || (u[3] > 0.0f) || (u[4] > 0.0f);
                const unsigned long long mask = __ballot(any);
-               if (((mask >> (lane & 56)) & 0xFFull) == 0ull) continue;
+               if (!group.any(mask)) continue;
                const float zt = vdt / E.dz_i;
                const bool pos = zt > 0.0f;
                const bool take = (E.kind == 0) ? pos : !pos;
@@ -292,7 +305,7 @@ __global__ __launch_bounds__(TWG) void k_trans(TransArgs a) {
                }
                acc = acc + contrib;
             }
-            store_block<ST>(a.out, b, acc, ab, a.dim, lane);
+            store_block<ST>(a.out, b, acc, lane);
          }
       }
    }
@@ -419,8 +432,8 @@ __global__ __launch_bounds__(TWG) __attribute__((amdgpu_waves_per_eu(ST == ST_F3
    const uint32_t nwaves = (gridDim.x * (uint32_t)TWG) >> 6;
    const uint32_t nunits = w.nseg * w.wps;
    const float lsc = limiter_scale(a.thr, a.scale), lus = limiter_unscale(a.thr);
-   const int ti = lane & 3, tj = (lane >> 2) & 3, tk = lane >> 4;
-   const int ab = (a.dim == 0) ? ti * 16 + tj * 4 + tk : (a.dim == 1) ? ti + tj * 16 + tk * 4 : lane;
+   const LaneGroup group = lane_group(a.dim, lane);
+   const int tk = lane_coord(a.dim, lane);
    for (uint32_t u = wave; u < nunits; u += nwaves) {
       const uint32_t s = u / w.wps;
       const uint32_t glo = w.bounds[u + s], ghi = w.bounds[u + s + 1];   // row s has wps + 1 bounds
@@ -499,7 +512,7 @@ __global__ __launch_bounds__(TWG) __attribute__((amdgpu_waves_per_eu(ST == ST_F3
          const unsigned long long vmask = __ballot(pidx != VACC_INVALID_ID);
          const uint32_t vidx = (pidx != VACC_INVALID_ID) ? pidx : 0u;
          auto val = [&](int q) -> float {
-            const float x = pool_val<ST>(a.in, (uint32_t)__builtin_amdgcn_readlane((int)vidx, q & 63), ab);
+            const float x = pool_val<ST>(a.in, (uint32_t)__builtin_amdgcn_readlane((int)vidx, q & 63), lane);
             return (vmask & (1ull << (q & 63))) ? x : 0.0f;
          };
          float c1 = 0.0f, c2 = 0.0f;   // carry registers
@@ -510,14 +523,14 @@ __global__ __launch_bounds__(TWG) __attribute__((amdgpu_waves_per_eu(ST == ST_F3
             if constexpr (ST == ST_F32) {
                // the sum an earlier launch level stored into this block
                if (((inits & tmask) >> q) & 1ull)
-                  return static_cast<const float*>(a.out.f)[(size_t)__builtin_amdgcn_readlane((int)ob, q) * 64 + ab];
+                  return static_cast<const float*>(a.out.f)[(size_t)__builtin_amdgcn_readlane((int)ob, q) * 64 + lane];
             }
             return ((init1 >> q) & 1ull) ? c1 : ((init2 >> q) & 1ull) ? c2 : 0.0f;
          };
          // end of window position q's sum x: into a carry register or the block
          const unsigned long long plain = tmask & ~(save1 | save2);
          auto retire = [&](int q, float x) {
-            if (plain & (1ull << q)) store_block<ST>(a.out, (uint32_t)__builtin_amdgcn_readlane((int)ob, q), x, ab, a.dim, lane);
+            if (plain & (1ull << q)) store_block<ST>(a.out, (uint32_t)__builtin_amdgcn_readlane((int)ob, q), x, lane);
             else if (save1 & tmask & (1ull << q)) c1 = x;
             else if (save2 & tmask & (1ull << q)) c2 = x;
          };
@@ -584,7 +597,7 @@ __global__ __launch_bounds__(TWG) __attribute__((amdgpu_waves_per_eu(ST == ST_F3
                         am = am + (!pos ? x : 0.0f) * lanef(rl, j - 1);
                      }
                   } else {
-                     const bool act = ((amask >> (lane & 56)) & 0xFFull) != 0ull;
+                     const bool act = group.any(amask);
                      if ((tm & 2ull) && act) a0 = a0 + (u2 - ng) * lanef(rl, j);
                      if ((tm & 4ull) && __ballot(pos && act)) {
                         const float x = (ng * dzj) / lanef(dzl, j + 1);
