@@ -1176,9 +1176,11 @@ __device__ inline int row_min16(int x) {
 // (their codec alone would need 111 to 116 VGPRs).  Five waves issue about 7 % more per pass
 // than four on the PQM workloads for FP32 and make the 16-bit forms' step 3 % faster.
 // Bound by VALU issue and latency: with limiters and face tests as medians of three, halved
-// derivatives and the short quartic (vacc_lean.h), and targets placed by a minimum in place of
-// a range test, a PQM cell without a second boundary takes 65 VALU instructions instead of 87;
-// x, y, z passes over 26 million blocks 4.88, 5.31, 5.05 -> 4.32, 5.09, 4.60 ms (PQM, FP32).
+// derivatives (vacc_lean.h) and targets placed by a minimum in place of a range test, a PQM cell
+// without a second boundary takes 68 VALU instructions instead of 87; x, y, z passes over 26 million
+// blocks 4.88, 5.31, 5.05 -> 4.3, 4.7, 4.6 ms with the y blocks read by rows (PQM, FP32).  The face
+// estimates on the matrix cores (v_mfma_f32_4x4x1, 15 VALU instructions a cell fewer) made the step
+// 2 to 6 % slower: the operands' registers went to scratch.
 template <int DIM, int METHOD, int ST, int WGS, bool STATS>
 __global__ __launch_bounds__(WGS, 5) void k_remap_lean(RemapArgs a) {
    using R = ReconLean<METHOD>;

@@ -152,13 +152,13 @@ struct ReconLean<VACC_PQM> {
       hb = 0.5f * b;
       out = lean_outside(fv - v[0], -b);
    }
-   // c[1..4] from the face deviations and half derivatives gl, gr (d = 2 g), with e = ul + ur,
-   // p = gr - gl and q = ul + gl: eight operations
+   // c[2..4] from the face deviations and half derivatives gl, gr (d = 2 g): ten operations.  Sharing
+   // e = ul + ur, gr - gl and ul + gl between the three takes eight, about 1 % of a step, but rounds
+   // otherwise, which 16-bit subcycles carry on to 3e-5 of the momentum.
    VACC_HD static void quartic(float ul, float ur, float gl, float gr, float& c2, float& c3, float& c4) {
-      const float e = ul + ur, p = gr - gl, q = ul + gl;
-      c2 = fmaf(-4.0f, e, fmaf(-2.0f, q, p));
-      c3 = fmaf(7.0f, e, fmaf(-2.0f, p, q));
-      c4 = fmaf(-3.0f, e, p);
+      c2 = fmaf(-6.0f, ul, fmaf(-4.0f, ur, fmaf(-3.0f, gl, gr)));
+      c3 = fmaf(8.0f, ul, fmaf(7.0f, ur, fmaf(3.0f, gl, -2.0f * gr)));
+      c4 = fmaf(-3.0f, ul + ur, gr - gl);
    }
    VACC_HD void coeffs(const float* v, float* c) {
       const float vk = v[0];
