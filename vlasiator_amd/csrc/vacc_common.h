@@ -61,7 +61,7 @@ VACC_HD void gid_xyz(uint32_t g, const GidSplit& s, uint32_t& x, uint32_t& y, ui
    x = r - y * s.nx.d;
 }
 
-// Median of three finite values.
+// Median of three values; with a NaN among them the host's and the device's results differ.
 VACC_HD float med3(float x, float y, float z) {
 #if defined(__HIP_DEVICE_COMPILE__)
    return __builtin_amdgcn_fmed3f(x, y, z);

@@ -60,11 +60,26 @@ VACC_HD float deriv_h7(const float* v) {
 // and larger of |a|, |b|, the inner slopes are lo and min(2 lo, hi): the smaller of a and b is
 // med3(a, b, 0) (0 for opposite signs), the limited slope med3(a, b, 2 smaller), and their
 // product, the outer test's, underflows to 0 whenever one of the inner products does.  Six
-// instructions in place of seventeen, the same bits for finite a and b.
+// instructions in place of seventeen, the same bits.  A NaN among a and b (the scaled values of a
+// cell with threshold 0 are infinite or NaN) takes the reference's expression: its comparisons
+// and products then choose 2b in both inner tests, or NaN if b is.  That costs a compare and a
+// branch not taken: 2048 cells' exact PQM step 10.85 -> 10.87 ms, 16 cells' PPM step 306 -> 313 us.
 VACC_HD float superbee_ab(float a, float b) {
    const float lo = med3(a, b, 0.0f);
    const float s = med3(a, b, lo + lo);
-   return (lo * s <= 0.0f) ? 0.0f : s;
+   float r = (lo * s <= 0.0f) ? 0.0f : s;
+   const bool nan = __builtin_isunordered(a, b);
+#if defined(__HIP_DEVICE_COMPILE__)
+   if (__builtin_expect(__builtin_amdgcn_ballot_w64(nan) != 0ull, 0))
+#endif
+   {
+      float d = b + b;
+#if defined(__HIP_DEVICE_COMPILE__)
+      asm volatile("" : "+v"(d));   // keeps the branch: the compiler would turn it into selects
+#endif
+      r = nan ? ((d * b <= 0.0f) ? 0.0f : d) : r;
+   }
+   return r;
 }
 
 // x / 3 with IEEE rounding from a multiply by RN(1/3) and one FMA residual correction
