@@ -50,6 +50,7 @@ struct vacc_ctx {
    size_t cap = 0;             // block capacity of lists, pools and pass scratch
    int lcur = 0, fcur = 0;
    uint64_t nblocks = 0;       // total blocks as of the last synchronisation point
+   bool overflow = false;      // a call found the pool too small: no list until the next load
    bool content_valid = false;
    bool moments_valid = false; // `moments` holds the moments of the current list
    // blk_stats holds the block sums of pool F[fcur] (written by the last remap pass of a
@@ -423,8 +424,15 @@ static int refresh_count(vacc_ctx* c) {
    return 0;
 }
 
+// After a capacity overflow the current list is unwritten (its offsets reach beyond the buffers):
+// calls that walk it are refused until cells are loaded again.
+static int check_lists(const vacc_ctx* c) {
+   return c->overflow ? set_err(VACC_E_STATE, "block pool capacity was exceeded: load the cells again") : 0;
+}
+
 // Keep head-room for the growth of one step (new target blocks and adjust halo blocks).
 static int reserve_for_step(vacc_ctx* c) {
+   if (const int rc = check_lists(c)) return rc;
    const size_t want = c->nblocks + c->nblocks / 2 + 64 * (size_t)c->ncells + 4096;
    if (want > c->cap) return ensure_blocks(c, want + want / 4);
    return 0;
@@ -451,6 +459,7 @@ static int enqueue_pass(vacc_ctx* c, int dim, int grid_mult, int wgs = 0, bool s
    ca.n_units = c->n_units;
    ca.n_targets = c->n_tgt;
    ca.status = c->status;
+   ca.flags = c->flags;
    ca.ncells = c->ncells;
    for (int d = 0; d < 3; ++d) ca.len[d] = c->mi.len[d];
    ca.gs = make_gid_split(c->mi.len);
@@ -573,11 +582,12 @@ static int do_relist(vacc_ctx* c, int add_width, bool want_loss, const SpatialIn
       c->content_valid = false;
    }
    if (add_width >= 0 && !c->content_valid) {
-      launch_content_cells(c->off[li], c->src[li], pool(c, c->fcur), c->minval, c->content, c->ncells, c->stream);
+      launch_content_cells(c->off[li], c->src[li], pool(c, c->fcur), c->minval, c->content, c->flags, c->ncells,
+                           c->stream);
       c->content_valid = true;
    }
    const bool conserve = add_width >= 0 && c->sp.sparse_conserve_mass;
-   if (conserve) launch_cell_sums(c->off[li], c->src[li], pool(c, c->fcur), c->csum_pre, c->ncells, c->stream);
+   if (conserve) launch_cell_sums(c->off[li], c->src[li], pool(c, c->fcur), c->csum_pre, c->flags, c->ncells, c->stream);
    AdjustArgs aa{};
    aa.cell_off = c->off[li];
    aa.gid = c->gid[li];
@@ -630,8 +640,9 @@ static int do_relist(vacc_ctx* c, int add_width, bool want_loss, const SpatialIn
    aa.src_out = c->src[lo];
    launch_adjust(aa, true, c->stream);
    if (conserve) {   // block_adjust_cpu.cpp:96-113
-      launch_cell_sums(c->off[lo], c->src[lo], pool(c, c->fcur), c->csum_post, c->ncells, c->stream);
-      launch_cell_scale(c->off[lo], c->src[lo], pool(c, c->fcur), c->csum_pre, c->csum_post, c->ncells, c->stream);
+      launch_cell_sums(c->off[lo], c->src[lo], pool(c, c->fcur), c->csum_post, c->flags, c->ncells, c->stream);
+      launch_cell_scale(c->off[lo], c->src[lo], pool(c, c->fcur), c->csum_pre, c->csum_post, c->flags, c->ncells,
+                        c->stream);
       c->stats_valid = false;   // f was rescaled
    }
    HIPCHK(hipGetLastError());
@@ -666,8 +677,10 @@ static int finish_enqueue(vacc_ctx* c, bool loss) {
 static int finish_wait(vacc_ctx* c, double* rho_loss) {
    HIPCHK(hipStreamSynchronize(c->stream));
    c->stage_used = 0;
-   if (c->h_sum[0] & VACC_STATUS_CAPACITY)
+   if (c->h_sum[0] & VACC_STATUS_CAPACITY) {
+      c->overflow = true;
       return set_err(VACC_E_STATE, "block pool capacity exceeded; state is undefined");
+   }
    c->nblocks = c->h_sum[1];
    if (rho_loss) std::memcpy(rho_loss, c->h_res, c->ncells * sizeof(double));
    return (int)(c->h_sum[2] & 0x7FFFFFFFu);
@@ -772,6 +785,7 @@ static void abort_load(vacc_ctx* c) {
    drop_graphs(c);
    c->ncells = 0;
    c->nblocks = 0;
+   c->overflow = false;
    c->lcur = c->fcur = 0;
    c->sorted = false;
    c->cell_epoch++;
@@ -803,6 +817,7 @@ static int prepare_load(vacc_ctx* c, uint32_t ncells, const uint64_t* offsets, c
    }
    c->ncells = ncells;
    c->nblocks = 0;
+   c->overflow = false;
    c->lcur = 0;
    c->fcur = 0;
    c->sorted = false;
@@ -931,7 +946,9 @@ void ctx_mesh(const vacc_ctx* c, vacc_mesh* mesh, double cell[3]) {
 }
 
 int export_lists(vacc_ctx* c, std::vector<uint32_t>& counts, std::vector<uint32_t>& gids) {
-   int rc = refresh_count(c);
+   int rc = check_lists(c);
+   if (rc) return rc;
+   rc = refresh_count(c);
    if (rc) return rc;
    rc = do_relist(c, -1, false);    // ascending GID order, same blocks
    if (rc) return rc;
@@ -1346,6 +1363,7 @@ static int init_peaks_load(vacc_ctx* c, uint32_t ncells, uint32_t max_peaks, con
    c->lcur = 0;
    c->fcur = 0;
    c->nblocks = 0;
+   c->overflow = false;
    c->sorted = false;
    c->cell_epoch++;
    c->content_valid = false;
@@ -1584,8 +1602,8 @@ int vacc_get_counts(vacc_ctx* c, uint32_t* ncells, uint32_t* counts) {
 int vacc_download_cells(vacc_ctx* c, uint64_t* offsets, uint32_t* gids, float* f) {
    if (!c || !offsets) return set_err(VACC_E_ARG, "null argument");
    if (!c->off[0]) return set_err(VACC_E_HIP, "the context holds no lists: nothing was loaded");
-   int rc = stage_begin(c);
-   if (rc) return rc;
+   int rc = check_lists(c);
+   if (rc || (rc = stage_begin(c))) return rc;
    rc = do_relist(c, -1, false);    // ascending GID order, same blocks
    if (rc) return rc;
    rc = do_compact(c);
@@ -1672,6 +1690,7 @@ static MomentArgs moment_args(const vacc_ctx* c) {
    ma.pool = pool(c, c->fcur);
    ma.out = c->moments;
    ma.part = c->parts;
+   ma.flags = c->flags;
    ma.ncells = c->ncells;
    for (int d = 0; d < 3; ++d) {
       ma.len[d] = c->mi.len[d];
@@ -1735,6 +1754,7 @@ int vacc_set_fields(vacc_ctx* c, const vacc_cell_fields* fields) {
 int vacc_compute_cell_intersections(vacc_ctx* c, const vacc_cell_fields* fields, uint32_t map_order, int32_t use_moments) {
    if (!c || map_order > 2) return set_err(VACC_E_ARG, "bad argument");
    if (!c->ncells) return 0;
+   if (const int rc = use_moments ? check_lists(c) : 0) return rc;
    if (fields) {
       const int rc = upload_fields(c, fields);
       if (rc) return rc;
@@ -2137,7 +2157,8 @@ int vacc_find_blocks(vacc_ctx* c, uint64_t nq, const uint32_t* cells, const uint
    if (!c) return set_err(VACC_E_ARG, "null context");
    if (!nq) return 0;
    if (!cells || !gids || !index) return set_err(VACC_E_ARG, "null argument");
-   int rc = 0;
+   int rc = check_lists(c);
+   if (rc) return rc;
    if (c->ncells && !c->sorted && (rc = do_relist(c, -1, false))) return rc;   // ascending GIDs, same blocks
    // queries go through the device in chunks of FIND_CHUNK: cell, GID and the answer
    constexpr uint64_t FIND_CHUNK = 1u << 24;
@@ -2171,7 +2192,8 @@ int vacc_find_blocks_noalloc(vacc_ctx* c, uint64_t nq, const uint32_t* cells, co
       return set_err(VACC_E_HIP, std::string("vacc_find_blocks_noalloc: no scratch address for this device: ") +
                                      hipGetErrorString(e));
    }
-   int rc = 0;
+   int rc = check_lists(c);
+   if (rc) return rc;
    if (c->ncells && !c->sorted && (rc = do_relist(c, -1, false))) return rc;   // ascending GIDs, no allocation
    const uint32_t m = (uint32_t)nq;
    uint32_t* qc = d;
@@ -2190,6 +2212,7 @@ int vacc_find_blocks_noalloc(vacc_ctx* c, uint64_t nq, const uint32_t* cells, co
 int vacc_moments(vacc_ctx* c, double* out) {
    if (!c || (!out && c->ncells)) return set_err(VACC_E_ARG, "null argument");
    if (!c->ncells) return 0;
+   if (const int rc = check_lists(c)) return rc;
    if (c->moments_valid) launch_copy_f64(c->d_res, c->moments, 4 * c->ncells, c->stream);
    else enqueue_moments(c, c->d_res);
    HIPCHK(hipGetLastError());
@@ -2201,6 +2224,7 @@ int vacc_moments(vacc_ctx* c, double* out) {
 int vacc_pressure(vacc_ctx* c, const double* pivot, double* out) {
    if (!c || (!out && c->ncells)) return set_err(VACC_E_ARG, "null argument");
    if (!c->ncells) return 0;
+   if (const int rc = check_lists(c)) return rc;
    const size_t n = c->ncells;
    // without a pivot the kernel takes the population's own bulk velocity from its first moments
    if (pivot) HIPCHK(hipMemcpyAsync(c->press, pivot, 3 * n * sizeof(double), hipMemcpyHostToDevice, c->stream));
@@ -2365,7 +2389,8 @@ int vacc_trans_map_1d(vacc_ctx* c, uint32_t dim, double dt) {
    if (!c->ncells) return 0;
    // captured steps stay valid: no buffer moves, and the list/pool parity and validity flags
    // that select a captured variant are updated below
-   int rc = 0;
+   int rc = check_lists(c);
+   if (rc) return rc;
    if (!c->sorted && (rc = do_relist(c, -1, false))) return rc;   // ascending GIDs, same blocks
    TransArgs ta{};
    ta.off = c->off[c->lcur];
