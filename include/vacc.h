@@ -60,7 +60,8 @@ enum { VACC_STORE_F32 = 0, VACC_STORE_BF16 = 1, VACC_STORE_F16 = 2 };
 #define VACC_STATUS_WALL 1u        /* target blocks within wall margin (cpu_acc_map.cpp:325-338) */
 #define VACC_STATUS_DK 2u          /* non-positive intersection_dk, or a deposit span (dv + 3|di| + 3|dj|)/dk
                                       above 118 cells: cell passed through, not remapped */
-#define VACC_STATUS_CAPACITY 4u    /* block pool capacity exceeded: step not performed */
+#define VACC_STATUS_CAPACITY 4u    /* block pool capacity exceeded: the call returns VACC_E_STATE, and so
+                                      do later ones that need the blocks, until cells are loaded */
 
 /* errors */
 #define VACC_E_ARG (-1)
@@ -273,7 +274,9 @@ int vacc_accelerate_subcycled(vacc_ctx* ctx, double dt, uint32_t map_order, int3
  * (calculateMoments_V, arch_moments.cpp:342-440: V = sum m nV / sum m n, RHOQ = sum q n).
  * Then its three remaps and, when adjust != 0, its adjust.  rho_loss may be NULL, or hold npop
  * pointers (each NULL or ncells doubles).  One host synchronisation; returns the OR of the
- * per-cell status bits of all populations. */
+ * per-cell status bits of all populations, or the first error.  A population whose storage
+ * overflows does not hold up the others: they are stepped, and their lists, counts and removed
+ * masses are those of the step. */
 int vacc_accelerate_populations(vacc_ctx* const* ctxs, uint32_t npop, uint32_t map_order, int32_t use_moments,
                                 int32_t adjust, double* const* rho_loss);
 /* Synthetic initial state, the project helper used by tests and benchmarks: mirrors

@@ -98,3 +98,52 @@ def test_overflow_is_an_error_and_a_load_clears_it(call, form):
             assert np.array_equal(a, b)
         fresh.close()
     ctx.close()
+
+
+@pytest.mark.parametrize("use_moments", [False, True])
+@pytest.mark.parametrize("bad", [0, 1, 2])
+def test_populations_behind_one_that_overflows_are_finished(bad, use_moments):
+    """Three populations of four cells, one of which overflows: the call is an error, and the others'
+    counts, lists, f and removed mass are those of a step of their own, also through a translation."""
+    from vlasiator_amd import trans as T
+    print(f"population {bad} overflows, use_moments={use_moments}", flush=True)
+    fields = rotation() * 4
+    # the compact cells' content reaches their edges, so that the step changes their block counts
+    cells = [[compact_cell(10 * p + i, 5 + i) for i in range(4)] for p in range(3)]
+    cells[bad] = [scattered_cell(i) for i in range(4)]
+    ctxs = [context(tolerance=True) for _ in range(3)]
+    for ctx, cw in zip(ctxs, cells):
+        ctx.upload_cells(cw)
+        ctx.set_fields(fields)
+    before = [ctx.total_blocks() for ctx in ctxs]
+    loss = [np.full(4, -1.0) for _ in range(3)]
+    refused(lambda: V.accelerate_populations(ctxs, 0, use_moments=use_moments, adjust=True, rho_loss=loss))
+    pencils = T.build_pencils_uniform((4, 1, 1), (True, True, True), np.zeros(4, np.uint8), (1e7,) * 3, 0)
+    for p in range(3):
+        if p == bad:
+            refused(lambda: ctxs[p].download())
+            continue
+        total = ctxs[p].total_blocks()
+        assert total != before[p] and total == sum(ctxs[p].counts())
+        T.set_pencils(ctxs[p], 0, pencils)
+        got = [ctxs[p].download_cells()]
+        T.trans_map_1d(ctxs[p], 0, 1.0)
+        got.append(ctxs[p].download_cells())
+        assert sum(g.size for g, _ in got[0]) == total
+        if use_moments:   # a pivot of its own: only the counts compare
+            continue
+        alone, lost = context(tolerance=True), np.zeros(4)
+        alone.upload_cells(cells[p])
+        alone.set_fields(fields)
+        alone.step(0, use_moments=False, rho_loss=lost)
+        want = [alone.download_cells()]
+        T.set_pencils(alone, 0, pencils)
+        T.trans_map_1d(alone, 0, 1.0)
+        want.append(alone.download_cells())
+        for a, b in zip(got, want):
+            for (g1, f1), (g2, f2) in zip(a, b):
+                assert np.array_equal(g1, g2) and np.array_equal(f1, f2)
+        assert np.array_equal(loss[p], lost)
+        alone.close()
+    for ctx in ctxs:
+        ctx.close()

@@ -50,6 +50,7 @@ struct vacc_ctx {
    size_t cap = 0;             // block capacity of lists, pools and pass scratch
    int lcur = 0, fcur = 0;
    uint64_t nblocks = 0;       // total blocks as of the last synchronisation point
+   bool count_stale = false;   // launches since then changed the list: nblocks is that of the list before
    bool overflow = false;      // a call found the pool too small: no list until the next load
    bool content_valid = false;
    bool moments_valid = false; // `moments` holds the moments of the current list
@@ -413,14 +414,14 @@ static int ensure_blocks(vacc_ctx* c, size_t want) {
    return 0;
 }
 
-// Read the total block count of the current list (synchronises the stream).  Every call that
-// changes the list ends with the count known (finish, a load), so only the synthetic initial
-// state, which sizes its buffers by it, reads it here.
+// Read the total block count of the current list (synchronises the stream): for the synthetic
+// initial state, which sizes its buffers by it, and for the calls that hand out counts.
 static int refresh_count(vacc_ctx* c) {
    uint32_t tot = 0;
    HIPCHK(hipMemcpyAsync(&tot, c->off[c->lcur] + c->ncells, sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
    HIPCHK(hipStreamSynchronize(c->stream));
    c->nblocks = tot;
+   c->count_stale = false;
    return 0;
 }
 
@@ -430,9 +431,18 @@ static int check_lists(const vacc_ctx* c) {
    return c->overflow ? set_err(VACC_E_STATE, "block pool capacity was exceeded: load the cells again") : 0;
 }
 
+// What a call that uses nblocks starts with.  A call that changes the list ends with the count known
+// (finish, a load); only after one that failed between its launches is it collected here.
+static int finish(vacc_ctx* c, double* rho_loss = nullptr);
+static int known_count(vacc_ctx* c) {
+   int rc = check_lists(c);
+   if (!rc && c->count_stale) rc = finish(c);
+   return rc < 0 ? rc : 0;
+}
+
 // Keep head-room for the growth of one step (new target blocks and adjust halo blocks).
 static int reserve_for_step(vacc_ctx* c) {
-   if (const int rc = check_lists(c)) return rc;
+   if (const int rc = known_count(c)) return rc;
    const size_t want = c->nblocks + c->nblocks / 2 + 64 * (size_t)c->ncells + 4096;
    if (want > c->cap) return ensure_blocks(c, want + want / 4);
    return 0;
@@ -549,6 +559,7 @@ static int do_pass(vacc_ctx* c, int dim, bool stats = false) {
    }
    c->lcur = lo;
    c->fcur = fo;
+   c->count_stale = true;
    c->content_valid = true;
    c->moments_valid = false;
    c->stats_valid = stats;
@@ -647,6 +658,7 @@ static int do_relist(vacc_ctx* c, int add_width, bool want_loss, const SpatialIn
    }
    HIPCHK(hipGetLastError());
    c->lcur = lo;
+   if (add_width >= 0) c->count_stale = true;
    c->content_valid = false;
    c->sorted = true;
    if (add_width >= 0) c->moments_valid = false;   // blocks may have been removed
@@ -682,11 +694,12 @@ static int finish_wait(vacc_ctx* c, double* rho_loss) {
       return set_err(VACC_E_STATE, "block pool capacity exceeded; state is undefined");
    }
    c->nblocks = c->h_sum[1];
+   c->count_stale = false;
    if (rho_loss) std::memcpy(rho_loss, c->h_res, c->ncells * sizeof(double));
    return (int)(c->h_sum[2] & 0x7FFFFFFFu);
 }
 
-static int finish(vacc_ctx* c, double* rho_loss = nullptr) {
+static int finish(vacc_ctx* c, double* rho_loss) {
    const int rc = finish_enqueue(c, rho_loss != nullptr);
    return rc ? rc : finish_wait(c, rho_loss);
 }
@@ -785,7 +798,7 @@ static void abort_load(vacc_ctx* c) {
    drop_graphs(c);
    c->ncells = 0;
    c->nblocks = 0;
-   c->overflow = false;
+   c->count_stale = c->overflow = false;
    c->lcur = c->fcur = 0;
    c->sorted = false;
    c->cell_epoch++;
@@ -817,7 +830,7 @@ static int prepare_load(vacc_ctx* c, uint32_t ncells, const uint64_t* offsets, c
    }
    c->ncells = ncells;
    c->nblocks = 0;
-   c->overflow = false;
+   c->count_stale = c->overflow = false;
    c->lcur = 0;
    c->fcur = 0;
    c->sorted = false;
@@ -1363,7 +1376,7 @@ static int init_peaks_load(vacc_ctx* c, uint32_t ncells, uint32_t max_peaks, con
    c->lcur = 0;
    c->fcur = 0;
    c->nblocks = 0;
-   c->overflow = false;
+   c->count_stale = c->overflow = false;
    c->sorted = false;
    c->cell_epoch++;
    c->content_valid = false;
@@ -1602,7 +1615,7 @@ int vacc_get_counts(vacc_ctx* c, uint32_t* ncells, uint32_t* counts) {
 int vacc_download_cells(vacc_ctx* c, uint64_t* offsets, uint32_t* gids, float* f) {
    if (!c || !offsets) return set_err(VACC_E_ARG, "null argument");
    if (!c->off[0]) return set_err(VACC_E_HIP, "the context holds no lists: nothing was loaded");
-   int rc = check_lists(c);
+   int rc = known_count(c);
    if (rc || (rc = stage_begin(c))) return rc;
    rc = do_relist(c, -1, false);    // ascending GID order, same blocks
    if (rc) return rc;
@@ -1979,6 +1992,7 @@ static int graph_step(vacc_ctx* c, uint32_t map_order, int32_t use_moments, int3
          HIPCHK(hipGraphLaunch(g.exec, c->stream));
          c->lcur = g.lcur_out;
          c->fcur = g.fcur_out;
+         c->count_stale = true;
          c->moments_valid = g.moments_out;
          c->content_valid = g.content_out;
          c->stats_valid = g.stats_out;
@@ -2085,6 +2099,46 @@ int vacc_accelerate_subcycled(vacc_ctx* c, double dt, uint32_t map_order, int32_
    return st;
 }
 
+// The launches of population p's part of a step: pivot, transform, three passes, adjust.
+static int enqueue_population(vacc_ctx* const* ctxs, uint32_t npop, uint32_t p, uint32_t map_order, int32_t use_moments,
+                              int32_t adjust) {
+   vacc_ctx* c = ctxs[p];
+   if (use_moments) {
+      PlasmaArgs pa{};
+      pa.npop = (int)npop;
+      pa.ncells = c->ncells;
+      pa.out = c->pivot;
+      for (uint32_t q = 0; q < npop; ++q) {
+         vacc_ctx* o = ctxs[q];
+         enqueue_moments(o);
+         if (q != p) {
+            HIPCHK(hipEventRecord(o->mom_ev, o->stream));
+            HIPCHK(hipStreamWaitEvent(c->stream, o->mom_ev, 0));
+         }
+         pa.mom[q] = o->moments;
+         pa.mass[q] = o->sp.mass;
+         pa.charge[q] = o->sp.charge;
+      }
+      {
+         ProfScope ps(c, 3);
+         launch_plasma(pa, c->stream);
+      }
+      enqueue_transform(c, map_order, 2);
+   } else {
+      enqueue_transform(c, map_order, 0);
+   }
+   for (int d = 0; d < 3; ++d) {
+      const int rc = do_pass(c, pass_dim((int)map_order, d), d == 2);
+      if (rc) return rc;
+   }
+   if (adjust) {
+      const int rc = do_relist(c, c->sp.sparse_add_width_v, true);
+      if (rc) return rc;
+   }
+   HIPCHK(hipGetLastError());
+   return 0;
+}
+
 int vacc_accelerate_populations(vacc_ctx* const* ctxs, uint32_t npop, uint32_t map_order, int32_t use_moments,
                                 int32_t adjust, double* const* rho_loss) {
    if (!ctxs || npop == 0 || npop > (uint32_t)MAX_POP || map_order > 2) return set_err(VACC_E_ARG, "bad argument");
@@ -2101,56 +2155,31 @@ int vacc_accelerate_populations(vacc_ctx* const* ctxs, uint32_t npop, uint32_t m
       const int rc = reserve_for_step(ctxs[p]);
       if (rc) return rc;
    }
+   // the first error is the call's; it must not keep the other populations from being finished,
+   // whose lists have changed too
+   int err = 0, st = 0;
+   std::string what;
+   auto ok = [&](int rc) {
+      if (rc < 0 && !err) {
+         err = rc;
+         what = g_err;
+      }
+      return rc >= 0;
+   };
    // populations one after another, as calculateAcceleration's loop over popID
    // (vlasovmover.cpp:503-565): each one's pivot sees the others' current state
-   for (uint32_t p = 0; p < npop; ++p) {
-      vacc_ctx* c = ctxs[p];
-      if (use_moments) {
-         PlasmaArgs pa{};
-         pa.npop = (int)npop;
-         pa.ncells = c->ncells;
-         pa.out = c->pivot;
-         for (uint32_t q = 0; q < npop; ++q) {
-            vacc_ctx* o = ctxs[q];
-            enqueue_moments(o);
-            if (q != p) {
-               HIPCHK(hipEventRecord(o->mom_ev, o->stream));
-               HIPCHK(hipStreamWaitEvent(c->stream, o->mom_ev, 0));
-            }
-            pa.mom[q] = o->moments;
-            pa.mass[q] = o->sp.mass;
-            pa.charge[q] = o->sp.charge;
-         }
-         {
-            ProfScope ps(c, 3);
-            launch_plasma(pa, c->stream);
-         }
-         enqueue_transform(c, map_order, 2);
-      } else {
-         enqueue_transform(c, map_order, 0);
-      }
-      for (int d = 0; d < 3; ++d) {
-         const int rc = do_pass(c, pass_dim((int)map_order, d), d == 2);
-         if (rc) return rc;
-      }
-      if (adjust) {
-         const int rc = do_relist(c, c->sp.sparse_add_width_v, true);
-         if (rc) return rc;
-      }
-      HIPCHK(hipGetLastError());
+   uint32_t stepped = 0;   // populations whose launches are all enqueued
+   while (stepped < npop && ok(enqueue_population(ctxs, npop, stepped, map_order, use_moments, adjust))) ++stepped;
+   const uint32_t begun = std::min(stepped + 1, npop);
+   bool enqueued[MAX_POP];
+   auto loss = [&](uint32_t p) { return (adjust && rho_loss && p < stepped) ? rho_loss[p] : nullptr; };
+   for (uint32_t p = 0; p < begun; ++p) enqueued[p] = ok(finish_enqueue(ctxs[p], loss(p) != nullptr));
+   for (uint32_t p = 0; p < begun; ++p) {
+      if (!enqueued[p]) continue;   // its count stays stale, for the next call on it to collect
+      const int rc = finish_wait(ctxs[p], loss(p));
+      if (ok(rc)) st |= rc;
    }
-   const bool loss = adjust && rho_loss;
-   for (uint32_t p = 0; p < npop; ++p) {
-      const int rc = finish_enqueue(ctxs[p], loss && rho_loss[p]);
-      if (rc) return rc;
-   }
-   int st = 0;
-   for (uint32_t p = 0; p < npop; ++p) {
-      const int rc = finish_wait(ctxs[p], loss ? rho_loss[p] : nullptr);
-      if (rc < 0) return rc;
-      st |= rc;
-   }
-   return st;
+   return err ? set_err(err, what) : st;
 }
 
 int vacc_find_blocks(vacc_ctx* c, uint64_t nq, const uint32_t* cells, const uint32_t* gids, uint32_t* index) {
@@ -2389,7 +2418,7 @@ int vacc_trans_map_1d(vacc_ctx* c, uint32_t dim, double dt) {
    if (!c->ncells) return 0;
    // captured steps stay valid: no buffer moves, and the list/pool parity and validity flags
    // that select a captured variant are updated below
-   int rc = check_lists(c);
+   int rc = known_count(c);
    if (rc) return rc;
    if (!c->sorted && (rc = do_relist(c, -1, false))) return rc;   // ascending GIDs, same blocks
    TransArgs ta{};
