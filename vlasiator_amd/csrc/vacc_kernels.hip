@@ -281,7 +281,9 @@ __device__ inline bool max_lane_rule_binds(int b0, int b1, int ks, float I, floa
 // lowest target any lane still accumulates; the lanes' boundaries lie within
 // (3|di| + 3|dj|)/dk + 1 cells of each other, and block alignment adds 7 cells.  So the open
 // span stays within (4 dv + 3|di| + 3|dj|)/dk + 10 cells, and a cell whose span bound
-// exceeds LEAN_SPAN = LEAN_RING - 10 is left to the exact kernel (32-cell ring).
+// exceeds LEAN_SPAN = LEAN_RING - 10 is left to the exact kernel (32-cell ring).  Blocks that the
+// previous source block finished are stored behind this one's first cell; where the ring
+// has no room for them until then (from about 5.5 cells of span on) they are stored at once.
 constexpr int LEAN_RING = 16;
 constexpr float LEAN_SPAN = (float)(LEAN_RING - 10);
 
@@ -1275,9 +1277,14 @@ __global__ __launch_bounds__(WGS, 5) void k_remap_lean(RemapArgs a) {
             const int openLim = row_max16(min(reach, hi));
             const int flushLim = row_min16(fx.o);
             while (next_open <= lk && WID * next_open <= openLim) {
-               if (next_open - next_flush >= LEAN_RING / WID) {   // ring full: not for LEAN_SPAN cells
-                  atomicOr(&a.status[c], VACC_STATUS_DK);
-                  atomicOr(&a.status[a.ncells], VACC_STATUS_DK);
+               if (next_open - next_flush >= LEAN_RING / WID) {
+                  // ring full: the oldest block is finished (its deposits ended with the previous
+                  // source block, its store would follow this block's first cell), which the
+                  // span of a LEAN_SPAN cell sees to
+                  if (WID * next_flush + WID - 1 >= flushLim) {
+                     atomicOr(&a.status[c], VACC_STATUS_DK);
+                     atomicOr(&a.status[a.ncells], VACC_STATUS_DK);
+                  }
                   flush_block<DIM, ST, LEAN_RING, WGS, true, STATS>(a, ring, tid, l16, setlane0, o, next_flush, slotb + (next_flush - fk), thc);
                   ++next_flush;
                }
