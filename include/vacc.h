@@ -112,8 +112,9 @@ typedef struct vacc_options {
                                  intersections (f within 5e-6 of an FP64 run per cell, L-inf
                                  relative to the cell's max and L1; block lists unchanged).
                                  Cells whose deposits outrun the tolerance kernel's target ring,
-                                 and columns where the reference's 8-lane maximum rule binds,
-                                 take the exact arithmetic. */
+                                 and columns that start below the low wall of the mesh (where
+                                 the reference truncates indices towards 0), take the exact
+                                 arithmetic. */
    int32_t use_graph;         /* 1: vacc_step captures its launches in a hipGraph per state
                                  variant (map order, list/pool parity, options) on first use
                                  and replays it afterwards; results are identical.  Not used

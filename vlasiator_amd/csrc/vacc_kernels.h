@@ -26,9 +26,10 @@ struct Pool {
 //   w: output slot of the first target block (cell-local)
 constexpr uint32_t COPY_FLAG = 0x80000000u;
 // The tolerance-form remap (k_remap_lean) leaves a unit to the exact kernel when one of its
-// columns starts with every lane of an 8-lane group at or below the Lagrangian base (the
-// reference's maximum-lane rule, cpu_acc_map.cpp:515-529, then bounds the deposits by the
-// group's first lane), or when its cell's deposits over a source block could outrun the ring.
+// columns starts below the low wall of the mesh in some lane, or with every lane of an 8-lane group
+// at or below it (the reference truncates indices towards 0 and bounds the group's deposits by
+// its first lane, cpu_acc_map.cpp:515-529), or when its cell's deposits over a source block could
+// outrun the ring.
 constexpr uint32_t EXACT_FLAG = 0x40000000u;
 // Units of cells whose deposit span exceeds MAX_SPAN_CELLS (up to MAX_SPAN_WIDE) go to the
 // wide instance of the exact kernel, in either arithmetic form.

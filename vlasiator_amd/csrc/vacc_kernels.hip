@@ -258,21 +258,27 @@ __device__ inline void column_extent(int ks, int ke, const SetGeom& g, float dv,
    wallhit = (fk < wall) || (fk >= maxlen - wall) || (lk < wall) || (lk >= maxlen - wall);
 }
 
-// The reference's lanes of minimum and maximum Lagrangian index (cpu_acc_map.cpp:515-529)
-// start from DBL_MIN, so a group of 8 lanes whose Lagrangian indices at the column start are
-// all <= 0 takes its first lane as the maximum.  True when that happens to either group of the
-// column's 16 pencils (the expressions are k_remap's, so the signs agree exactly).
-__device__ inline bool max_lane_rule_binds(int b0, int b1, int ks, float I, float di, float dj, float dv, float vmin) {
+// Columns whose deposits take the exact arithmetic in the tolerance form, because the reference
+// treats Lagrangian indices below 0 by rules that the flux form does not have:
+//   its lanes of minimum and maximum index (cpu_acc_map.cpp:515-529) start from DBL_MIN, so a group
+//   of 8 lanes whose indices at the column start are all <= 0 takes its first lane as the maximum;
+//   an index is truncated towards 0 (:505-508, :564), so at the low wall of the mesh the mass between
+//   -1 and 0 goes to target 0, together with that target's own.
+// True when a lane's index at the column start is below 0, or a group's are all <= 0 (the
+// expressions are k_remap's, so the signs agree exactly).
+__device__ inline bool starts_below_zero(int b0, int b1, int ks, float I, float di, float dj, float dv, float vmin) {
    const float vr = (float)(uint32_t)(WID * ks) * dv + vmin;
-   bool none_pos[2] = {true, true};
+   bool none_pos[2] = {true, true}, neg = false;
 #pragma unroll
    for (int jp = 0; jp < WID; ++jp)
 #pragma unroll
       for (int ip = 0; ip < WID; ++ip) {
          const float imin = (I + (float)(uint32_t)(b0 * WID + ip) * di) + (float)(uint32_t)(b1 * WID + jp) * dj;
-         if (vr - imin > 0.0f) none_pos[jp >> 1] = false;
+         const float x = vr - imin;
+         if (x > 0.0f) none_pos[jp >> 1] = false;
+         neg |= x < 0.0f;
       }
-   return none_pos[0] || none_pos[1];
+   return neg || none_pos[0] || none_pos[1];
 }
 
 // Target ring of the tolerance-form remap, in cells per lane.  Before each source block the
@@ -493,7 +499,7 @@ __global__ __launch_bounds__(CWG, 8) void k_columns(ColumnArgs a) {
          const uint32_t bb = (uint32_t)b0 | ((uint32_t)b1 << 16), cf = copy ? COPY_FLAG : 0u;
          auto exact_col = [&](uint32_t j) {
             return a.fast && !copy &&
-                   max_lane_rule_binds(b0, b1, (int)(a.col_rec[off + cb + j].x & 0xFFFFu), I, di, dj, a.dv, a.vmin);
+                   starts_below_zero(b0, b1, (int)(a.col_rec[off + cb + j].x & 0xFFFFu), I, di, dj, a.dv, a.vmin);
          };
          if (overlap) {
             bool ex = lean_wide || lean_shared;
