@@ -1,13 +1,14 @@
 // vacc_kernels.hip -- gfx950 kernels of the velocity-space acceleration step.
 //
-// One 1-D remap pass along a dimension is four launches over all cells:
+// One 1-D remap pass along a dimension is four launches over all cells, five in the tolerance form
+// (k_remap_lean, which leaves a few units to k_remap):
 //   k_columns  one workgroup per cell: LDS bitmap counting sort of the cell's
 //              blocks into column sets / columns along the pass axis, target
 //              extents of every column (cpu_acc_map.cpp:250-353) and the
 //              output slot of every target block.
 //   k_build_scan  exclusive scans over cells of the target and unit counts (output
-//              offsets, work list) and of the units per length bin, then
-//              k_order: the global work list, longest units first.
+//              offsets, work list) and of the units per length bin.
+//   k_order    the global work list, longest units first.
 //   k_remap    persistent: 16 lanes per column set, one lane per transverse
 //              pencil, walks the columns of the set sourcing the blocks from
 //              HBM once and writing every target block once, with the PLM,
@@ -1185,9 +1186,10 @@ __device__ inline int row_min16(int x) {
 }
 
 // At least five waves per SIMD (at most 96 VGPRs).  The values that no longer fit are kept in
-// scratch across the per-unit setup and the column ends, not in the block loop: none to 8
-// bytes per lane for FP32 storage (PQM; up to 16 with block sums), 32 to 84 for the 16-bit forms
-// (their codec alone would need 111 to 116 VGPRs).  Five waves issue about 7 % more per pass
+// scratch across the per-unit setup and the column ends, not in the block loop.  Bytes per lane,
+// PQM: 20, 16 and none along x, y and z for FP32 storage (36, 52 and 16 with block sums), 28 to 72
+// for the 16-bit forms (56 to 100 with block sums; their codec alone would need 111 to 116 VGPRs);
+// PPM: none to 8 and none to 52.  Five waves issue about 7 % more per pass
 // than four on the PQM workloads for FP32 and make the 16-bit forms' step 3 % faster.
 // Bound by VALU issue and latency: with limiters and face tests as medians of three, halved
 // derivatives (vacc_lean.h) and targets placed by a minimum in place of a range test, a PQM cell

@@ -323,15 +323,6 @@ __device__ inline uint32_t wave_min(uint32_t x) {
    return min(min(a, b), min(c, d));
 }
 
-// The groups of 8 lanes with a bit in m, all their bits set (check_skip_remapping's groups).
-__device__ inline unsigned long long group8(unsigned long long m) {
-   m |= m >> 4;
-   m |= m >> 2;
-   m |= m >> 1;
-   m &= 0x0101010101010101ull;
-   return (m << 8) - m;
-}
-
 // Work split of the pencil walk: for each segment, the walked cells' blocks (pairs of a walked
 // position and a block it holds) counted in a histogram of WB_BINS GID bins in LDS, then
 // bounds[s][0..wps] = GID bounds of wps shares holding equal numbers of pairs, to a bin:
@@ -412,13 +403,14 @@ __global__ __launch_bounds__(TWG) void k_walk_bounds(WalkArgs w, uint32_t* bound
 // different segments of one pencil, is walked in launch levels in the reference's order; a
 // later level's sum starts from the block the earlier one stored (FP32).
 // Bound by the latency of its loads and by its scalar work per source (window bits, branches,
-// addresses), less by VALU issue: 20 % fewer VALU instructions alone gained nothing, while runs with
+// addresses), less by VALU issue (an instruction issues in 0.59 of the quad-cycles; waves wait for
+// memory and the scalar unit 0.48 of their cycles): 20 % fewer VALU instructions alone gained nothing, while runs with
 // a shifting window mask, one test per finished position, a path without the 8-lane groups and
 // pool indices fetched with the GIDs took a call over 7.3 million blocks (1024 cells, PQM
 // workload, 16 x 8 x 8 periodic) from 3.35 to 2.89 ms.  Faces through scalar loads instead of LDS
 // (3.03 ms), values two sources ahead (no change) and a shared reciprocal for the widths' quotients
 // (3 % slower: its range test costs a branch) were measured and not kept.
-// Waves per SIMD: eight for FP32 (64 VGPRs, 8 bytes per lane spilled; 2 % faster than seven) and
+// Waves per SIMD: eight for FP32 (64 VGPRs, 12 bytes per lane spilled; 2 % faster than seven) and
 // seven for the 16-bit forms.
 template <int ST>
 __global__ __launch_bounds__(TWG) __attribute__((amdgpu_waves_per_eu(ST == ST_F32 ? 8 : 7))) void k_trans_walk(
