@@ -425,8 +425,8 @@ static int refresh_count(vacc_ctx* c) {
    return 0;
 }
 
-// After a capacity overflow the current list is unwritten (its offsets reach beyond the buffers):
-// calls that walk it are refused until cells are loaded again.
+// After a capacity overflow the current list is empty (scan_counts): calls that need the blocks are
+// refused until cells are loaded again.
 static int check_lists(const vacc_ctx* c) {
    return c->overflow ? set_err(VACC_E_STATE, "block pool capacity was exceeded: load the cells again") : 0;
 }
@@ -469,7 +469,6 @@ static int enqueue_pass(vacc_ctx* c, int dim, int grid_mult, int wgs = 0, bool s
    ca.n_units = c->n_units;
    ca.n_targets = c->n_tgt;
    ca.status = c->status;
-   ca.flags = c->flags;
    ca.ncells = c->ncells;
    for (int d = 0; d < 3; ++d) ca.len[d] = c->mi.len[d];
    ca.gs = make_gid_split(c->mi.len);
@@ -593,12 +592,11 @@ static int do_relist(vacc_ctx* c, int add_width, bool want_loss, const SpatialIn
       c->content_valid = false;
    }
    if (add_width >= 0 && !c->content_valid) {
-      launch_content_cells(c->off[li], c->src[li], pool(c, c->fcur), c->minval, c->content, c->flags, c->ncells,
-                           c->stream);
+      launch_content_cells(c->off[li], c->src[li], pool(c, c->fcur), c->minval, c->content, c->ncells, c->stream);
       c->content_valid = true;
    }
    const bool conserve = add_width >= 0 && c->sp.sparse_conserve_mass;
-   if (conserve) launch_cell_sums(c->off[li], c->src[li], pool(c, c->fcur), c->csum_pre, c->flags, c->ncells, c->stream);
+   if (conserve) launch_cell_sums(c->off[li], c->src[li], pool(c, c->fcur), c->csum_pre, c->ncells, c->stream);
    AdjustArgs aa{};
    aa.cell_off = c->off[li];
    aa.gid = c->gid[li];
@@ -651,9 +649,8 @@ static int do_relist(vacc_ctx* c, int add_width, bool want_loss, const SpatialIn
    aa.src_out = c->src[lo];
    launch_adjust(aa, true, c->stream);
    if (conserve) {   // block_adjust_cpu.cpp:96-113
-      launch_cell_sums(c->off[lo], c->src[lo], pool(c, c->fcur), c->csum_post, c->flags, c->ncells, c->stream);
-      launch_cell_scale(c->off[lo], c->src[lo], pool(c, c->fcur), c->csum_pre, c->csum_post, c->flags, c->ncells,
-                        c->stream);
+      launch_cell_sums(c->off[lo], c->src[lo], pool(c, c->fcur), c->csum_post, c->ncells, c->stream);
+      launch_cell_scale(c->off[lo], c->src[lo], pool(c, c->fcur), c->csum_pre, c->csum_post, c->ncells, c->stream);
       c->stats_valid = false;   // f was rescaled
    }
    HIPCHK(hipGetLastError());
@@ -1705,7 +1702,6 @@ static MomentArgs moment_args(const vacc_ctx* c) {
    ma.pool = pool(c, c->fcur);
    ma.out = c->moments;
    ma.part = c->parts;
-   ma.flags = c->flags;
    ma.ncells = c->ncells;
    for (int d = 0; d < 3; ++d) {
       ma.len[d] = c->mi.len[d];

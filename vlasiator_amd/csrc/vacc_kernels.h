@@ -59,7 +59,6 @@ struct ColumnArgs {
    uint32_t* n_units;          // [ncells]
    uint32_t* n_targets;        // [ncells]
    uint32_t* status;           // [ncells + 1] OR-ed status bits; entry ncells ORs all cells
-   const uint32_t* flags;      // device flags word (capacity overflow -> skip)
    uint32_t ncells;
    uint32_t len[3];
    GidSplit gs;                // block coordinates of a GID (from len)
@@ -165,7 +164,7 @@ struct AdjustArgs {
    double* rho_loss;           // [ncells] (count phase, may be null)
    const float4* blk_stats;    // null, or per pool block its sums (the remap's blk_stats): the
                                // count phase then takes a removed block's mass from them
-   const uint32_t* flags;      // global flags (capacity overflow -> skip)
+   const uint32_t* flags;      // global flags (capacity overflow -> the write phase is skipped)
    uint32_t ncells;
    uint32_t len[3];
    GidSplit gs;                // block coordinates of a GID (from len)
@@ -194,7 +193,6 @@ struct MomentArgs {
    double* part;               // partial sums: 4 (moments) or 6 (pressure) doubles per workgroup,
                                // ncells * cell_split(ncells) workgroups
    double* host;               // null, or where the moments also go (device address of pinned memory)
-   const uint32_t* flags;      // global flags (capacity overflow -> skip)
    uint32_t ncells;
    uint32_t len[3];
    GidSplit gs;                // block coordinates of a GID (from len)
@@ -271,14 +269,14 @@ void launch_sparse_min(const SparseArgs& p, const double* moments, const uint32_
                        uint32_t ncells, hipStream_t s);
 // content flag of every block of a list with the cell's threshold
 void launch_content_cells(const uint32_t* off, const uint32_t* src, const Pool& pool, const double* minval,
-                          uint8_t* content, const uint32_t* flags, uint32_t ncells, hipStream_t s);
+                          uint8_t* content, uint32_t ncells, hipStream_t s);
 // FP64 sum of f over each cell's blocks
-void launch_cell_sums(const uint32_t* off, const uint32_t* src, const Pool& pool, double* out, const uint32_t* flags,
-                      uint32_t ncells, hipStream_t s);
+void launch_cell_sums(const uint32_t* off, const uint32_t* src, const Pool& pool, double* out, uint32_t ncells,
+                      hipStream_t s);
 // sparse_conserve_mass (block_adjust_cpu.cpp:96-113): f *= pre[c] / post[c] where post != 0,
 // each product rounded to FP32 (16-bit forms: the block scale)
 void launch_cell_scale(const uint32_t* off, const uint32_t* src, const Pool& pool, const double* pre,
-                       const double* post, const uint32_t* flags, uint32_t ncells, hipStream_t s);
+                       const double* post, uint32_t ncells, hipStream_t s);
 void launch_fill_f64(double* dst, double v, uint32_t n, hipStream_t s);
 // Workgroups per cell of the kernels that read a cell's blocks, about CELL_PARTS in all and at most
 // CELL_SPLIT_MAX per cell.

@@ -108,11 +108,6 @@ __device__ inline bool pass_is_wide(float dv, float di, float dj, float dk) {
    return !(pass_span(dv, di, dj, dk) <= (float)MAX_SPAN_CELLS);
 }
 
-// The capacity flag of the context.  The scan that sizes a pass's or an adjust's output sets it when
-// the output would not fit: that list's offsets then point beyond the buffers and nothing is
-// written at them, so every kernel that walks a list looks at the flag before it does.
-__device__ inline bool overflown(const uint32_t* flags) { return (*flags & VACC_STATUS_CAPACITY) != 0u; }
-
 // DPP data movement within a wave, all lanes active; lanes without a source keep `old`
 template <int CTRL, int ROWS = 0xF>
 __device__ inline uint32_t dpp_u(uint32_t old, uint32_t x) {
@@ -330,7 +325,6 @@ __global__ __launch_bounds__(CWG, 8) void k_columns(ColumnArgs a) {
    const uint32_t c = blockIdx.x;
    const uint32_t off = a.cell_off[c];
    const uint32_t n = a.cell_off[c + 1] - off;
-   if (overflown(a.flags)) return;
    if (n == 0) {
       if (t == 0) {
          a.n_units[c] = 0;
@@ -578,7 +572,10 @@ __device__ inline uint32_t scan_row(uint32_t* row, uint32_t n, uint32_t* sh) {
    return carry;
 }
 
-// exclusive scans of one or two per-cell count arrays, and the capacity check
+// exclusive scans of one or two per-cell count arrays, and the capacity check.  Where the blocks of
+// a don't fit, the list gets no entries (the flag keeps k_remap and the adjust's write phase from
+// running) and must not be walked by the launches behind this one: every offset is set to 0, so that
+// they find empty cells.  (A look at the flag in each of them cost a small step 3 us of 160.)
 __device__ inline void scan_counts(const ScanArgs& a, uint32_t* sh) {
    uint32_t carry0 = 0, carry1 = 0;   // running totals, the same in every thread
    for (uint32_t base = 0; base < a.n; base += 1024 * SCAN_K) {
@@ -609,10 +606,21 @@ __device__ inline void scan_counts(const ScanArgs& a, uint32_t* sh) {
       carry0 += tot[0];
       carry1 += tot[1];
    }
+   const bool over = a.cap_a && carry0 > a.cap_a && a.flags;
+   if (over) {   // each thread over the entries that it wrote
+      for (uint32_t base = 0; base < a.n; base += 1024 * SCAN_K)
+         for (uint32_t k = 0; k < SCAN_K; ++k) {
+            const uint32_t i = base + threadIdx.x * SCAN_K + k;
+            if (i < a.n) {
+               a.a_off[i] = 0u;
+               if (a.b) a.b_off[i] = 0u;
+            }
+         }
+   }
    if (threadIdx.x == 0) {
-      a.a_off[a.n] = carry0;
-      if (a.b) a.b_off[a.n] = carry1;
-      if (a.cap_a && carry0 > a.cap_a && a.flags) atomicOr(a.flags, VACC_STATUS_CAPACITY);
+      a.a_off[a.n] = over ? 0u : carry0;
+      if (a.b) a.b_off[a.n] = over ? 0u : carry1;
+      if (over) atomicOr(a.flags, VACC_STATUS_CAPACITY);
    }
 }
 
@@ -664,7 +672,7 @@ __global__ __launch_bounds__(WG) void k_order(OrderArgs a) {
    // plus the bin's prefix over cells; units take positions in it through an LDS cursor per bin
    static_assert(LEN_BINS == 64, "one wave scans the bins");
    __shared__ uint32_t cursor[LEN_BINS];
-   if (overflown(a.flags)) return;
+   if (*a.flags & VACC_STATUS_CAPACITY) return;
    const uint32_t c = blockIdx.x;
    const uint32_t base = a.unit_base[c];
    const uint32_t nu = a.unit_base[c + 1] - base;
@@ -1147,7 +1155,7 @@ template <int DIM, int METHOD, int ST>
 __global__ __launch_bounds__(WG) void k_remap(RemapArgs a, double i_dv) {
    __shared__ float lds[RING * WG];
    static_assert(RING_WIDE * WG_WIDE <= RING * WG, "the wide ring shares the LDS");
-   if (overflown(a.flags)) return;
+   if (*a.flags & VACC_STATUS_CAPACITY) return;
    const uint32_t all = a.unit_base[a.ncells], nwide = a.len_hist[WIDE_BIN];
    if (blockIdx.x < a.main_grid) {
       const uint32_t first = (a.range == RANGE_EXACT) ? all - nwide - a.len_hist[EXACT_BIN] : 0u;
@@ -1202,7 +1210,7 @@ __global__ __launch_bounds__(WGS, 5) void k_remap_lean(RemapArgs a) {
    using R = ReconLean<METHOD>;
    constexpr int NC = R::NC;
    __shared__ float ring[LEAN_RING][WGS];
-   if (overflown(a.flags)) return;
+   if (*a.flags & VACC_STATUS_CAPACITY) return;
    const int tid = threadIdx.x;
    const int l16 = tid & 15;
    const int ip = l16 & 3, jp = l16 >> 2;
@@ -1407,11 +1415,11 @@ __global__ __launch_bounds__(AWG) void k_adjust(AdjustArgs a) {
    __shared__ uint32_t sh[AWG / 64];
    __shared__ uint32_t carry;
    __shared__ double wloss[AWG / 64];
+   if (WRITE && (*a.flags & VACC_STATUS_CAPACITY)) return;
    const int t = threadIdx.x;
    const uint32_t c = blockIdx.x;
    const uint32_t off = a.cell_off[c];
    const uint32_t n = a.cell_off[c + 1] - off;
-   if (overflown(a.flags)) return;
    const int w = a.add_width;
    const int ww = (w > 0) ? w : 0;
    const uint32_t nx = a.len[0], ny = a.len[1], nz = a.len[2];
@@ -1739,7 +1747,6 @@ __global__ __launch_bounds__(WG) void k_pressure(MomentArgs a, const double* piv
    const int t = threadIdx.x;
    const uint32_t c = blockIdx.x / split, sp = blockIdx.x - c * split;
    const uint32_t off = a.cell_off[c], n = a.cell_off[c + 1] - off;
-   if (overflown(a.flags)) return;
    const int q = t & 15;
    double p[3];
    if (pivot) {
@@ -1819,11 +1826,9 @@ __global__ void k_sparse_min(SparseArgs p, const double* moments, const uint32_t
 // 1.0 million blocks in 300 cells, 2.08 -> 0.33 ms over 1024 cells.
 template <int ST>
 __global__ __launch_bounds__(WG) void k_content_cells(const uint32_t* off, const uint32_t* src, Pool pl,
-                                                      const double* minval, uint8_t* content, const uint32_t* flags,
-                                                      uint32_t split) {
+                                                      const double* minval, uint8_t* content, uint32_t split) {
    const uint32_t c = blockIdx.x / split, sp = blockIdx.x - c * split;
    const uint32_t o = off[c], n = off[c + 1] - o;
-   if (overflown(flags)) return;
    const int t = threadIdx.x, l16 = t & 15, lane0 = (t & 63) & ~15;
    const float thc = content_threshold(minval[c]);
    constexpr uint32_t GROUPS = WG / 16;
@@ -1850,10 +1855,8 @@ __global__ __launch_bounds__(WG) void k_content_cells(const uint32_t* off, const
 }
 
 // FP64 sum of each cell's f: one workgroup per cell, one wave per block
-__global__ __launch_bounds__(WG) void k_cell_sums(const uint32_t* off, const uint32_t* src, Pool pl, double* out,
-                                                  const uint32_t* flags) {
+__global__ __launch_bounds__(WG) void k_cell_sums(const uint32_t* off, const uint32_t* src, Pool pl, double* out) {
    __shared__ double part[WG / 64];
-   if (overflown(flags)) return;
    const uint32_t c = blockIdx.x;
    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
    double acc = 0.0;
@@ -1873,8 +1876,7 @@ __global__ __launch_bounds__(WG) void k_cell_sums(const uint32_t* off, const uin
 
 // f *= pre / post per cell (block_adjust_cpu.cpp:108-112); one workgroup per cell
 __global__ __launch_bounds__(WG) void k_cell_scale(const uint32_t* off, const uint32_t* src, Pool pl,
-                                                   const double* pre, const double* post, const uint32_t* flags) {
-   if (overflown(flags)) return;
+                                                   const double* pre, const double* post) {
    const uint32_t c = blockIdx.x;
    if (post[c] == 0.0) return;
    const double r = pre[c] / post[c];
@@ -1908,7 +1910,6 @@ __global__ __launch_bounds__(WG) void k_moments(MomentArgs a, uint32_t split) {
    const uint32_t c = blockIdx.x / split, sp = blockIdx.x - c * split;
    const uint32_t off = a.cell_off[c];
    const uint32_t n = a.cell_off[c + 1] - off;
-   if (overflown(a.flags)) return;
    const int q = t & 15;
    const int j = q & 3, k = q >> 2;
    const double bx = a.cell[0] * WID, by = a.cell[1] * WID, bz = a.cell[2] * WID;
@@ -1968,7 +1969,6 @@ __global__ __launch_bounds__(WG) void k_moments_sums(MomentArgs a, uint32_t spli
    const uint32_t c = blockIdx.x / split, sp = blockIdx.x - c * split;
    const uint32_t off = a.cell_off[c];
    const uint32_t n = a.cell_off[c + 1] - off;
-   if (overflown(a.flags)) return;
    const double bx = a.cell[0] * WID, by = a.cell[1] * WID, bz = a.cell[2] * WID;
    double s0 = 0.0, sx = 0.0, sy = 0.0, sz = 0.0, wx = 0.0, wy = 0.0, wz = 0.0;
    constexpr int UNR = 4;   // blocks per lane in flight
@@ -2489,28 +2489,28 @@ void launch_sparse_min(const SparseArgs& p, const double* moments, const uint32_
 }
 
 void launch_content_cells(const uint32_t* off, const uint32_t* src, const Pool& pool, const double* minval,
-                          uint8_t* content, const uint32_t* flags, uint32_t ncells, hipStream_t s) {
+                          uint8_t* content, uint32_t ncells, hipStream_t s) {
    if (ncells == 0) return;
    const uint32_t split = cell_split(ncells);
    const dim3 grid(ncells * split);
    if (pool.storage == ST_F32)
-      hipLaunchKernelGGL(k_content_cells<ST_F32>, grid, dim3(WG), 0, s, off, src, pool, minval, content, flags, split);
+      hipLaunchKernelGGL(k_content_cells<ST_F32>, grid, dim3(WG), 0, s, off, src, pool, minval, content, split);
    else if (pool.storage == ST_BF16)
-      hipLaunchKernelGGL(k_content_cells<ST_BF16>, grid, dim3(WG), 0, s, off, src, pool, minval, content, flags, split);
+      hipLaunchKernelGGL(k_content_cells<ST_BF16>, grid, dim3(WG), 0, s, off, src, pool, minval, content, split);
    else
-      hipLaunchKernelGGL(k_content_cells<ST_F16>, grid, dim3(WG), 0, s, off, src, pool, minval, content, flags, split);
+      hipLaunchKernelGGL(k_content_cells<ST_F16>, grid, dim3(WG), 0, s, off, src, pool, minval, content, split);
 }
 
-void launch_cell_sums(const uint32_t* off, const uint32_t* src, const Pool& pool, double* out, const uint32_t* flags,
-                      uint32_t ncells, hipStream_t s) {
+void launch_cell_sums(const uint32_t* off, const uint32_t* src, const Pool& pool, double* out, uint32_t ncells,
+                      hipStream_t s) {
    if (ncells == 0) return;
-   hipLaunchKernelGGL(k_cell_sums, dim3(ncells), dim3(WG), 0, s, off, src, pool, out, flags);
+   hipLaunchKernelGGL(k_cell_sums, dim3(ncells), dim3(WG), 0, s, off, src, pool, out);
 }
 
 void launch_cell_scale(const uint32_t* off, const uint32_t* src, const Pool& pool, const double* pre,
-                       const double* post, const uint32_t* flags, uint32_t ncells, hipStream_t s) {
+                       const double* post, uint32_t ncells, hipStream_t s) {
    if (ncells == 0) return;
-   hipLaunchKernelGGL(k_cell_scale, dim3(ncells), dim3(WG), 0, s, off, src, pool, pre, post, flags);
+   hipLaunchKernelGGL(k_cell_scale, dim3(ncells), dim3(WG), 0, s, off, src, pool, pre, post);
 }
 
 void launch_fill_u32(uint32_t* dst, uint32_t v, uint32_t n, hipStream_t s) {
