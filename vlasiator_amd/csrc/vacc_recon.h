@@ -63,7 +63,7 @@ VACC_HD float deriv_h7(const float* v) {
 // instructions in place of seventeen, the same bits.  A NaN among a and b (the scaled values of a
 // cell with threshold 0 are infinite or NaN) takes the reference's expression: its comparisons
 // and products then choose 2b in both inner tests, or NaN if b is.  That costs a compare and a
-// branch not taken: 2048 cells' exact PQM step 10.85 -> 10.87 ms, 16 cells' PPM step 306 -> 313 us.
+// branch not taken: 2048 cells' exact PQM step 10.86 -> 10.87 ms, 16 cells' PPM step 309 -> 314 us.
 VACC_HD float superbee_ab(float a, float b) {
    const float lo = med3(a, b, 0.0f);
    const float s = med3(a, b, lo + lo);
